@@ -99,7 +99,7 @@ __device__ __forceinline__ void speed_grads(const double* s, double gamma, int o
 }
 
 // Transposed derivative contraction: with a[v] of every node of the
-// workgroup in s (stride S), Fo[v] = Σ_k M[k,i] a[v](k, j) and
+// workgroup in s (put4), Fo[v] = Σ_k M[k,i] a[v](k, j) and
 // Go[v] = Σ_k M[k,j] a[v](i, k) -- the adjoint of contract<n, S>.
 template <int n, int S>
 __device__ __forceinline__ void contract_t(const double* s, int base, int i, int j, const double* M, double* Fo,
@@ -107,19 +107,25 @@ __device__ __forceinline__ void contract_t(const double* s, int base, int i, int
     double Mi[n], Mj[n];
 #pragma unroll
     for (int k = 0; k < n; ++k) {
-        Mi[k] = M[k * n + i];
-        Mj[k] = M[k * n + j];
+        Mi[k] = M[k * op_stride(n) + i];
+        Mj[k] = M[k * op_stride(n) + j];
     }
+    const double2* p = reinterpret_cast<const double2*>(s);
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        double af = 0.0, ag = 0.0;
+    for (int h = 0; h < 2; ++h) {
+        double af = 0.0, bf = 0.0, ag = 0.0, bg = 0.0;
 #pragma unroll
         for (int k = 0; k < n; ++k) {
-            af = fma(Mi[k], s[v * S + base + j * n + k], af);
-            ag = fma(Mj[k], s[v * S + base + k * n + i], ag);
+            const double2 x = p[h * S + base + j * n + k], y = p[h * S + base + k * n + i];
+            af = fma(Mi[k], x.x, af);
+            bf = fma(Mi[k], x.y, bf);
+            ag = fma(Mj[k], y.x, ag);
+            bg = fma(Mj[k], y.y, bg);
         }
-        Fo[v] = af;
-        Go[v] = ag;
+        Fo[2 * h] = af;
+        Fo[2 * h + 1] = bf;
+        Go[2 * h] = ag;
+        Go[2 * h + 1] = bg;
     }
 }
 
@@ -132,8 +138,9 @@ __device__ __forceinline__ void adj_forward(const double* uN, double dt, double 
     using G_ = VGeo<N, EB>;
     constexpr int n = G_::n, NN = G_::NN, S = G_::S;
     if (threadIdx.x < NN) {
-        sDm[threadIdx.x] = -dt * c->D[threadIdx.x / n][threadIdx.x % n];
-        sDh[threadIdx.x] = c->Dhat[threadIdx.x / n][threadIdx.x % n];
+        const int q = (threadIdx.x / n) * G_::MS + threadIdx.x % n;
+        sDm[q] = -dt * c->D[threadIdx.x / n][threadIdx.x % n];
+        sDh[q] = c->Dhat[threadIdx.x / n][threadIdx.x % n];
     }
     double F[4], G[4], vol[4];
     if constexpr (N == 4)
@@ -150,8 +157,8 @@ template <int N, int EB>
 __global__ __launch_bounds__((VGeo<N, EB>::NT), 2) void k_adj_records(KArgs a) {
     using G_ = VGeo<N, EB>;
     constexpr int n = G_::n, NN = G_::NN;
-    __shared__ double lds[G_::LDS];
-    __shared__ double sDm[NN], sDh[NN];
+    __shared__ alignas(16) double lds[G_::LDS];
+    __shared__ alignas(16) double sDm[G_::M], sDh[G_::M];
     const int tid = threadIdx.x;
     const int le = tid / NN, node = tid - (tid / NN) * NN;
     const int i = node % n, j = node / n;
@@ -194,8 +201,8 @@ template <int N, int EB>
 __global__ __launch_bounds__((VGeo<N, EB>::NT), 2) void k_adjoint(KArgs a) {
     using G_ = VGeo<N, EB>;
     constexpr int n = G_::n, NN = G_::NN, S = G_::S;
-    __shared__ double lds[G_::LDS];
-    __shared__ double sDm[NN], sDh[NN];
+    __shared__ alignas(16) double lds[G_::LDS];
+    __shared__ alignas(16) double sDm[G_::M], sDh[G_::M];
     const int tid = threadIdx.x;
     const int le = tid / NN, node = tid - (tid / NN) * NN;
     const int i = node % n, j = node / n;
@@ -457,8 +464,8 @@ template <int N, int EB, int STAGE>
 __global__ __launch_bounds__((VGeo<N, EB>::NT), 2) void k_adj_records_md(AdjArgs a) {
     using G_ = VGeo<N, EB>;
     constexpr int n = G_::n, NN = G_::NN;
-    __shared__ double lds[G_::LDS];
-    __shared__ double sDm[NN];
+    __shared__ alignas(16) double lds[G_::LDS];
+    __shared__ alignas(16) double sDm[G_::M];
     const int tid = threadIdx.x;
     const int le = tid / NN, node = tid - (tid / NN) * NN;
     const int i = node % n, j = node / n;
@@ -471,7 +478,7 @@ __global__ __launch_bounds__((VGeo<N, EB>::NT), 2) void k_adj_records_md(AdjArgs
     const DevConst* c = a.c;
     const double dt = a.dt, invJ = a.inv_jac[e];
     const size_t off = ((size_t)e * NN + node) * 4;
-    if (tid < NN) sDm[tid] = -dt * c->D[tid / n][tid % n];
+    if (tid < NN) sDm[(tid / n) * G_::MS + tid % n] = -dt * c->D[tid / n][tid % n];
     double uN[4], usn[4] = {0, 0, 0, 0}, ut[4], ust[4], Uc[4];
     load4(a.u + off, uN);
     if constexpr (STAGE == 2) load4(a.us + off, usn);
@@ -502,8 +509,8 @@ template <int N, int EB, int STAGE>
 __global__ __launch_bounds__((VGeo<N, EB>::NT), 2) void k_adjoint_md(AdjArgs a) {
     using G_ = VGeo<N, EB>;
     constexpr int n = G_::n, NN = G_::NN, S = G_::S;
-    __shared__ double lds[G_::LDS];
-    __shared__ double sDm[NN], sDh[NN];
+    __shared__ alignas(16) double lds[G_::LDS];
+    __shared__ alignas(16) double sDm[G_::M], sDh[G_::M];
     const int tid = threadIdx.x;
     const int le = tid / NN, node = tid - (tid / NN) * NN;
     const int i = node % n, j = node / n;
@@ -518,8 +525,9 @@ __global__ __launch_bounds__((VGeo<N, EB>::NT), 2) void k_adjoint_md(AdjArgs a) 
     const double dt = a.dt, invJ = a.inv_jac[e];
     const size_t off = ((size_t)e * NN + node) * 4;
     if (tid < NN) {
-        sDm[tid] = -dt * c->D[tid / n][tid % n];
-        sDh[tid] = c->Dhat[tid / n][tid % n];
+        const int q = (tid / n) * G_::MS + tid % n;
+        sDm[q] = -dt * c->D[tid / n][tid % n];
+        sDh[q] = c->Dhat[tid / n][tid % n];
     }
     double uN[4], usn[4] = {0, 0, 0, 0}, lam[4], ut[4], ust[4] = {0, 0, 0, 0}, Uc[4];
     load4(a.u + off, uN);
@@ -740,8 +748,9 @@ __device__ __forceinline__ void adj_forward_sc(const AdjArgs& a, const double* a
     const DevConst* c = a.c;
     const double dt = a.dt, invJ = a.inv_jac[e], gamma = c->gamma, gm1 = gamma - 1.0;
     if (threadIdx.x < NN) {
-        sDm[threadIdx.x] = -dt * c->D[threadIdx.x / n][threadIdx.x % n];
-        sDh[threadIdx.x] = c->Dhat[threadIdx.x / n][threadIdx.x % n];
+        const int q = (threadIdx.x / n) * G_::MS + threadIdx.x % n;
+        sDm[q] = -dt * c->D[threadIdx.x / n][threadIdx.x % n];
+        sDh[q] = c->Dhat[threadIdx.x / n][threadIdx.x % n];
     }
     double vol[4];
     if constexpr (N == 4)
@@ -762,14 +771,12 @@ __device__ __forceinline__ void adj_forward_sc(const AdjArgs& a, const double* a
     double w[4];
     // subcell flux between nodes (0, j) and (1, j), or (n-2, j) and (n-1, j); likewise in y
     if (i == 0 || i == n - 1) {
-#pragma unroll
-        for (int v = 0; v < 4; ++v) w[v] = su[v * S + sidx + (i == 0 ? 1 : -1)];
+        get4<S>(su, sidx + (i == 0 ? 1 : -1), w);
         if (i == 0) rusanov(uN, w, gamma, 1, fnlx);
         else rusanov(w, uN, gamma, 1, fnlx);
     }
     if (j == 0 || j == n - 1) {
-#pragma unroll
-        for (int v = 0; v < 4; ++v) w[v] = su[v * S + sidx + (j == 0 ? n : -n)];
+        get4<S>(su, sidx + (j == 0 ? n : -n), w);
         if (j == 0) rusanov(uN, w, gamma, 2, fnly);
         else rusanov(w, uN, gamma, 2, fnly);
     }
@@ -791,8 +798,8 @@ template <int N, int EB>
 __global__ __launch_bounds__((VGeo<N, EB>::NT), 2) void k_adj_records_sc(AdjArgs a, const double* alpha_tmp) {
     using G_ = VGeo<N, EB>;
     constexpr int n = G_::n, NN = G_::NN;
-    __shared__ double lds[G_::LDS];
-    __shared__ double sDm[NN], sDh[NN];
+    __shared__ alignas(16) double lds[G_::LDS];
+    __shared__ alignas(16) double sDm[G_::M], sDh[G_::M];
     const int tid = threadIdx.x;
     const int le = tid / NN, node = tid - (tid / NN) * NN;
     const int i = node % n, j = node / n;
@@ -829,8 +836,8 @@ template <int N, int EB>
 __global__ __launch_bounds__((VGeo<N, EB>::NT), 1) void k_adjoint_sc(AdjArgs a, const double* alpha_tmp, double J0) {
     using G_ = VGeo<N, EB>;
     constexpr int n = G_::n, NN = G_::NN, S = G_::S;
-    __shared__ double lds[G_::LDS];
-    __shared__ double sDm[NN], sDh[NN];
+    __shared__ alignas(16) double lds[G_::LDS];
+    __shared__ alignas(16) double sDm[G_::M], sDh[G_::M];
     const int tid = threadIdx.x;
     const int le = tid / NN, node = tid - (tid / NN) * NN;
     const int i = node % n, j = node / n;
@@ -921,21 +928,19 @@ __global__ __launch_bounds__((VGeo<N, EB>::NT), 1) void k_adjoint_sc(AdjArgs a, 
         if (blended && i > 0) {  // subcell face between (i-1, j) and (i, j)
             double w[4], ob[4];
             const double iwl = 1.0 / c->weights[i - 1];
+            get4<S>(su, sidx - 1, w);
+            get4<S>(ss, sidx - 1, ob);
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                w[v] = su[v * S + sidx - 1];
-                ob[v] = iwl * ss[v * S + sidx - 1] - iwi * sv[v];
-            }
+            for (int v = 0; v < 4; ++v) ob[v] = iwl * ob[v] - iwi * sv[v];
             rusanov_vjp(w, uN, gamma, 1, ob, bx, ub);
         }
         if (blended && j > 0) {
             double w[4], ob[4];
             const double iwl = 1.0 / c->weights[j - 1];
+            get4<S>(su, sidx - n, w);
+            get4<S>(ss, sidx - n, ob);
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                w[v] = su[v * S + sidx - n];
-                ob[v] = iwl * ss[v * S + sidx - n] - iwj * sv[v];
-            }
+            for (int v = 0; v < 4; ++v) ob[v] = iwl * ob[v] - iwj * sv[v];
             rusanov_vjp(w, uN, gamma, 2, ob, by, ub);
         }
         if (act) {
@@ -944,12 +949,16 @@ __global__ __launch_bounds__((VGeo<N, EB>::NT), 1) void k_adjoint_sc(AdjArgs a, 
         }
         __syncthreads();
         if (blended && i < n - 1) {
+            double q[4];
+            get4<S>(sl, sidx + 1, q);
 #pragma unroll
-            for (int v = 0; v < 4; ++v) ub[v] += sl[v * S + sidx + 1];
+            for (int v = 0; v < 4; ++v) ub[v] += q[v];
         }
         if (blended && j < n - 1) {
+            double q[4];
+            get4<S>(sl + 4 * S, sidx + n, q);
 #pragma unroll
-            for (int v = 0; v < 4; ++v) ub[v] += sl[4 * S + v * S + sidx + n];
+            for (int v = 0; v < 4; ++v) ub[v] += q[v];
         }
         __syncthreads();
     }

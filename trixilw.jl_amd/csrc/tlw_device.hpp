@@ -44,13 +44,18 @@ constexpr int kTraceQSC = 16;
 template <bool SC> constexpr int kRQ = SC ? kTraceQSC : kTraceQ;
 constexpr int kSurfBlock = 128;
 
+// Row stride of an n x n operator kept in LDS: rounded up to a pair of doubles,
+// so that a row is read in 16-byte loads.
+constexpr int op_stride(int n) { return (n + 1) & ~1; }
+
 // Volume workgroup geometry: EB elements, NT threads (a multiple of 64).
 template <int N, int EB> struct VGeo {
     static constexpr int n = N + 1;
     static constexpr int NN = n * n;
-    static constexpr int S = EB * NN;  // LDS stride of one exchanged variable
+    static constexpr int S = EB * NN;  // nodes of a workgroup: LDS stride of one exchanged pair of variables
     static constexpr int NT = ((EB * NN + 63) / 64) * 64;
     static constexpr int LDS = 3 * 8 * S;  // three exchange buffers
+    static constexpr int MS = op_stride(n), M = n * MS;  // row stride and size of an operator in LDS
 };
 // Surface / reduction workgroup geometry: 128 threads.
 template <int N> struct SGeo {
@@ -580,33 +585,64 @@ __device__ inline void boundary_value(const DevConst* c, double x, double y, dou
     u[3] = p / (gamma - 1) + 0.5 * rho * (v1 * v1 + v2 * v2);
 }
 
-// Derivative contraction of one element: out[v] = Σ_k M[i,k] s_f[v][j,k] + Σ_k M[j,k] s_g[v][k,i]
-// where s holds f (variables 0..3) and g (4..7) of every node of the workgroup
-// with stride S between variables, and M (n x n, row-major) is in LDS.
+// Exchange buffers in LDS hold the variables of every node of the workgroup in
+// pairs, [pair][node][2], so that each access moves 16 bytes.  An LDS access
+// takes about 4.5 cycles of a CU per wave instruction for 8 and for 16 bytes a
+// lane alike, and the contractions are bound by it: with 8-byte accesses LW N=4
+// at 1024² spent 1.50 ms in the volume kernel at 10 elements per workgroup.
+template <int S> __device__ __forceinline__ void put4(double* s, int idx, const double* w) {
+    double2* p = reinterpret_cast<double2*>(s);
+    p[idx] = make_double2(w[0], w[1]);
+    p[S + idx] = make_double2(w[2], w[3]);
+}
+template <int S> __device__ __forceinline__ void get4(const double* s, int idx, double* w) {
+    const double2* p = reinterpret_cast<const double2*>(s);
+    const double2 a = p[idx], b = p[S + idx];
+    w[0] = a.x; w[1] = a.y; w[2] = b.x; w[3] = b.y;
+}
+// f (variables 0..3) in the first two pairs, g in the last two
+template <int S> __device__ __forceinline__ void put8(double* s, int idx, const double* f, const double* g) {
+    put4<S>(s, idx, f);
+    put4<S>(s + 4 * S, idx, g);
+}
+// row i of an operator in LDS
+template <int n> __device__ __forceinline__ void op_row(const double* M, int i, double* r) {
+    const double* q = M + i * op_stride(n);
+#pragma unroll
+    for (int k = 0; k + 1 < n; k += 2) {
+        const double2 x = *reinterpret_cast<const double2*>(q + k);
+        r[k] = x.x;
+        r[k + 1] = x.y;
+    }
+    if constexpr (n & 1) r[n - 1] = q[n - 1];
+}
+
+// Derivative contraction of one element: out[v] = Σ_k M[i,k] f[v](k, j) + Σ_k M[j,k] g[v](i, k)
+// with f and g of every node of the workgroup in s (put8) and M (n x n, rows
+// of op_stride(n)) in LDS.
 template <int n, int S>
 __device__ __forceinline__ void contract(const double* s, int base, int i, int j, const double* M, double* out) {
     double Di[n], Dj[n];
+    op_row<n>(M, i, Di);
+    op_row<n>(M, j, Dj);
+    const double2* p = reinterpret_cast<const double2*>(s);
 #pragma unroll
-    for (int k = 0; k < n; ++k) {
-        Di[k] = M[i * n + k];
-        Dj[k] = M[j * n + k];
-    }
+    for (int h = 0; h < 2; ++h) {
+        double a = 0.0, b = 0.0;
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        double acc = 0.0;
+        for (int k = 0; k < n; ++k) {
+            const double2 x = p[h * S + base + j * n + k];
+            a = fma(Di[k], x.x, a);
+            b = fma(Di[k], x.y, b);
+        }
 #pragma unroll
-        for (int k = 0; k < n; ++k) acc = fma(Di[k], s[v * S + base + j * n + k], acc);
-#pragma unroll
-        for (int k = 0; k < n; ++k) acc = fma(Dj[k], s[(4 + v) * S + base + k * n + i], acc);
-        out[v] = acc;
-    }
-}
-
-template <int S> __device__ __forceinline__ void put8(double* s, int idx, const double* f, const double* g) {
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        s[v * S + idx] = f[v];
-        s[(4 + v) * S + idx] = g[v];
+        for (int k = 0; k < n; ++k) {
+            const double2 x = p[(2 + h) * S + base + k * n + i];
+            a = fma(Dj[k], x.x, a);
+            b = fma(Dj[k], x.y, b);
+        }
+        out[2 * h] = a;
+        out[2 * h + 1] = b;
     }
 }
 
@@ -769,7 +805,7 @@ __device__ __forceinline__ void mh_face_pair(double* s, const double* u, double 
 }
 
 // Face values of node (i, j) after the Hancock half-step.  s1 holds the
-// element's uⁿ (variable-major, stride S).  End nodes (ξ = ±1) keep zero
+// element's uⁿ (put4).  End nodes (ξ = ±1) keep zero
 // slope: the reference's one-sided differences there are 0/0.  Half-step
 // terms (all added to the four face values, in the reference's order):
 // +Δt/2 J⁻¹ f(left) / hw[i] for 0 < i < n-1, -Δt/2 J⁻¹ f(right) / hw[i] for
@@ -780,19 +816,24 @@ __device__ __forceinline__ void mh_faces(const double* s1, int sidx, int i, int 
                                          double* qd, double* qu) {
     constexpr int n = N + 1;
     double sx[4] = {0.0, 0.0, 0.0, 0.0}, sy[4] = {0.0, 0.0, 0.0, 0.0};
+    double lo[4], hi[4];
     if (i > 0 && i < n - 1) {
+        get4<S>(s1, sidx - 1, lo);
+        get4<S>(s1, sidx + 1, hi);
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            const double ul = s1[v * S + sidx - 1], ur = s1[v * S + sidx + 1];
+            const double ul = lo[v], ur = hi[v];
             const double back = (u[v] - ul) / c->mh_dx1[i], fwd = (ur - u[v]) / c->mh_dx2[i];
             const double cent = fma(c->mh_fc[i], ur, fma(c->mh_fa[i], ul, c->mh_fb[i] * u[v]));
             sx[v] = minmod3(back, cent, fwd, beta);
         }
     }
     if (j > 0 && j < n - 1) {
+        get4<S>(s1, sidx - n, lo);
+        get4<S>(s1, sidx + n, hi);
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            const double ud = s1[v * S + sidx - n], uu = s1[v * S + sidx + n];
+            const double ud = lo[v], uu = hi[v];
             const double back = (u[v] - ud) / c->mh_dx1[j], fwd = (uu - u[v]) / c->mh_dx2[j];
             const double cent = fma(c->mh_fc[j], uu, fma(c->mh_fa[j], ud, c->mh_fb[j] * u[v]));
             sy[v] = minmod3(back, cent, fwd, beta);
@@ -1044,12 +1085,15 @@ __device__ __forceinline__ void lw4_element(const double* uN, double dt, double 
 #pragma unroll
     for (int v = 0; v < 4; ++v) { dx[v] = -fa[v]; dy[v] = -ga[v]; }
     euler_fluxes(up, gm1, fa, ga);
+    double f0[4], g0[4];
+    get4<S>(s0, sidx, f0);
+    get4<S>(s0 + 4 * S, sidx, g0);
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
         dx[v] = fma(16.0, fa[v], dx[v]);
         dy[v] = fma(16.0, ga[v], dy[v]);
-        dx[v] = fma(-30.0, s0[v * S + sidx], dx[v]);
-        dy[v] = fma(-30.0, s0[(4 + v) * S + sidx], dy[v]);
+        dx[v] = fma(-30.0, f0[v], dx[v]);
+        dy[v] = fma(-30.0, g0[v], dy[v]);
     }
     euler_fluxes(um, gm1, fa, ga);
 #pragma unroll
@@ -1122,12 +1166,14 @@ __device__ __forceinline__ void lw4_element(const double* uN, double dt, double 
 #pragma unroll
     for (int v = 0; v < 4; ++v) { dx[v] = fa[v]; dy[v] = ga[v]; }
     euler_fluxes(up, gm1, fa, ga);
+    get4<S>(s0, sidx, f0);
+    get4<S>(s0 + 4 * S, sidx, g0);
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
         dx[v] = fma(-4.0, fa[v], dx[v]);
         dy[v] = fma(-4.0, ga[v], dy[v]);
-        dx[v] = fma(6.0, s0[v * S + sidx], dx[v]);
-        dy[v] = fma(6.0, s0[(4 + v) * S + sidx], dy[v]);
+        dx[v] = fma(6.0, f0[v], dx[v]);
+        dy[v] = fma(6.0, g0[v], dy[v]);
     }
     euler_fluxes(um, gm1, fa, ga);
 #pragma unroll
@@ -1243,10 +1289,13 @@ __device__ __forceinline__ void lw3_element(const double* uN, double dt, double 
     }
     // f_tt = f(u+1) - 2 f + f(u-1)
     euler_fluxes(up, gm1, fa, ga);
+    double f0[4], g0[4];
+    get4<S>(s0, sidx, f0);
+    get4<S>(s0 + 4 * S, sidx, g0);
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-        dx[v] = fma(-2.0, s0[v * S + sidx], fa[v]);
-        dy[v] = fma(-2.0, s0[(4 + v) * S + sidx], ga[v]);
+        dx[v] = fma(-2.0, f0[v], fa[v]);
+        dy[v] = fma(-2.0, g0[v], ga[v]);
     }
     euler_fluxes(um, gm1, fa, ga);
 #pragma unroll
@@ -1451,33 +1500,31 @@ __device__ __forceinline__ void mdrk2_element(const double* uN, const double* us
 // calc_interface_flux_hyperbolic_parabolic!, dg_2d_parabolic.jl:1911-1948;
 // mdrk_kernel_1!/2!, multi_derivative_2d_parabolic.jl:221-711.
 
-// Separate x and y contractions of the 4 variables in s (stride S):
-// ox[v] = Σ_k M[i,k] s[v][j,k], oy[v] = Σ_k M[j,k] s[v][k,i].
+// Separate x and y contractions of the 4 variables in s (put4):
+// ox[v] = Σ_k M[i,k] s[v](k, j), oy[v] = Σ_k M[j,k] s[v](i, k).
 template <int n, int S>
 __device__ __forceinline__ void contract_xy(const double* s, int base, int i, int j, const double* M, double* ox,
                                             double* oy) {
     double Mi[n], Mj[n];
+    op_row<n>(M, i, Mi);
+    op_row<n>(M, j, Mj);
+    const double2* p = reinterpret_cast<const double2*>(s);
 #pragma unroll
-    for (int k = 0; k < n; ++k) {
-        Mi[k] = M[i * n + k];
-        Mj[k] = M[j * n + k];
-    }
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        double ax = 0.0, ay = 0.0;
+    for (int h = 0; h < 2; ++h) {
+        double ax = 0.0, bx = 0.0, ay = 0.0, by = 0.0;
 #pragma unroll
         for (int k = 0; k < n; ++k) {
-            ax = fma(Mi[k], s[v * S + base + j * n + k], ax);
-            ay = fma(Mj[k], s[v * S + base + k * n + i], ay);
+            const double2 x = p[h * S + base + j * n + k], y = p[h * S + base + k * n + i];
+            ax = fma(Mi[k], x.x, ax);
+            bx = fma(Mi[k], x.y, bx);
+            ay = fma(Mj[k], y.x, ay);
+            by = fma(Mj[k], y.y, by);
         }
-        ox[v] = ax;
-        oy[v] = ay;
+        ox[2 * h] = ax;
+        ox[2 * h + 1] = bx;
+        oy[2 * h] = ay;
+        oy[2 * h + 1] = by;
     }
-}
-
-template <int S> __device__ __forceinline__ void put4(double* s, int idx, const double* w) {
-#pragma unroll
-    for (int v = 0; v < 4; ++v) s[v * S + idx] = w[v];
 }
 
 // Viscous fluxes of CompressibleNavierStokesDiffusion2D from the conservative
@@ -1861,12 +1908,15 @@ __device__ __forceinline__ void lwp_element(const double* uN, const double* gxN,
 #pragma unroll
         for (int v = 0; v < 4; ++v) { dx[v] = -fa[v]; dy[v] = -ga[v]; }
         P.flux(0, gm1, c, fa, ga);
+        double f0[4], g0[4];
+        get4<S>(s0, sidx, f0);
+        get4<S>(s0 + 4 * S, sidx, g0);
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
             dx[v] = fma(16.0, fa[v], dx[v]);
             dy[v] = fma(16.0, ga[v], dy[v]);
-            dx[v] = fma(-30.0, s0[v * S + sidx], dx[v]);
-            dy[v] = fma(-30.0, s0[(4 + v) * S + sidx], dy[v]);
+            dx[v] = fma(-30.0, f0[v], dx[v]);
+            dy[v] = fma(-30.0, g0[v], dy[v]);
         }
         P.flux(1, gm1, c, fa, ga);
 #pragma unroll
@@ -1880,10 +1930,13 @@ __device__ __forceinline__ void lwp_element(const double* uN, const double* gxN,
     } else {
         // stage 2: f_tt = f(u+) - 2 f + f(u-)
         P.flux(0, gm1, c, fa, ga);
+        double f0[4], g0[4];
+        get4<S>(s0, sidx, f0);
+        get4<S>(s0 + 4 * S, sidx, g0);
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            dx[v] = fma(-2.0, s0[v * S + sidx], fa[v]);
-            dy[v] = fma(-2.0, s0[(4 + v) * S + sidx], ga[v]);
+            dx[v] = fma(-2.0, f0[v], fa[v]);
+            dy[v] = fma(-2.0, g0[v], ga[v]);
         }
         P.flux(1, gm1, c, fa, ga);
 #pragma unroll
@@ -1944,12 +1997,15 @@ __device__ __forceinline__ void lwp_element(const double* uN, const double* gxN,
 #pragma unroll
         for (int v = 0; v < 4; ++v) { dx[v] = fa[v]; dy[v] = ga[v]; }
         P.flux(0, gm1, c, fa, ga);
+        double f0[4], g0[4];
+        get4<S>(s0, sidx, f0);
+        get4<S>(s0 + 4 * S, sidx, g0);
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
             dx[v] = fma(-4.0, fa[v], dx[v]);
             dy[v] = fma(-4.0, ga[v], dy[v]);
-            dx[v] = fma(6.0, s0[v * S + sidx], dx[v]);
-            dy[v] = fma(6.0, s0[(4 + v) * S + sidx], dy[v]);
+            dx[v] = fma(6.0, f0[v], dx[v]);
+            dy[v] = fma(6.0, g0[v], dy[v]);
         }
         P.flux(1, gm1, c, fa, ga);
 #pragma unroll
@@ -2617,7 +2673,7 @@ template <bool TWO> constexpr int kVolWaves = TWO ? 2 : TLW_VOL_WAVES;
 // PAR: hyperbolic-parabolic (compressible Navier-Stokes) element procedures,
 // same register budget as shock capturing.
 // The volume workgroup `bid` of a's table, with its LDS: lds [G_::LDS], sDm,
-// sDh, sD [NN] (-dt D, D̂ and D, row-major) and s_alpha [EB] (smoothed blending
+// sDh, sD [G_::M] (-dt D, D̂ and D, rows of G_::MS) and s_alpha [EB] (smoothed blending
 // factors of the curvilinear interfaces).
 template <int N, int EB, int KIND, bool SC, bool PAR, bool CURV>
 __device__ __forceinline__ void volume_body(const KArgs& a, int bid, double* lds, double* sDm, double* sDh, double* sD,
@@ -2674,9 +2730,10 @@ __device__ __forceinline__ void volume_body(const KArgs& a, int bid, double* lds
     }
 
     if (tid < NN) {  // published by the first barrier of the element computation
-        sDm[tid] = -dt * c->D[tid / n][tid % n];
-        sDh[tid] = c->Dhat[tid / n][tid % n];
-        if constexpr (PAR) sD[tid] = c->D[tid / n][tid % n];
+        const int q = (tid / n) * G_::MS + tid % n;
+        sDm[q] = -dt * c->D[tid / n][tid % n];
+        sDh[q] = c->Dhat[tid / n][tid % n];
+        if constexpr (PAR) sD[q] = c->D[tid / n][tid % n];
     }
     double uN[4], Uc[4], F[4], G[4], vol[4];
     double terr = 0.0;  // temporal error of the node (adaptive steps, LW N=4)
@@ -2805,9 +2862,7 @@ __device__ __forceinline__ void volume_body(const KArgs& a, int bid, double* lds
         // order (Trixi calcflux_fv!): the face values are the node values.  A
         // blended element away from the domain boundary with MUSCL-Hancock takes
         // the reconstructed, half-step-evolved face values (mh_faces).
-#pragma unroll
-        for (int v = 0; v < 4; ++v)
-            if (act) s1[v * S + sidx] = uN[v];
+        if (act) put4<S>(s1, sidx, uN);
         __syncthreads();
         const bool blended = !(fabs(alpha_e) <= 1e-12);  // pure_and_blended_element_ids!
         double ql[4], qr[4], qd[4], qu[4];
@@ -2823,8 +2878,7 @@ __device__ __forceinline__ void volume_body(const KArgs& a, int bid, double* lds
         __syncthreads();
         double fxl[4] = {0, 0, 0, 0}, gyl[4] = {0, 0, 0, 0}, w[4];
         if (i > 0) {
-#pragma unroll
-            for (int v = 0; v < 4; ++v) w[v] = s0[v * S + sidx - 1];
+            get4<S>(s0, sidx - 1, w);
             if constexpr (CURV) {
                 // Trixi's subcell normal, or for a pure-DG element at subcell face n-1 the
                 // normal of the reference's calc_fn_low! (structured/dg_2d.jl:111-173)
@@ -2836,8 +2890,7 @@ __device__ __forceinline__ void volume_body(const KArgs& a, int bid, double* lds
             }
         }
         if (j > 0) {
-#pragma unroll
-            for (int v = 0; v < 4; ++v) w[v] = s0[(4 + v) * S + sidx - n];
+            get4<S>(s0 + 4 * S, sidx - n, w);
             if constexpr (CURV) {
                 const double* nq = (!blended && j == n - 1) ? a.sqrk + ((size_t)e * n + i) * 4 + 2
                                                              : a.snrm + ((size_t)e * NN + node) * 4 + 2;
@@ -2849,15 +2902,17 @@ __device__ __forceinline__ void volume_body(const KArgs& a, int bid, double* lds
         if (act) put8<S>(s2, sidx, fxl, gyl);
         __syncthreads();
         const double iwi = 1.0 / c->weights[i], iwj = 1.0 / c->weights[j];
+        double fxr4[4] = {0.0, 0.0, 0.0, 0.0}, gyr4[4] = {0.0, 0.0, 0.0, 0.0};
+        if (i < n - 1) get4<S>(s2, sidx + 1, fxr4);
+        if (j < n - 1) get4<S>(s2 + 4 * S, sidx + n, gyr4);
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            const double fxr = (i < n - 1) ? s2[v * S + sidx + 1] : 0.0;
-            const double gyr = (j < n - 1) ? s2[(4 + v) * S + sidx + n] : 0.0;
+            const double fxr = fxr4[v], gyr = gyr4[v];
             const double fv = iwi * (fxr - fxl[v]) + iwj * (gyr - gyl[v]);
             vol[v] = (1.0 - alpha_e) * vol[v] + (blended ? alpha_e * fv : 0.0);
             // fn_low: the subcell fluxes next to the element faces (load_fn_low!)
-            fnlx[v] = (fx == 0) ? s2[v * S + sidx + 1] : fxl[v];
-            fnly[v] = (fy == 2) ? s2[(4 + v) * S + sidx + n] : gyl[v];
+            fnlx[v] = (fx == 0) ? fxr : fxl[v];
+            fnly[v] = (fy == 2) ? gyr : gyl[v];
         }
         __syncthreads();  // s0, s1 and s2 are reused for the face records and interface sums
     }
@@ -2930,7 +2985,7 @@ __device__ __forceinline__ void volume_body(const KArgs& a, int bid, double* lds
     // workgroup is evaluated once, by the slot of its left element's + face, and
     // its flux goes to both adjacent nodes (accx for x faces, accy for y faces);
     // the record of a face leaving the workgroup goes to HBM for the surface kernel.
-    double* accx = lds + 16 * S;  // [4][S], in s2 (free after the last contraction)
+    double* accx = lds + 16 * S;  // pairs of variables (put4), in s2 (free after the last contraction)
     double* accy = accx + 4 * S;
     constexpr int NSLOT = EB * 4 * n;
     static_assert(NSLOT <= NT, "one face slot per lane");
@@ -2964,11 +3019,8 @@ __device__ __forceinline__ void volume_body(const KArgs& a, int bid, double* lds
                     face_numflux(Lr, Rr, Fs);
                 }
                 double* acc = (f == 1) ? accx : accy;
-#pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    acc[v * S + ls * NN + nodeL] = Fs[v];
-                    acc[v * S + (ne - e0) * NN + nodeR] = Fs[v];
-                }
+                put4<S>(acc, ls * NN + nodeL, Fs);
+                put4<S>(acc, (ne - e0) * NN + nodeR, Fs);
             }
         }
     }
@@ -2979,13 +3031,17 @@ __device__ __forceinline__ void volume_body(const KArgs& a, int bid, double* lds
     double surf[4] = {0.0, 0.0, 0.0, 0.0};
     if (intx) {
         const double wf = (fx & 1) ? c->bnd_hi : -c->bnd_lo;
+        double Fs[4];
+        get4<S>(accx, sidx, Fs);
 #pragma unroll
-        for (int v = 0; v < 4; ++v) surf[v] = accx[v * S + sidx] * wf;
+        for (int v = 0; v < 4; ++v) surf[v] = Fs[v] * wf;
     }
     if (inty) {
         const double wf = (fy & 1) ? c->bnd_hi : -c->bnd_lo;
+        double Fs[4];
+        get4<S>(accy, sidx, Fs);
 #pragma unroll
-        for (int v = 0; v < 4; ++v) surf[v] = fma(accy[v * S + sidx], wf, surf[v]);
+        for (int v = 0; v < 4; ++v) surf[v] = fma(Fs[v], wf, surf[v]);
     }
     double val[4];
 #pragma unroll
@@ -3040,8 +3096,8 @@ constexpr int kVolWavesOf =
 template <int N, int EB, int KIND, bool SC, bool PAR = false, bool CURV = false>
 __global__ __launch_bounds__((VGeo<N, EB>::NT), (kVolWavesOf<KIND, SC, PAR>)) void k_volume(KArgs a) {
     using G_ = VGeo<N, EB>;
-    __shared__ double lds[G_::LDS];
-    __shared__ double sDm[G_::NN], sDh[G_::NN], sD[G_::NN];
+    __shared__ alignas(16) double lds[G_::LDS];
+    __shared__ alignas(16) double sDm[G_::M], sDh[G_::M], sD[G_::M];
     __shared__ double s_alpha[(SC && CURV) ? EB : 1];
     volume_body<N, EB, KIND, SC, PAR, CURV>(a, blockIdx.x, lds, sDm, sDh, sD, s_alpha);
 }
@@ -3925,8 +3981,11 @@ template <int EB3, int EB4>
 __global__ __launch_bounds__((VGeo<4, EB4>::NT), kVolWaves<false>) void k_volume_pair(KArgs a3, KArgs a4, int g3) {
     static_assert(VGeo<3, EB3>::NT == VGeo<4, EB4>::NT, "one block size for both halves");
     constexpr int L = VGeo<3, EB3>::LDS > VGeo<4, EB4>::LDS ? VGeo<3, EB3>::LDS : VGeo<4, EB4>::LDS;
-    __shared__ double lds[L];
-    __shared__ double sDm[25], sDh[25], sD[25], s_alpha[1];
+    constexpr int M = VGeo<4, EB4>::M;
+    static_assert(M >= VGeo<3, EB3>::M, "operators of both degrees");
+    __shared__ alignas(16) double lds[L];
+    __shared__ alignas(16) double sDm[M], sDh[M], sD[M];
+    __shared__ double s_alpha[1];
     if ((int)blockIdx.x < g3)
         volume_body<3, EB3, VOL_LW, false, false, false>(a3, blockIdx.x, lds, sDm, sDh, sD, s_alpha);
     else
