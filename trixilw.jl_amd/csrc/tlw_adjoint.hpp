@@ -22,7 +22,7 @@ namespace tlw {
 constexpr int kAdjQ = 10;  // adjoint face record: u 4, |v_n| 1, c 1, s̄ 4
 
 // Taylor states of the FD flux derivatives: w = u + Σ_d a[kind][d] u^(d+1) for
-// kind = u+2, u+1, u-1, u-2 (the incremental updates of lw4_element/lw3_element)
+// kind = u+2, u+1, u-1, u-2 (the incremental updates of lw_element)
 struct LWTaylor {
     static constexpr double a[4][4] = {{2.0, 2.0, 4.0 / 3.0, 2.0 / 3.0},
                                        {1.0, 0.5, 1.0 / 6.0, 1.0 / 24.0},
@@ -132,23 +132,22 @@ __device__ __forceinline__ void contract_t(const double* s, int base, int i, int
 template <int N> constexpr int kEBA = (N == 4) ? 5 : 8;  // elements per adjoint workgroup
 
 template <int N, int EB, bool KEEP>
-__device__ __forceinline__ void adj_forward(const double* uN, double dt, double invJ, double gm1, const DevConst* c,
-                                            int i, int j, bool act, int sidx, int sbase, double* lds, double* sDm,
+__device__ __forceinline__ void adj_forward(const double* uN, double dt, double invJ, double gm1, DevC c,
+                                            int i, int j, bool act, int sidx, int sbase, double* lds, double* sD,
                                             double* sDh, double* Uc, double* tder) {
     using G_ = VGeo<N, EB>;
     constexpr int n = G_::n, NN = G_::NN, S = G_::S;
     if (threadIdx.x < NN) {
         const int q = (threadIdx.x / n) * G_::MS + threadIdx.x % n;
-        sDm[q] = -dt * c->D[threadIdx.x / n][threadIdx.x % n];
+        sD[q] = c->D[threadIdx.x / n][threadIdx.x % n];
         sDh[q] = c->Dhat[threadIdx.x / n][threadIdx.x % n];
     }
     double F[4], G[4], vol[4];
-    if constexpr (N == 4)
-        lw4_element<N, EB, KEEP>(uN, dt, invJ, gm1, c, i, j, act, sidx, sbase, lds, lds + 8 * S, lds + 16 * S, sDm,
-                                 sDh, Uc, F, G, vol, tder);
-    else
-        lw3_element<N, EB, KEEP>(uN, dt, invJ, gm1, c, i, j, act, sidx, sbase, lds, lds + 8 * S, lds + 16 * S, sDm,
-                                 sDh, Uc, F, G, vol, tder);
+    // the last exchange is in s2 (lds + 16 S)
+    double* A = (N == 4) ? lds + 16 * S : lds + 8 * S;
+    double* B = (N == 4) ? lds + 8 * S : lds + 16 * S;
+    lw_element<N, EB, false, KEEP>(uN, nullptr, dt, -dt * invJ, c->gamma, i, j, act, sidx, sbase, A, B, sD, sDh, Uc, F, G,
+                                   vol, tder);
 }
 
 // Face records of the adjoint: every face node's u, the λ ingredients of Ũ and
@@ -158,7 +157,7 @@ __global__ __launch_bounds__((VGeo<N, EB>::NT), 2) void k_adj_records(KArgs a) {
     using G_ = VGeo<N, EB>;
     constexpr int n = G_::n, NN = G_::NN;
     __shared__ alignas(16) double lds[G_::LDS];
-    __shared__ alignas(16) double sDm[G_::M], sDh[G_::M];
+    __shared__ alignas(16) double sD[G_::M], sDh[G_::M];
     const int tid = threadIdx.x;
     const int le = tid / NN, node = tid - (tid / NN) * NN;
     const int i = node % n, j = node / n;
@@ -168,12 +167,12 @@ __global__ __launch_bounds__((VGeo<N, EB>::NT), 2) void k_adj_records(KArgs a) {
     const int lec = le < nel ? le : nel - 1;
     const int e = e0 + lec;
     const int sidx = lec * NN + node, sbase = lec * NN;
-    const DevConst* c = a.c;
+    const DevC c = dev_const(a.c);
     const double dt = a.dt_arg, invJ = a.inv_jac[e];
     const size_t off = ((size_t)e * NN + node) * 4;
     double uN[4], Uc[4];
     load4(a.u + off, uN);
-    adj_forward<N, EB, false>(uN, dt, invJ, c->gamma - 1.0, c, i, j, act, sidx, sbase, lds, sDm, sDh, Uc, nullptr);
+    adj_forward<N, EB, false>(uN, dt, invJ, c->gamma - 1.0, c, i, j, act, sidx, sbase, lds, sD, sDh, Uc, nullptr);
     const int fx = (i == 0) ? 0 : ((i == n - 1) ? 1 : -1);
     const int fy = (j == 0) ? 2 : ((j == n - 1) ? 3 : -1);
     if (!act || (fx < 0 && fy < 0)) return;
@@ -202,7 +201,7 @@ __global__ __launch_bounds__((VGeo<N, EB>::NT), 2) void k_adjoint(KArgs a) {
     using G_ = VGeo<N, EB>;
     constexpr int n = G_::n, NN = G_::NN, S = G_::S;
     __shared__ alignas(16) double lds[G_::LDS];
-    __shared__ alignas(16) double sDm[G_::M], sDh[G_::M];
+    __shared__ alignas(16) double sD[G_::M], sDh[G_::M];
     const int tid = threadIdx.x;
     const int le = tid / NN, node = tid - (tid / NN) * NN;
     const int i = node % n, j = node / n;
@@ -212,14 +211,18 @@ __global__ __launch_bounds__((VGeo<N, EB>::NT), 2) void k_adjoint(KArgs a) {
     const int lec = le < nel ? le : nel - 1;
     const int e = e0 + lec;
     const int sidx = lec * NN + node, sbase = lec * NN;
-    const DevConst* c = a.c;
+    const DevC c = dev_const(a.c);
     const double gamma = c->gamma, gm1 = gamma - 1.0;
     const double dt = a.dt_arg, invJ = a.inv_jac[e];
     const size_t off = ((size_t)e * NN + node) * 4;
     double uN[4], lam[4], Uc[4], ud[N][4];
     load4(a.u + off, uN);
     load4(a.us + off, lam);
-    adj_forward<N, EB, true>(uN, dt, invJ, gm1, c, i, j, act, sidx, sbase, lds, sDm, sDh, Uc, &ud[0][0]);
+    adj_forward<N, EB, true>(uN, dt, invJ, gm1, c, i, j, act, sidx, sbase, lds, sD, sDh, Uc, &ud[0][0]);
+    // the reverse sweep's Taylor states equal the forward's: formed anew rather than
+    // kept (with their reciprocals) over the whole kernel in private memory
+#pragma unroll
+    for (int v = 0; v < 4; ++v) asm volatile("" : "+v"(uN[v]));
 
     // --- interface fluxes of this node's faces
     double sb[4], Fb[4] = {0, 0, 0, 0}, Gb[4] = {0, 0, 0, 0}, Ucb[4] = {0, 0, 0, 0}, ub[4] = {0, 0, 0, 0};
@@ -304,11 +307,11 @@ __global__ __launch_bounds__((VGeo<N, EB>::NT), 2) void k_adjoint(KArgs a) {
             buf ^= 1;
             double t4[4];
 #pragma unroll
-            for (int v = 0; v < 4; ++v) t4[v] = invJ * udb[k][v];
+            for (int v = 0; v < 4; ++v) t4[v] = (-dt * invJ) * udb[k][v];
             if (act) put4<S>(ex, sidx, t4);
             __syncthreads();
             double cf[4], cg[4];
-            contract_t<n, S>(ex, sbase, i, j, sDm, cf, cg);
+            contract_t<n, S>(ex, sbase, i, j, sD, cf, cg);
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
                 dxb[v] += cf[v];
@@ -348,11 +351,11 @@ __global__ __launch_bounds__((VGeo<N, EB>::NT), 2) void k_adjoint(KArgs a) {
         double* ex = buf ? ex1 : ex0;
         double t4[4];
 #pragma unroll
-        for (int v = 0; v < 4; ++v) t4[v] = invJ * udb[0][v];
+        for (int v = 0; v < 4; ++v) t4[v] = (-dt * invJ) * udb[0][v];
         if (act) put4<S>(ex, sidx, t4);
         __syncthreads();
         double cf[4], cg[4];
-        contract_t<n, S>(ex, sbase, i, j, sDm, cf, cg);
+        contract_t<n, S>(ex, sbase, i, j, sD, cf, cg);
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
             F0b[v] += cf[v];
@@ -430,8 +433,8 @@ __device__ __forceinline__ void mdrk_ft_vjp(const double* u, const double* ut, d
 
 // Forward quantities of a stage the adjoint needs: ut (and ust) and Ũ.
 template <int N, int EB, int STAGE>
-__device__ __forceinline__ void mdrk_adj_forward(const double* uN, const double* usn, double invJ, double gm1, int i,
-                                                 int j, bool act, int sidx, int sbase, double* lds, const double* sDm,
+__device__ __forceinline__ void mdrk_adj_forward(const double* uN, const double* usn, double sc, double gm1, int i,
+                                                 int j, bool act, int sidx, int sbase, double* lds, const double* sD,
                                                  double* ut, double* ust, double* Uc) {
     using G_ = VGeo<N, EB>;
     constexpr int n = G_::n, S = G_::S;
@@ -443,14 +446,14 @@ __device__ __forceinline__ void mdrk_adj_forward(const double* uN, const double*
         if (act) put8<S>(lds + 8 * S, sidx, f, g);
     }
     __syncthreads();
-    contract<n, S>(lds, sbase, i, j, sDm, ut);
+    contract<n, S>(lds, sbase, i, j, sD, ut);
 #pragma unroll
-    for (int v = 0; v < 4; ++v) ut[v] *= invJ;
+    for (int v = 0; v < 4; ++v) ut[v] *= sc;
     if constexpr (STAGE == 2) {
-        contract<n, S>(lds + 8 * S, sbase, i, j, sDm, ust);
+        contract<n, S>(lds + 8 * S, sbase, i, j, sD, ust);
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            ust[v] *= invJ;
+            ust[v] *= sc;
             Uc[v] = fma(1.0 / 3.0, ust[v], fma(1.0 / 6.0, ut[v], uN[v]));
         }
     } else {
@@ -465,7 +468,7 @@ __global__ __launch_bounds__((VGeo<N, EB>::NT), 2) void k_adj_records_md(AdjArgs
     using G_ = VGeo<N, EB>;
     constexpr int n = G_::n, NN = G_::NN;
     __shared__ alignas(16) double lds[G_::LDS];
-    __shared__ alignas(16) double sDm[G_::M];
+    __shared__ alignas(16) double sD[G_::M];
     const int tid = threadIdx.x;
     const int le = tid / NN, node = tid - (tid / NN) * NN;
     const int i = node % n, j = node / n;
@@ -475,14 +478,14 @@ __global__ __launch_bounds__((VGeo<N, EB>::NT), 2) void k_adj_records_md(AdjArgs
     const int lec = le < nel ? le : nel - 1;
     const int e = e0 + lec;
     const int sidx = lec * NN + node, sbase = lec * NN;
-    const DevConst* c = a.c;
+    const DevC c = dev_const(a.c);
     const double dt = a.dt, invJ = a.inv_jac[e];
     const size_t off = ((size_t)e * NN + node) * 4;
-    if (tid < NN) sDm[(tid / n) * G_::MS + tid % n] = -dt * c->D[tid / n][tid % n];
+    if (tid < NN) sD[(tid / n) * G_::MS + tid % n] = c->D[tid / n][tid % n];
     double uN[4], usn[4] = {0, 0, 0, 0}, ut[4], ust[4], Uc[4];
     load4(a.u + off, uN);
     if constexpr (STAGE == 2) load4(a.us + off, usn);
-    mdrk_adj_forward<N, EB, STAGE>(uN, usn, invJ, c->gamma - 1.0, i, j, act, sidx, sbase, lds, sDm, ut, ust, Uc);
+    mdrk_adj_forward<N, EB, STAGE>(uN, usn, -dt * invJ, c->gamma - 1.0, i, j, act, sidx, sbase, lds, sD, ut, ust, Uc);
     const int fx = (i == 0) ? 0 : ((i == n - 1) ? 1 : -1);
     const int fy = (j == 0) ? 2 : ((j == n - 1) ? 3 : -1);
     if (!act || (fx < 0 && fy < 0)) return;
@@ -510,7 +513,7 @@ __global__ __launch_bounds__((VGeo<N, EB>::NT), 2) void k_adjoint_md(AdjArgs a) 
     using G_ = VGeo<N, EB>;
     constexpr int n = G_::n, NN = G_::NN, S = G_::S;
     __shared__ alignas(16) double lds[G_::LDS];
-    __shared__ alignas(16) double sDm[G_::M], sDh[G_::M];
+    __shared__ alignas(16) double sD[G_::M], sDh[G_::M];
     const int tid = threadIdx.x;
     const int le = tid / NN, node = tid - (tid / NN) * NN;
     const int i = node % n, j = node / n;
@@ -520,20 +523,20 @@ __global__ __launch_bounds__((VGeo<N, EB>::NT), 2) void k_adjoint_md(AdjArgs a) 
     const int lec = le < nel ? le : nel - 1;
     const int e = e0 + lec;
     const int sidx = lec * NN + node, sbase = lec * NN;
-    const DevConst* c = a.c;
+    const DevC c = dev_const(a.c);
     const double gamma = c->gamma, gm1 = gamma - 1.0;
     const double dt = a.dt, invJ = a.inv_jac[e];
     const size_t off = ((size_t)e * NN + node) * 4;
     if (tid < NN) {
         const int q = (tid / n) * G_::MS + tid % n;
-        sDm[q] = -dt * c->D[tid / n][tid % n];
+        sD[q] = c->D[tid / n][tid % n];
         sDh[q] = c->Dhat[tid / n][tid % n];
     }
     double uN[4], usn[4] = {0, 0, 0, 0}, lam[4], ut[4], ust[4] = {0, 0, 0, 0}, Uc[4];
     load4(a.u + off, uN);
     if constexpr (STAGE == 2) load4(a.us + off, usn);
     load4(a.lam + off, lam);
-    mdrk_adj_forward<N, EB, STAGE>(uN, usn, invJ, gm1, i, j, act, sidx, sbase, lds, sDm, ut, ust, Uc);
+    mdrk_adj_forward<N, EB, STAGE>(uN, usn, -dt * invJ, gm1, i, j, act, sidx, sbase, lds, sD, ut, ust, Uc);
 
     // --- interface fluxes of this node's faces (the LW step's: jump on uⁿ, λ from Ũ)
     double sb[4], Fb[4] = {0, 0, 0, 0}, Gb[4] = {0, 0, 0, 0}, Ucb[4] = {0, 0, 0, 0}, ub[4] = {0, 0, 0, 0};
@@ -625,17 +628,17 @@ __global__ __launch_bounds__((VGeo<N, EB>::NT), 2) void k_adjoint_md(AdjArgs a) 
     {
         double t4[4];
 #pragma unroll
-        for (int v = 0; v < 4; ++v) t4[v] = invJ * utb[v];
+        for (int v = 0; v < 4; ++v) t4[v] = (-dt * invJ) * utb[v];
         if (act) put4<S>(ex1, sidx, t4);
         if constexpr (STAGE == 2) {
 #pragma unroll
-            for (int v = 0; v < 4; ++v) t4[v] = invJ * ustb[v];
+            for (int v = 0; v < 4; ++v) t4[v] = (-dt * invJ) * ustb[v];
             if (act) put4<S>(ex0, sidx, t4);
         }
     }
     __syncthreads();
     double cf[4], cg[4], wb[4];
-    contract_t<n, S>(ex1, sbase, i, j, sDm, cf, cg);
+    contract_t<n, S>(ex1, sbase, i, j, sD, cf, cg);
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
         f0b[v] += cf[v];
@@ -645,7 +648,7 @@ __global__ __launch_bounds__((VGeo<N, EB>::NT), 2) void k_adjoint_md(AdjArgs a) 
 #pragma unroll
     for (int v = 0; v < 4; ++v) ub[v] += wb[v];
     if constexpr (STAGE == 2) {
-        contract_t<n, S>(ex0, sbase, i, j, sDm, cf, cg);
+        contract_t<n, S>(ex0, sbase, i, j, sD, cf, cg);
         euler_fluxes_vjp(usn, gm1, cf, cg, wb);
 #pragma unroll
         for (int v = 0; v < 4; ++v) usb[v] += wb[v];
@@ -740,25 +743,24 @@ __device__ __forceinline__ double sc_face_alp(const double* L, const double* R, 
 // derivatives (KEEP), α_e and the subcell fluxes next to the node's faces.
 template <int N, int EB, bool KEEP>
 __device__ __forceinline__ void adj_forward_sc(const AdjArgs& a, const double* alpha_tmp, const double* uN, int e,
-                                               int i, int j, bool act, int sidx, int sbase, double* lds, double* sDm,
+                                               int i, int j, bool act, int sidx, int sbase, double* lds, double* sD,
                                                double* sDh, double* Uc, double* F, double* G, double* tder,
                                                double& alpha_e, double* fnlx, double* fnly) {
     using G_ = VGeo<N, EB>;
     constexpr int n = G_::n, NN = G_::NN, S = G_::S;
-    const DevConst* c = a.c;
+    const DevC c = dev_const(a.c);
     const double dt = a.dt, invJ = a.inv_jac[e], gamma = c->gamma, gm1 = gamma - 1.0;
     if (threadIdx.x < NN) {
         const int q = (threadIdx.x / n) * G_::MS + threadIdx.x % n;
-        sDm[q] = -dt * c->D[threadIdx.x / n][threadIdx.x % n];
+        sD[q] = c->D[threadIdx.x / n][threadIdx.x % n];
         sDh[q] = c->Dhat[threadIdx.x / n][threadIdx.x % n];
     }
     double vol[4];
-    if constexpr (N == 4)
-        lw4_element<N, EB, KEEP>(uN, dt, invJ, gm1, c, i, j, act, sidx, sbase, lds, lds + 8 * S, lds + 16 * S, sDm,
-                                 sDh, Uc, F, G, vol, tder);
-    else
-        lw3_element<N, EB, KEEP>(uN, dt, invJ, gm1, c, i, j, act, sidx, sbase, lds, lds + 8 * S, lds + 16 * S, sDm,
-                                 sDh, Uc, F, G, vol, tder);
+    // the last exchange is in s2 (lds + 16 S)
+    double* A = (N == 4) ? lds + 16 * S : lds + 8 * S;
+    double* B = (N == 4) ? lds + 8 * S : lds + 16 * S;
+    lw_element<N, EB, false, KEEP>(uN, nullptr, dt, -dt * invJ, c->gamma, i, j, act, sidx, sbase, A, B, sD, sDh, Uc, F, G,
+                                   vol, tder);
     alpha_e = alpha_tmp[e];
     if (c->alpha_smooth) {
 #pragma unroll
@@ -799,7 +801,7 @@ __global__ __launch_bounds__((VGeo<N, EB>::NT), 2) void k_adj_records_sc(AdjArgs
     using G_ = VGeo<N, EB>;
     constexpr int n = G_::n, NN = G_::NN;
     __shared__ alignas(16) double lds[G_::LDS];
-    __shared__ alignas(16) double sDm[G_::M], sDh[G_::M];
+    __shared__ alignas(16) double sD[G_::M], sDh[G_::M];
     const int tid = threadIdx.x;
     const int le = tid / NN, node = tid - (tid / NN) * NN;
     const int i = node % n, j = node / n;
@@ -812,12 +814,12 @@ __global__ __launch_bounds__((VGeo<N, EB>::NT), 2) void k_adj_records_sc(AdjArgs
     const size_t off = ((size_t)e * NN + node) * 4;
     double uN[4], Uc[4], F[4], G[4], fnlx[4] = {0, 0, 0, 0}, fnly[4] = {0, 0, 0, 0}, alpha_e;
     load4(a.u + off, uN);
-    adj_forward_sc<N, EB, false>(a, alpha_tmp, uN, e, i, j, act, sidx, sbase, lds, sDm, sDh, Uc, F, G, nullptr,
+    adj_forward_sc<N, EB, false>(a, alpha_tmp, uN, e, i, j, act, sidx, sbase, lds, sD, sDh, Uc, F, G, nullptr,
                                  alpha_e, fnlx, fnly);
     const int fx = (i == 0) ? 0 : ((i == n - 1) ? 1 : -1);
     const int fy = (j == 0) ? 2 : ((j == n - 1) ? 3 : -1);
     if (!act || (fx < 0 && fy < 0)) return;
-    const double invJ = a.inv_jac[e], gamma = a.c->gamma;
+    const double invJ = a.inv_jac[e], gamma = dev_const(a.c)->gamma;
     double lam[4], r[kAdjQSC];
     load4(a.lam + off, lam);
 #pragma unroll
@@ -837,7 +839,7 @@ __global__ __launch_bounds__((VGeo<N, EB>::NT), 1) void k_adjoint_sc(AdjArgs a, 
     using G_ = VGeo<N, EB>;
     constexpr int n = G_::n, NN = G_::NN, S = G_::S;
     __shared__ alignas(16) double lds[G_::LDS];
-    __shared__ alignas(16) double sDm[G_::M], sDh[G_::M];
+    __shared__ alignas(16) double sD[G_::M], sDh[G_::M];
     const int tid = threadIdx.x;
     const int le = tid / NN, node = tid - (tid / NN) * NN;
     const int i = node % n, j = node / n;
@@ -847,14 +849,14 @@ __global__ __launch_bounds__((VGeo<N, EB>::NT), 1) void k_adjoint_sc(AdjArgs a, 
     const int lec = le < nel ? le : nel - 1;
     const int e = e0 + lec;
     const int sidx = lec * NN + node, sbase = lec * NN;
-    const DevConst* c = a.c;
+    const DevC c = dev_const(a.c);
     const double gamma = c->gamma, gm1 = gamma - 1.0;
     const double dt = a.dt, invJ = a.inv_jac[e];
     const size_t off = ((size_t)e * NN + node) * 4;
     double uN[4], lam[4], Uc[4], F[4], G[4], ud[N][4], fnlx[4] = {0, 0, 0, 0}, fnly[4] = {0, 0, 0, 0}, alpha_e;
     load4(a.u + off, uN);
     load4(a.lam + off, lam);
-    adj_forward_sc<N, EB, true>(a, alpha_tmp, uN, e, i, j, act, sidx, sbase, lds, sDm, sDh, Uc, F, G, &ud[0][0],
+    adj_forward_sc<N, EB, true>(a, alpha_tmp, uN, e, i, j, act, sidx, sbase, lds, sD, sDh, Uc, F, G, &ud[0][0],
                                 alpha_e, fnlx, fnly);
     const bool blended = !(fabs(alpha_e) <= 1e-12);
 
@@ -1006,11 +1008,11 @@ __global__ __launch_bounds__((VGeo<N, EB>::NT), 1) void k_adjoint_sc(AdjArgs a, 
             buf ^= 1;
             double t4[4];
 #pragma unroll
-            for (int v = 0; v < 4; ++v) t4[v] = invJ * udb[k][v];
+            for (int v = 0; v < 4; ++v) t4[v] = (-dt * invJ) * udb[k][v];
             if (act) put4<S>(ex, sidx, t4);
             __syncthreads();
             double cf[4], cg[4];
-            contract_t<n, S>(ex, sbase, i, j, sDm, cf, cg);
+            contract_t<n, S>(ex, sbase, i, j, sD, cf, cg);
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
                 dxb[v] += cf[v];
@@ -1050,11 +1052,11 @@ __global__ __launch_bounds__((VGeo<N, EB>::NT), 1) void k_adjoint_sc(AdjArgs a, 
         double* ex = buf ? ex1 : ex0;
         double t4[4];
 #pragma unroll
-        for (int v = 0; v < 4; ++v) t4[v] = invJ * udb[0][v];
+        for (int v = 0; v < 4; ++v) t4[v] = (-dt * invJ) * udb[0][v];
         if (act) put4<S>(ex, sidx, t4);
         __syncthreads();
         double cf[4], cg[4];
-        contract_t<n, S>(ex, sbase, i, j, sDm, cf, cg);
+        contract_t<n, S>(ex, sbase, i, j, sD, cf, cg);
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
             F0b[v] += cf[v];

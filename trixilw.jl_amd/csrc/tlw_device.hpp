@@ -55,6 +55,8 @@ template <int N, int EB> struct VGeo {
     static constexpr int S = EB * NN;  // nodes of a workgroup: LDS stride of one exchanged pair of variables
     static constexpr int NT = ((EB * NN + 63) / 64) * 64;
     static constexpr int LDS = 3 * 8 * S;  // three exchange buffers
+    // two exchange buffers, the second large enough for the face records
+    static constexpr int LDS2 = 8 * S + (EB * 4 * n * kTraceQ > 8 * S ? EB * 4 * n * kTraceQ : 8 * S);
     static constexpr int MS = op_stride(n), M = n * MS;  // row stride and size of an operator in LDS
 };
 // Surface / reduction workgroup geometry: 128 threads.
@@ -122,6 +124,19 @@ struct DevState {
     int adaptive, nfail;
     long long nreject;
 };
+
+// Both structs as the kernels read them: constant for the whole launch (a kernel
+// that changes the state writes through the plain pointer, and to fields it does
+// not read), so that their fields come by scalar loads.  Through plain pointers
+// each one after a store is a vector load the wave waits for, with every load
+// in flight before it.
+using DevC = const __attribute__((address_space(4))) DevConst*;
+using DevS = const __attribute__((address_space(4))) DevState*;
+__device__ __forceinline__ DevC dev_const(const DevConst* p) { return (DevC)(uintptr_t)p; }
+__device__ __forceinline__ DevS dev_state(const DevState* p) { return (DevS)(uintptr_t)p; }
+// an array of the same kind (workgroup tables, neighbours)
+template <class T> using ConstArr = const __attribute__((address_space(4))) T*;
+template <class T> __device__ __forceinline__ ConstArr<T> const_arr(const T* p) { return (ConstArr<T>)(uintptr_t)p; }
 
 enum BufSel { SEL_EXPLICIT = 0, SEL_CUR = 1, SEL_OTHER = 2 };
 // RED_ADAPT: adaptive step (per-workgroup sums of the temporal errors and the
@@ -233,15 +248,15 @@ struct KArgs {
 };
 
 // ---------------------------------------------------------------------------
-// 1/x from the hardware reciprocal estimate and two Newton-Raphson steps
-// r <- r + r (1 - x r); the result is within a few ulp of the correctly
-// rounded reciprocal for the positive, normal densities it is applied to.
+// 1/x from the hardware reciprocal estimate r and one third-order step
+// r <- r + r (e + e²), e = 1 - x r: the estimate's relative error is below
+// 2^-24, so the step leaves e³ < 2^-72 and the result is rounded once, within
+// an ulp for the normal densities it is applied to.  Three FMAs on top of the
+// estimate (itself the time of four), where two Newton steps take four.
 __device__ __forceinline__ double rcp_nr(double x) {
-    double r = __builtin_amdgcn_rcp(x);
-    double e = fma(-x, r, 1.0);
-    r = fma(r, e, r);
-    e = fma(-x, r, 1.0);
-    return fma(r, e, r);
+    const double r = __builtin_amdgcn_rcp(x);
+    const double e = fma(-x, r, 1.0);
+    return fma(r, fma(e, e, e), r);
 }
 
 // Euler flux, both directions (Trixi flux(u, 1|2, CompressibleEulerEquations2D)).
@@ -259,6 +274,63 @@ __device__ __forceinline__ void euler_fluxes(const double* u, double gm1, double
     g[1] = m2 * v1;
     g[2] = m2 * v2 + p;
     g[3] = (E + p) * v2;
+}
+
+// The quadratic parts of both Euler fluxes,
+// q = (ρv1², ρv1v2, ρv2², (ρe+p)v1, (ρe+p)v2): the mass flux and the ρe inside p
+// are linear in u, so a flux difference over Taylor states needs these five
+// sums only (8 for two whole flux vectors), and its linear part is the time
+// derivative of u itself, free of cancellation.  kh = -(γ-1)/2.
+__device__ __forceinline__ void euler_q(const double* u, double gamma, double kh, double* q) {
+    const double ir = rcp_nr(u[0]);
+    const double v1 = u[1] * ir, v2 = u[2] * ir;
+    q[0] = u[1] * v1;
+    q[1] = u[1] * v2;
+    q[2] = u[2] * v2;
+    const double H = fma(gamma, u[3], kh * (q[0] + q[2]));  // ρe + p
+    q[3] = H * v1;
+    q[4] = H * v2;
+}
+// The flux pair of the sums q and the linear parts (l1, l2, lE) of ρv1, ρv2, ρe.
+__device__ __forceinline__ void euler_join(const double* q, double l1, double l2, double lE, double gm1, double kh,
+                                           double* f, double* g) {
+    const double p = fma(kh, q[0] + q[2], gm1 * lE);
+    f[0] = l1;
+    f[1] = q[0] + p;
+    f[2] = q[1];
+    f[3] = q[3];
+    g[0] = l2;
+    g[1] = q[1];
+    g[2] = q[2] + p;
+    g[3] = q[4];
+}
+
+// The Taylor states of the LW procedure, u(t + s dt) for s = 1, -1, 2, -2
+// (rows): level m adds kTaylor[s][m-1] = s^m/m! times the m-th derivative.
+__device__ constexpr double kTaylor[4][4] = {{1.0, 0.5, 1.0 / 6.0, 1.0 / 24.0},
+                                             {-1.0, 0.5, -1.0 / 6.0, 1.0 / 24.0},
+                                             {2.0, 2.0, 4.0 / 3.0, 2.0 / 3.0},
+                                             {-2.0, 2.0, -4.0 / 3.0, 2.0 / 3.0}};
+// The k-th time difference of the flux: Σ_s c[s] f(state s) + c[4] f(uⁿ), times
+// scale (calc_time_differences of kernels 3 and 4: five points for f_t, f_tt at
+// N = 4 and f_ttt, three for f_tt at N = 3; the 0.5 of f_tttt is the
+// reference's, dg_2d.jl:1203-1206).  The coefficients are integers or powers of
+// two, so that equal states cancel exactly (a rounded 2/3 leaves an ulp of the
+// flux, which the next levels' derivatives amplify); a division by 12 comes last.
+// linear: what the stencil gives of a linear function, times its derivative.
+struct TimeDiff {
+    double c[5], scale, linear;
+};
+template <int N> __device__ constexpr TimeDiff time_diff(int k) {
+    if (k == 1) return {{8.0, -8.0, -1.0, 1.0, 0.0}, 1.0 / 12.0, 1.0};
+    if (k == 2 && N == 4) return {{16.0, 16.0, -1.0, -1.0, -30.0}, 1.0 / 12.0, 1.0};
+    if (k == 2) return {{1.0, 1.0, 0.0, 0.0, -2.0}, 1.0, 1.0};
+    if (k == 3) return {{-1.0, 1.0, 0.5, -0.5, 0.0}, 1.0, 1.0};
+    return {{-2.0, -2.0, 0.5, 0.5, 3.0}, 1.0, 0.5};
+}
+// weight of the k-th derivative in Ũ and F̃: 1/(k+1)!
+__device__ constexpr double lw_weight(int k) {
+    return k == 0 ? 1.0 : k == 1 ? 0.5 : k == 2 ? 1.0 / 6.0 : k == 3 ? 1.0 / 24.0 : 1.0 / 120.0;
 }
 
 // ---------------------------------------------------------------------------
@@ -377,7 +449,7 @@ __device__ __forceinline__ void src_level_c(const SrcPt& p, double dt, int k, bo
 struct NsSrcPt {
     double sx, cx, sy, cy, g, g1, g2, t, gamma, mu, prandtl;
 };
-__device__ __forceinline__ NsSrcPt ns_src_point(double x, double y, double t, const DevConst* c) {
+__device__ __forceinline__ NsSrcPt ns_src_point(double x, double y, double t, DevC c) {
     constexpr double pi = 3.141592653589793, A = 0.5;
     NsSrcPt p;
     sincos_cw(pi * x, &p.sx, &p.cx);
@@ -543,8 +615,8 @@ __device__ __forceinline__ int julia_isapprox(double x, double y) {
 }
 
 // Boundary value functions of the time-averaged Dirichlet condition.
-__device__ inline void boundary_value(const DevConst* c, double x, double y, double t, double* u) {
-    const double* par = c->bc_par;
+__device__ inline void boundary_value(DevC c, double x, double y, double t, double* u) {
+    const auto* par = c->bc_par;
     double rho, v1, v2, p, gamma;
     if (c->bc_kind == kBcConvergenceTest) {
         // Trixi's initial_condition_convergence_test: ρ = ρv1 = ρv2 = φ, ρe = φ²
@@ -655,7 +727,7 @@ __device__ __forceinline__ void load4(const double* p, double* u) {
 // Boundary state of face node l of element e's face at GLL time level q (q = n:
 // the time t itself): the caller's table (kBcTable) or a built-in function.
 template <int n>
-__device__ __forceinline__ void boundary_state(const DevConst* c, const int* bidx, const double* btab, int levels,
+__device__ __forceinline__ void boundary_state(DevC c, const int* bidx, const double* btab, int levels,
                                                int e, int face, int l, int q, double x, double y, double t,
                                                double* u) {
     if (c->bc_kind == kBcTable) {
@@ -711,9 +783,9 @@ __device__ __forceinline__ double* sel_out(const KArgs& a, int cur) {
 // bid is the workgroup's index in its own table (blockIdx.x, or the index
 // within its half of a two-context launch).
 __device__ __forceinline__ int4 load_blk_at(const int4* t, int bid) {
-    const int4 b = t[bid];
-    return make_int4(__builtin_amdgcn_readfirstlane(b.x), __builtin_amdgcn_readfirstlane(b.y),
-                     __builtin_amdgcn_readfirstlane(b.z), 0);
+    const ConstArr<int> q = const_arr(reinterpret_cast<const int*>(t + bid));
+    return make_int4(__builtin_amdgcn_readfirstlane(q[0]), __builtin_amdgcn_readfirstlane(q[1]),
+                     __builtin_amdgcn_readfirstlane(q[2]), 0);
 }
 __device__ __forceinline__ int4 load_blk(const int4* t) { return load_blk_at(t, blockIdx.x); }
 
@@ -811,7 +883,7 @@ __device__ __forceinline__ void mh_face_pair(double* s, const double* u, double 
 // +Δt/2 J⁻¹ f(left) / hw[i] for 0 < i < n-1, -Δt/2 J⁻¹ f(right) / hw[i] for
 // i < n-1, then the same in y.
 template <int N, int S>
-__device__ __forceinline__ void mh_faces(const double* s1, int sidx, int i, int j, const double* u, const DevConst* c,
+__device__ __forceinline__ void mh_faces(const double* s1, int sidx, int i, int j, const double* u, DevC c,
                                          double beta, double dtmh, double invJ, double gm1, double* ql, double* qr,
                                          double* qd, double* qu) {
     constexpr int n = N + 1;
@@ -996,461 +1068,250 @@ __device__ __forceinline__ void node_speeds(const double* un, double gamma, doub
 
 // ---------------------------------------------------------------------------
 // Element volume computations.  Each fills uN (state), Uc (Ũ), F, G (F̃) and
-// vol (D̂F̃ contraction) for the calling node; the final F̃ exchange is in s2,
-// so s0 and s1 are free once every thread has passed the last barrier.
+// vol (D̂F̃ contraction) for the calling node; sD and sDh hold D and D̂, and
+// sc = -dt J⁻¹ turns a D contraction into the next time derivative.  Exchanges alternate between two
+// LDS buffers A and B, one barrier each: a buffer is rewritten two exchanges
+// later, when every lane has passed its contraction.
 
-// lw_volume_kernel_4!, dg_2d.jl:918-1267 (the temporal-error estimate at
-// 1183-1199, 1251-1265 is an adaptive-mode output and is not computed).
+// Contravariant fluxes of a Cartesian pair: Ja¹·(f, g), Ja²·(f, g)
+// (contravariant_flux, structured/dg_2d.jl:550-556).
+__device__ __forceinline__ void to_contravariant(const double* J, const double* f, const double* g, double* fc,
+                                                 double* gc) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        fc[v] = fma(J[0], f[v], J[1] * g[v]);
+        gc[v] = fma(J[2], f[v], J[3] * g[v]);
+    }
+}
+// The node's flux pair into an exchange buffer, contravariant on a curvilinear mesh.
+template <int S, bool CURV>
+__device__ __forceinline__ void put_fluxes(double* s, int sidx, bool act, const double* J, const double* f,
+                                           const double* g) {
+    if constexpr (CURV) {
+        double cx[4], cy[4];
+        to_contravariant(J, f, g, cx, cy);
+        if (act) put8<S>(s, sidx, cx, cy);
+    } else {
+        if (act) put8<S>(s, sidx, f, g);
+    }
+}
+
+// lw_volume_kernel_3!/4!, dg_2d.jl:674-916, 918-1267, and on a curvilinear mesh
+// (CURV) structured/dg_2d.jl:1379-2105: the same procedure with the node's
+// contravariant vectors J = (Ja11, Ja12, Ja21, Ja22) turning each Cartesian
+// flux derivative for the contractions, while the Cartesian time averages F̃, G̃
+// feed the face records.  The last exchange is in A (N = 4) or B (N = 3).
+// Bound by FP64 issue with the LDS contractions beside it: per node and level
+// four euler_q with five sums each (22 issue slots + 4 for the estimate of 1/ρ),
+// 26 LDS loads and 4 stores.  LW N=4 1024², 10 elements per workgroup: whole
+// flux vectors, three buffers and plain loads of the constants 1283 us, this form
+// with the early loads of volume_body 1138 us.
 // With KEEP, tder receives the time derivatives ut, utt, ... (4 per order),
 // the intermediates an adjoint sweep needs.
 // With terr, the temporal error of the node for the adaptive controller
-// (dg_2d.jl:1183-1199, 1251-1265): u_np1 = u - dt J⁻¹ D F̃ and u_np1_low, the
-// same with F̃ before the f_tttt term, compared variable by variable as
+// (dg_2d.jl:1183-1199, 1251-1265; structured/dg_2d.jl:1595-1681, 1983-2077):
+// u_np1 = u - dt J⁻¹ D F̃ and u_np1_low, the same with F̃ before the last flux
+// derivative's term, compared variable by variable as
 // ((u_np1 - u_np1_low) / (abstol + reltol max(|u_np1|, |u_np1_low|)))², summed.
 // terr must be uniformly null or non-null over the workgroup (it adds barriers).
 // With SRC, the source terms of the node (*sp) enter every time derivative as
 // dt times the source's own difference (dg_2d.jl:980-987, 1033-1045, 1093-1103,
-// 1148-1160) and Ssrc receives S = s + s_t/2 + s_tt/6 + s_ttt/24 + s_tttt/120
-// (1228-1247), which the caller adds to the residual.
-template <int N, int EB, bool KEEP = false, bool SRC = false>
-__device__ __forceinline__ void lw4_element(const double* uN, double dt, double invJ, double gm1, const DevConst* c,
-                                            int i, int j, bool act, int sidx, int sbase, double* s0, double* s1,
-                                            double* s2, const double* sDm, const double* sDh, double* Uc, double* F,
-                                            double* G, double* vol, double* tder = nullptr, double* terr = nullptr,
-                                            double abstol = 0.0, double reltol = 0.0, const SrcPt* sp = nullptr,
-                                            double* Ssrc = nullptr) {
+// 1148-1160; five-point s_tt in the curvilinear kernel 4) and Ssrc receives
+// S = s + s_t/2 + s_tt/6 + ... (1228-1247), which the caller adds to the residual.
+template <int N, int EB, bool CURV = false, bool KEEP = false, bool SRC = false>
+__device__ __forceinline__ void lw_element(const double* uN, const double* J, double dt, double sc, double gamma,
+                                           int i, int j, bool act, int sidx, int sbase, double* A, double* B,
+                                           const double* sD, const double* sDh, double* Uc, double* F, double* G,
+                                           double* vol, double* tder = nullptr, double* terr = nullptr,
+                                           double abstol = 0.0, double reltol = 0.0, const SrcPt* sp = nullptr,
+                                           double* Ssrc = nullptr) {
     using G_ = VGeo<N, EB>;
     constexpr int n = G_::n, S = G_::S;
-    euler_fluxes(uN, gm1, F, G);
-    if (act) put8<S>(s0, sidx, F, G);
-    __syncthreads();
-    double ut[4], sk[4];
-    contract<n, S>(s0, sbase, i, j, sDm, ut);
-    if constexpr (SRC) src_eval(*sp, 0.0, sk);
-    double up[4], um[4], upp[4], umm[4];
+    const double gm1 = gamma - 1.0, kh = -0.5 * gm1;
+    double q0[5], sum[5], st[4][4], w[4], sk[4] = {0.0, 0.0, 0.0, 0.0};
+    euler_q(uN, gamma, kh, q0);
+    euler_join(q0, uN[1], uN[2], uN[3], gm1, kh, F, G);
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        ut[v] *= invJ;
-        if constexpr (SRC) {
-            ut[v] = fma(dt, sk[v], ut[v]);
-            Ssrc[v] = sk[v];
+    for (int m = 0; m < 5; ++m) sum[m] = q0[m];
+#pragma unroll
+    for (int k = 1; k <= N; ++k) {
+        // F, G: the (k-1)-th time difference of the flux pair
+        double* buf = (k & 1) ? A : B;
+        put_fluxes<S, CURV>(buf, sidx, act, J, F, G);
+        __syncthreads();
+        contract<n, S>(buf, sbase, i, j, sD, w);
+        if constexpr (SRC) src_level_c(*sp, dt, k - 1, CURV && N == 4, sk, Ssrc, lw_weight(k - 1));
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            w[v] *= sc;
+            if constexpr (SRC) w[v] = fma(dt, sk[v], w[v]);
+            if constexpr (KEEP) tder[4 * (k - 1) + v] = w[v];
+            Uc[v] = fma(lw_weight(k), w[v], k == 1 ? uN[v] : Uc[v]);
+#pragma unroll
+            for (int s = 0; s < 4; ++s) st[s][v] = fma(kTaylor[s][k - 1], w[v], k == 1 ? uN[v] : st[s][v]);
         }
-        if constexpr (KEEP) tder[v] = ut[v];
-        Uc[v] = fma(0.5, ut[v], uN[v]);
-        up[v] = uN[v] + ut[v];
-        um[v] = uN[v] - ut[v];
-        umm[v] = fma(-2.0, ut[v], uN[v]);
-        upp[v] = fma(2.0, ut[v], uN[v]);
-    }
-    double fa[4], ga[4], dx[4], dy[4];
-    // stage 1: f_t = (-f(u+2) + 8 f(u+1) - 8 f(u-1) + f(u-2)) / 12
-    euler_fluxes(upp, gm1, fa, ga);
+        constexpr TimeDiff tds[5] = {{}, time_diff<N>(1), time_diff<N>(2), time_diff<N>(3), time_diff<N>(4)};
+        const TimeDiff td = tds[k];
+        double d[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, q[5];
+        // in the order of time, uⁿ between u(t + dt) and u(t - dt): small partial sums
 #pragma unroll
-    for (int v = 0; v < 4; ++v) { dx[v] = -fa[v]; dy[v] = -ga[v]; }
-    euler_fluxes(up, gm1, fa, ga);
+        for (int r = 0; r < 5; ++r) {
+            const int s = r == 0 ? 2 : r == 1 ? 0 : r == 2 ? 4 : r == 3 ? 1 : 3;
+            if (td.c[s] == 0.0) continue;
+            if (s < 4) euler_q(st[s & 3], gamma, kh, q);
 #pragma unroll
-    for (int v = 0; v < 4; ++v) { dx[v] = fma(8.0, fa[v], dx[v]); dy[v] = fma(8.0, ga[v], dy[v]); }
-    euler_fluxes(um, gm1, fa, ga);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) { dx[v] = fma(-8.0, fa[v], dx[v]); dy[v] = fma(-8.0, ga[v], dy[v]); }
-    euler_fluxes(umm, gm1, fa, ga);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        dx[v] = (1.0 / 12.0) * (dx[v] + fa[v]);
-        dy[v] = (1.0 / 12.0) * (dy[v] + ga[v]);
-        F[v] = fma(0.5, dx[v], F[v]);
-        G[v] = fma(0.5, dy[v], G[v]);
-    }
-    if (act) put8<S>(s1, sidx, dx, dy);
-    __syncthreads();
-    double uk[4];
-    contract<n, S>(s1, sbase, i, j, sDm, uk);
-    if constexpr (SRC) src_t5(*sp, 0.0, dt, sk);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        double w = uk[v] * invJ;  // utt
-        if constexpr (SRC) {
-            w = fma(dt, sk[v], w);
-            Ssrc[v] = fma(0.5, sk[v], Ssrc[v]);
+            for (int m = 0; m < 5; ++m) d[m] = fma(td.c[s], s < 4 ? q[m] : q0[m], d[m]);
         }
-        if constexpr (KEEP) tder[4 + v] = w;
-        Uc[v] = fma(1.0 / 6.0, w, Uc[v]);
-        up[v] = fma(0.5, w, up[v]);
-        um[v] = fma(0.5, w, um[v]);
-        upp[v] = fma(2.0, w, upp[v]);
-        umm[v] = fma(2.0, w, umm[v]);
-    }
-    // stage 2: f_tt = (-f(u+2) + 16 f(u+1) - 30 f + 16 f(u-1) - f(u-2)) / 12
-    euler_fluxes(upp, gm1, fa, ga);
 #pragma unroll
-    for (int v = 0; v < 4; ++v) { dx[v] = -fa[v]; dy[v] = -ga[v]; }
-    euler_fluxes(up, gm1, fa, ga);
-    double f0[4], g0[4];
-    get4<S>(s0, sidx, f0);
-    get4<S>(s0 + 4 * S, sidx, g0);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        dx[v] = fma(16.0, fa[v], dx[v]);
-        dy[v] = fma(16.0, ga[v], dy[v]);
-        dx[v] = fma(-30.0, f0[v], dx[v]);
-        dy[v] = fma(-30.0, g0[v], dy[v]);
-    }
-    euler_fluxes(um, gm1, fa, ga);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) { dx[v] = fma(16.0, fa[v], dx[v]); dy[v] = fma(16.0, ga[v], dy[v]); }
-    euler_fluxes(umm, gm1, fa, ga);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        dx[v] = (1.0 / 12.0) * (dx[v] - fa[v]);
-        dy[v] = (1.0 / 12.0) * (dy[v] - ga[v]);
-        F[v] = fma(1.0 / 6.0, dx[v], F[v]);
-        G[v] = fma(1.0 / 6.0, dy[v], G[v]);
-    }
-    if (act) put8<S>(s2, sidx, dx, dy);
-    __syncthreads();
-    contract<n, S>(s2, sbase, i, j, sDm, uk);
-    if constexpr (SRC) src_tt3(*sp, dt, sk);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        double w = uk[v] * invJ;  // uttt
-        if constexpr (SRC) {
-            w = fma(dt, sk[v], w);
-            Ssrc[v] = fma(1.0 / 6.0, sk[v], Ssrc[v]);
+        for (int m = 0; m < 5; ++m) {
+            if (td.scale != 1.0) d[m] *= td.scale;
+            sum[m] = fma(lw_weight(k), d[m], sum[m]);
         }
-        if constexpr (KEEP) tder[8 + v] = w;
-        Uc[v] = fma(1.0 / 24.0, w, Uc[v]);
-        um[v] = fma(-1.0 / 6.0, w, um[v]);
-        up[v] = fma(1.0 / 6.0, w, up[v]);
-        umm[v] = fma(-4.0 / 3.0, w, umm[v]);
-        upp[v] = fma(4.0 / 3.0, w, upp[v]);
+        if (k < N || terr)
+            euler_join(d, td.linear * w[1], td.linear * w[2], td.linear * w[3], gm1, kh, F, G);
     }
-    // stage 3: f_ttt = (f(u+2) - 2 f(u+1) + 2 f(u-1) - f(u-2)) / 2
-    euler_fluxes(upp, gm1, fa, ga);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) { dx[v] = fa[v]; dy[v] = ga[v]; }
-    euler_fluxes(up, gm1, fa, ga);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) { dx[v] = fma(-2.0, fa[v], dx[v]); dy[v] = fma(-2.0, ga[v], dy[v]); }
-    euler_fluxes(um, gm1, fa, ga);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) { dx[v] = fma(2.0, fa[v], dx[v]); dy[v] = fma(2.0, ga[v], dy[v]); }
-    euler_fluxes(umm, gm1, fa, ga);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        dx[v] = 0.5 * (dx[v] - fa[v]);
-        dy[v] = 0.5 * (dy[v] - ga[v]);
-        F[v] = fma(1.0 / 24.0, dx[v], F[v]);
-        G[v] = fma(1.0 / 24.0, dy[v], G[v]);
-    }
-    if (act) put8<S>(s1, sidx, dx, dy);
-    __syncthreads();
-    contract<n, S>(s1, sbase, i, j, sDm, uk);
-    if constexpr (SRC) src_ttt5(*sp, dt, sk);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        double w = uk[v] * invJ;  // utttt
-        if constexpr (SRC) {
-            w = fma(dt, sk[v], w);
-            Ssrc[v] = fma(1.0 / 24.0, sk[v], Ssrc[v]);
-        }
-        if constexpr (KEEP) tder[12 + v] = w;
-        Uc[v] = fma(1.0 / 120.0, w, Uc[v]);
-        um[v] = fma(1.0 / 24.0, w, um[v]);
-        up[v] = fma(1.0 / 24.0, w, up[v]);
-        umm[v] = fma(2.0 / 3.0, w, umm[v]);
-        upp[v] = fma(2.0 / 3.0, w, upp[v]);
-    }
-    // stage 4: f_tttt = 0.5 (f(u+2) - 4 f(u+1) + 6 f - 4 f(u-1) + f(u-2)); the
-    // factor 0.5 is the reference's (dg_2d.jl:1203-1206)
-    euler_fluxes(upp, gm1, fa, ga);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) { dx[v] = fa[v]; dy[v] = ga[v]; }
-    euler_fluxes(up, gm1, fa, ga);
-    get4<S>(s0, sidx, f0);
-    get4<S>(s0 + 4 * S, sidx, g0);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        dx[v] = fma(-4.0, fa[v], dx[v]);
-        dy[v] = fma(-4.0, ga[v], dy[v]);
-        dx[v] = fma(6.0, f0[v], dx[v]);
-        dy[v] = fma(6.0, g0[v], dy[v]);
-    }
-    euler_fluxes(um, gm1, fa, ga);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) { dx[v] = fma(-4.0, fa[v], dx[v]); dy[v] = fma(-4.0, ga[v], dy[v]); }
-    euler_fluxes(umm, gm1, fa, ga);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        dx[v] = 0.5 * (dx[v] + fa[v]);
-        dy[v] = 0.5 * (dy[v] + ga[v]);
-        F[v] = fma(1.0 / 120.0, dx[v], F[v]);
-        G[v] = fma(1.0 / 120.0, dy[v], G[v]);
-    }
-    if (act) put8<S>(s2, sidx, F, G);
-    // s0 is read only at the own node since the first contraction: it takes f_tttt
-    if (terr && act) put8<S>(s0, sidx, dx, dy);
-    __syncthreads();
-    contract<n, S>(s2, sbase, i, j, sDh, vol);
-    if constexpr (SRC) {
-        src_tttt5(*sp, dt, sk);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) Ssrc[v] = fma(1.0 / 120.0, sk[v], Ssrc[v]);
-    }
+    // the source's last difference enters S only
+    if constexpr (SRC) src_level_c(*sp, dt, N, CURV && N == 4, sk, Ssrc, lw_weight(N));
+    double* last = (N & 1) ? B : A;   // the exchange of F̃
+    double* other = (N & 1) ? A : B;
     if (terr) {
+        __syncthreads();  // the last contraction has read this buffer
+        put_fluxes<S, CURV>(other, sidx, act, J, F, G);
+    }
+    // the linear parts of F̃: those of Ũ, up to the factor the last stencil puts on them
+    constexpr double miss = lw_weight(N) * (1.0 - time_diff<N>(N).linear);
+    double l[4];
+#pragma unroll
+    for (int v = 1; v < 4; ++v) l[v] = miss == 0.0 ? Uc[v] : fma(-miss, w[v], Uc[v]);
+    euler_join(sum, l[1], l[2], l[3], gm1, kh, F, G);
+    put_fluxes<S, CURV>(last, sidx, act, J, F, G);
+    __syncthreads();
+    contract<n, S>(last, sbase, i, j, sDh, vol);
+    if (terr) {
+        // one contraction at a time: interleaved, their loads spill 23 registers
         double a1[4], a2[4];
-        contract<n, S>(s2, sbase, i, j, sDm, a1);  // -dt D F̃
-        contract<n, S>(s0, sbase, i, j, sDm, a2);  // -dt D f_tttt
-        // u_np1 - u_np1_low is formed as the contraction of the f_tttt term itself,
+        __builtin_amdgcn_sched_barrier(0);
+        contract<n, S>(last, sbase, i, j, sD, a1);  // D F̃
+        __builtin_amdgcn_sched_barrier(0);
+        contract<n, S>(other, sbase, i, j, sD, a2);  // D of the last flux derivative
+        // u_np1 - u_np1_low is formed as the contraction of the last term itself,
         // not as a difference of the two updates (which cancels to ~1e-7 relative)
         double e = 0.0;
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            const double d = invJ * ((1.0 / 120.0) * a2[v]);
-            const double hi = fma(invJ, a1[v], uN[v]);
+            const double d = sc * (lw_weight(N) * a2[v]);
+            const double hi = fma(sc, a1[v], uN[v]);
             const double lo = hi - d;
             const double r = d / (abstol + reltol * dmax(fabs(hi), fabs(lo)));
             e = fma(r, r, e);
         }
         *terr = e;
-        __syncthreads();  // s0 is reused for the face records
+        __syncthreads();  // both buffers are reused for the face records
     }
 }
 
-// lw_volume_kernel_3!, dg_2d.jl:674-916
-// With KEEP, tder receives the time derivatives ut, utt, ... (4 per order),
-// the intermediates an adjoint sweep needs.  With SRC, source terms as in
-// lw4_element (732-740, 785-797, 841-851, 891-911): S = s + s_t/2 + s_tt/6 +
-// s_ttt/24.
-template <int N, int EB, bool KEEP = false, bool SRC = false>
-__device__ __forceinline__ void lw3_element(const double* uN, double dt, double invJ, double gm1, const DevConst* c,
-                                            int i, int j, bool act, int sidx, int sbase, double* s0, double* s1,
-                                            double* s2, const double* sDm, const double* sDh, double* Uc, double* F,
-                                            double* G, double* vol, double* tder = nullptr,
-                                            const SrcPt* sp = nullptr, double* Ssrc = nullptr) {
+// acc += weight · f_t of the two-level Taylor states u ± ut, u ± 2ut
+// (five euler_q sums; the linear part of f_t is ut)
+__device__ __forceinline__ void mdrk_ft(const double* u, const double* ut, double gamma, double kh, double weight,
+                                        double* acc) {
+    constexpr TimeDiff td = time_diff<4>(1);
+    double d[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, q[5], w[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int s = r == 0 ? 2 : r == 1 ? 0 : r == 2 ? 1 : 3;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) w[v] = fma(kTaylor[s][0], ut[v], u[v]);
+        euler_q(w, gamma, kh, q);
+#pragma unroll
+        for (int m = 0; m < 5; ++m) d[m] = fma(td.c[s], q[m], d[m]);
+    }
+#pragma unroll
+    for (int m = 0; m < 5; ++m) acc[m] = fma(weight * td.scale, d[m], acc[m]);
+}
+
+// mdrk_kernel_1!, tree/multi_derivative_2d.jl:263-420 and (CURV)
+// structured/multi_derivative_2d.jl:82-243: F̃ = f/2 + f_t/8, Ũ = u/2 + ut/8, ut
+// from the contravariant fluxes on a curvilinear mesh.  F2 = f + f_t/6 and
+// U2 = u + ut/6 are recomputed by the stage-2 kernel instead of being stored.
+// With SRC (323-379; structured 146-200): ut gets dt s(t), and
+// Ssrc = s/2 + s_t/8.  The last exchange is in B.
+template <int N, int EB, bool CURV = false, bool SRC = false>
+__device__ __forceinline__ void mdrk1_element(const double* uN, const double* J, double dt, double sc, double gamma,
+                                              int i, int j, bool act, int sidx, int sbase, double* A, double* B,
+                                              const double* sD, const double* sDh, double* Uc, double* F, double* G,
+                                              double* vol, const SrcPt* sp = nullptr, double* Ssrc = nullptr) {
     using G_ = VGeo<N, EB>;
     constexpr int n = G_::n, S = G_::S;
-    euler_fluxes(uN, gm1, F, G);
-    if (act) put8<S>(s0, sidx, F, G);
+    const double gm1 = gamma - 1.0, kh = -0.5 * gm1;
+    double q[5], ut[4];
+    euler_q(uN, gamma, kh, q);
+    euler_join(q, uN[1], uN[2], uN[3], gm1, kh, F, G);
+    put_fluxes<S, CURV>(A, sidx, act, J, F, G);
     __syncthreads();
-    double ut[4], sk[4];
-    contract<n, S>(s0, sbase, i, j, sDm, ut);
-    if constexpr (SRC) src_eval(*sp, 0.0, sk);
-    double up[4], um[4], upp[4], umm[4];
+    contract<n, S>(A, sbase, i, j, sD, ut);
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        ut[v] *= invJ;
-        if constexpr (SRC) {
-            ut[v] = fma(dt, sk[v], ut[v]);
-            Ssrc[v] = sk[v];
-        }
-        if constexpr (KEEP) tder[v] = ut[v];
-        Uc[v] = fma(0.5, ut[v], uN[v]);
-        up[v] = uN[v] + ut[v];
-        um[v] = uN[v] - ut[v];
-        umm[v] = fma(-2.0, ut[v], uN[v]);
-        upp[v] = fma(2.0, ut[v], uN[v]);
-    }
-    double fa[4], ga[4], dx[4], dy[4];
-    euler_fluxes(upp, gm1, fa, ga);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) { dx[v] = -fa[v]; dy[v] = -ga[v]; }
-    euler_fluxes(up, gm1, fa, ga);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) { dx[v] = fma(8.0, fa[v], dx[v]); dy[v] = fma(8.0, ga[v], dy[v]); }
-    euler_fluxes(um, gm1, fa, ga);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) { dx[v] = fma(-8.0, fa[v], dx[v]); dy[v] = fma(-8.0, ga[v], dy[v]); }
-    euler_fluxes(umm, gm1, fa, ga);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        dx[v] = (1.0 / 12.0) * (dx[v] + fa[v]);
-        dy[v] = (1.0 / 12.0) * (dy[v] + ga[v]);
-        F[v] = fma(0.5, dx[v], F[v]);
-        G[v] = fma(0.5, dy[v], G[v]);
-    }
-    if (act) put8<S>(s1, sidx, dx, dy);
-    __syncthreads();
-    double uk[4];
-    contract<n, S>(s1, sbase, i, j, sDm, uk);
-    if constexpr (SRC) src_t5(*sp, 0.0, dt, sk);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        double w = uk[v] * invJ;  // utt
-        if constexpr (SRC) {
-            w = fma(dt, sk[v], w);
-            Ssrc[v] = fma(0.5, sk[v], Ssrc[v]);
-        }
-        if constexpr (KEEP) tder[4 + v] = w;
-        Uc[v] = fma(1.0 / 6.0, w, Uc[v]);
-        up[v] = fma(0.5, w, up[v]);
-        um[v] = fma(0.5, w, um[v]);
-        upp[v] = fma(2.0, w, upp[v]);
-        umm[v] = fma(2.0, w, umm[v]);
-    }
-    // f_tt = f(u+1) - 2 f + f(u-1)
-    euler_fluxes(up, gm1, fa, ga);
-    double f0[4], g0[4];
-    get4<S>(s0, sidx, f0);
-    get4<S>(s0 + 4 * S, sidx, g0);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        dx[v] = fma(-2.0, f0[v], fa[v]);
-        dy[v] = fma(-2.0, g0[v], ga[v]);
-    }
-    euler_fluxes(um, gm1, fa, ga);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        dx[v] = dx[v] + fa[v];
-        dy[v] = dy[v] + ga[v];
-        F[v] = fma(1.0 / 6.0, dx[v], F[v]);
-        G[v] = fma(1.0 / 6.0, dy[v], G[v]);
-    }
-    if (act) put8<S>(s2, sidx, dx, dy);
-    __syncthreads();
-    contract<n, S>(s2, sbase, i, j, sDm, uk);
-    if constexpr (SRC) src_tt3(*sp, dt, sk);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        double w = uk[v] * invJ;  // uttt
-        if constexpr (SRC) {
-            w = fma(dt, sk[v], w);
-            Ssrc[v] = fma(1.0 / 6.0, sk[v], Ssrc[v]);
-        }
-        if constexpr (KEEP) tder[8 + v] = w;
-        Uc[v] = fma(1.0 / 24.0, w, Uc[v]);
-        um[v] = fma(-1.0 / 6.0, w, um[v]);
-        up[v] = fma(1.0 / 6.0, w, up[v]);
-        umm[v] = fma(-4.0 / 3.0, w, umm[v]);
-        upp[v] = fma(4.0 / 3.0, w, upp[v]);
-    }
-    // f_ttt = (f(u+2) - 2 f(u+1) + 2 f(u-1) - f(u-2)) / 2
-    euler_fluxes(upp, gm1, fa, ga);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) { dx[v] = fa[v]; dy[v] = ga[v]; }
-    euler_fluxes(up, gm1, fa, ga);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) { dx[v] = fma(-2.0, fa[v], dx[v]); dy[v] = fma(-2.0, ga[v], dy[v]); }
-    euler_fluxes(um, gm1, fa, ga);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) { dx[v] = fma(2.0, fa[v], dx[v]); dy[v] = fma(2.0, ga[v], dy[v]); }
-    euler_fluxes(umm, gm1, fa, ga);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        dx[v] = 0.5 * (dx[v] - fa[v]);
-        dy[v] = 0.5 * (dy[v] - ga[v]);
-        F[v] = fma(1.0 / 24.0, dx[v], F[v]);
-        G[v] = fma(1.0 / 24.0, dy[v], G[v]);
-    }
-    __syncthreads();  // every thread has finished reading s2 before it is reused
-    if (act) put8<S>(s2, sidx, F, G);
-    __syncthreads();
-    contract<n, S>(s2, sbase, i, j, sDh, vol);
+    for (int v = 0; v < 4; ++v) ut[v] *= sc;
     if constexpr (SRC) {
-        src_ttt5(*sp, dt, sk);
+        double s[4], sd[4];
+        src_eval(*sp, 0.0, s);
+        src_t5(*sp, 0.0, dt, sd);
 #pragma unroll
-        for (int v = 0; v < 4; ++v) Ssrc[v] = fma(1.0 / 24.0, sk[v], Ssrc[v]);
+        for (int v = 0; v < 4; ++v) {
+            ut[v] = fma(dt, s[v], ut[v]);
+            Ssrc[v] = fma(0.125, sd[v], 0.5 * s[v]);
+        }
     }
+#pragma unroll
+    for (int m = 0; m < 5; ++m) q[m] *= 0.5;
+    mdrk_ft(uN, ut, gamma, kh, 0.125, q);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) Uc[v] = fma(0.125, ut[v], 0.5 * uN[v]);
+    euler_join(q, Uc[1], Uc[2], Uc[3], gm1, kh, F, G);
+    put_fluxes<S, CURV>(B, sidx, act, J, F, G);
+    __syncthreads();
+    contract<n, S>(B, sbase, i, j, sDh, vol);
 }
 
-// f_t of the two-level Taylor states u ± ut, u ± 2ut:
-// (-f(u+2) + 8 f(u+1) - 8 f(u-1) + f(u-2)) / 12
-__device__ __forceinline__ void mdrk_ft(const double* u, const double* ut, double gm1, double* dx, double* dy) {
-    double w[4], fa[4], ga[4];
-#pragma unroll
-    for (int v = 0; v < 4; ++v) w[v] = fma(2.0, ut[v], u[v]);
-    euler_fluxes(w, gm1, fa, ga);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) { dx[v] = -fa[v]; dy[v] = -ga[v]; w[v] = u[v] + ut[v]; }
-    euler_fluxes(w, gm1, fa, ga);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) { dx[v] = fma(8.0, fa[v], dx[v]); dy[v] = fma(8.0, ga[v], dy[v]); w[v] = u[v] - ut[v]; }
-    euler_fluxes(w, gm1, fa, ga);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        dx[v] = fma(-8.0, fa[v], dx[v]);
-        dy[v] = fma(-8.0, ga[v], dy[v]);
-        w[v] = fma(-2.0, ut[v], u[v]);
-    }
-    euler_fluxes(w, gm1, fa, ga);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        dx[v] = (1.0 / 12.0) * (dx[v] + fa[v]);
-        dy[v] = (1.0 / 12.0) * (dy[v] + ga[v]);
-    }
-}
-
-// mdrk_kernel_1!, tree/multi_derivative_2d.jl:263-420: F̃ = f/2 + f_t/8,
-// Ũ = u/2 + ut/8.  F2 = f + f_t/6 and U2 = u + ut/6 are recomputed by the
-// stage-2 kernel instead of being stored.  With SRC (323-379): ut gets
-// dt s(t), and Ssrc = s/2 + s_t/8.
-template <int N, int EB, bool SRC = false>
-__device__ __forceinline__ void mdrk1_element(const double* uN, double dt, double invJ, double gm1, const DevConst* c,
-                                              int i, int j, bool act, int sidx, int sbase, double* s0, double* s1,
-                                              double* s2, const double* sDm, const double* sDh, double* Uc,
+// mdrk_kernel_2!, tree/multi_derivative_2d.jl:423-555 and (CURV)
+// structured/multi_derivative_2d.jl:245-445: F̃ = F2 + f_t(us)/3, Ũ = U2 + ust/3
+// with F2, U2 recomputed from uⁿ.  With SRC on a TreeMesh (487-522): the
+// recomputed stage-1 ut gets dt s(t) and S2 = s + s_t/6; ust gets dt s(t + dt/2),
+// and Ssrc = S2 + s_t(t + dt/2)/3.  On a StructuredMesh (326-339, 358-385): ut
+// and ust += dt s(t); Ssrc = s + s_t/3 about t, the reference's stage 2
+// overwriting the S2 it loads (stage 1's s + s_t/6) with s.  The last exchange
+// is in A, behind a barrier of its own (both buffers have just been read).
+template <int N, int EB, bool CURV = false, bool SRC = false>
+__device__ __forceinline__ void mdrk2_element(const double* uN, const double* usn, const double* J, double dt,
+                                              double sc, double gamma, int i, int j, bool act, int sidx, int sbase,
+                                              double* A, double* B, const double* sD, const double* sDh, double* Uc,
                                               double* F, double* G, double* vol, const SrcPt* sp = nullptr,
                                               double* Ssrc = nullptr) {
     using G_ = VGeo<N, EB>;
     constexpr int n = G_::n, S = G_::S;
-    double f[4], g[4];
-    euler_fluxes(uN, gm1, f, g);
-    if (act) put8<S>(s0, sidx, f, g);
+    const double gm1 = gamma - 1.0, kh = -0.5 * gm1;
+    double q[5], qs[5], ut[4], ust[4];
+    euler_q(uN, gamma, kh, q);
+    euler_join(q, uN[1], uN[2], uN[3], gm1, kh, F, G);
+    put_fluxes<S, CURV>(A, sidx, act, J, F, G);
+    euler_q(usn, gamma, kh, qs);
+    euler_join(qs, usn[1], usn[2], usn[3], gm1, kh, F, G);
+    put_fluxes<S, CURV>(B, sidx, act, J, F, G);
     __syncthreads();
-    double ut[4];
-    contract<n, S>(s0, sbase, i, j, sDm, ut);
-    double sk[4];
-    if constexpr (SRC) src_eval(*sp, 0.0, sk);
+    contract<n, S>(A, sbase, i, j, sD, ut);
+    contract<n, S>(B, sbase, i, j, sD, ust);
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        ut[v] *= invJ;
-        if constexpr (SRC) {
-            ut[v] = fma(dt, sk[v], ut[v]);
-            Ssrc[v] = 0.5 * sk[v];
+    for (int v = 0; v < 4; ++v) { ut[v] *= sc; ust[v] *= sc; }
+    if constexpr (SRC && CURV) {
+        double s[4], sd[4];
+        src_eval(*sp, 0.0, s);
+        src_t5(*sp, 0.0, dt, sd);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            ut[v] = fma(dt, s[v], ut[v]);
+            ust[v] = fma(dt, s[v], ust[v]);
+            Ssrc[v] = fma(1.0 / 3.0, sd[v], s[v]);
         }
-    }
-    if constexpr (SRC) {
-        src_t5(*sp, 0.0, dt, sk);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) Ssrc[v] = fma(0.125, sk[v], Ssrc[v]);
-    }
-    double dx[4], dy[4];
-    mdrk_ft(uN, ut, gm1, dx, dy);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        F[v] = fma(0.125, dx[v], 0.5 * f[v]);
-        G[v] = fma(0.125, dy[v], 0.5 * g[v]);
-        Uc[v] = fma(0.125, ut[v], 0.5 * uN[v]);
-    }
-    if (act) put8<S>(s2, sidx, F, G);
-    __syncthreads();
-    contract<n, S>(s2, sbase, i, j, sDh, vol);
-}
-
-// mdrk_kernel_2!, tree/multi_derivative_2d.jl:423-555: F̃ = F2 + f_t(us)/3,
-// Ũ = U2 + ust/3 with F2, U2 recomputed from uⁿ.  With SRC (487-522): the
-// recomputed stage-1 ut gets dt s(t) and S2 = s + s_t/6; ust gets
-// dt s(t + dt/2), and Ssrc = S2 + s_t(t + dt/2)/3.
-template <int N, int EB, bool SRC = false>
-__device__ __forceinline__ void mdrk2_element(const double* uN, const double* usn, double dt, double invJ, double gm1,
-                                              const DevConst* c, int i, int j, bool act, int sidx, int sbase,
-                                              double* s0, double* s1, double* s2, const double* sDm,
-                                              const double* sDh, double* Uc, double* F, double* G, double* vol,
-                                              const SrcPt* sp = nullptr, double* Ssrc = nullptr) {
-    using G_ = VGeo<N, EB>;
-    constexpr int n = G_::n, S = G_::S;
-    double f[4], g[4], fs[4], gs[4];
-    euler_fluxes(uN, gm1, f, g);
-    euler_fluxes(usn, gm1, fs, gs);
-    if (act) {
-        put8<S>(s0, sidx, f, g);
-        put8<S>(s1, sidx, fs, gs);
-    }
-    __syncthreads();
-    double ut[4], ust[4];
-    contract<n, S>(s0, sbase, i, j, sDm, ut);
-    contract<n, S>(s1, sbase, i, j, sDm, ust);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) { ut[v] *= invJ; ust[v] *= invJ; }
-    if constexpr (SRC) {
+    } else if constexpr (SRC) {
         double sk[4], sh[4];
         src_eval(*sp, 0.0, sk);
         src_eval(*sp, 0.5 * dt, sh);
@@ -1465,24 +1326,15 @@ __device__ __forceinline__ void mdrk2_element(const double* uN, const double* us
 #pragma unroll
         for (int v = 0; v < 4; ++v) Ssrc[v] = fma(1.0 / 3.0, sh[v], fma(1.0 / 6.0, sk[v], Ssrc[v]));
     }
-    double dx[4], dy[4];
-    mdrk_ft(uN, ut, gm1, dx, dy);
+    mdrk_ft(uN, ut, gamma, kh, 1.0 / 6.0, q);    // F2
+    mdrk_ft(usn, ust, gamma, kh, 1.0 / 3.0, q);
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        F[v] = fma(1.0 / 6.0, dx[v], f[v]);   // F2
-        G[v] = fma(1.0 / 6.0, dy[v], g[v]);
-        Uc[v] = fma(1.0 / 6.0, ut[v], uN[v]);  // U2
-    }
-    mdrk_ft(usn, ust, gm1, dx, dy);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        F[v] = fma(1.0 / 3.0, dx[v], F[v]);
-        G[v] = fma(1.0 / 3.0, dy[v], G[v]);
-        Uc[v] = fma(1.0 / 3.0, ust[v], Uc[v]);
-    }
-    if (act) put8<S>(s2, sidx, F, G);
+    for (int v = 0; v < 4; ++v) Uc[v] = fma(1.0 / 3.0, ust[v], fma(1.0 / 6.0, ut[v], uN[v]));
+    euler_join(q, Uc[1], Uc[2], Uc[3], gm1, kh, F, G);
     __syncthreads();
-    contract<n, S>(s2, sbase, i, j, sDh, vol);
+    put_fluxes<S, CURV>(A, sidx, act, J, F, G);
+    __syncthreads();
+    contract<n, S>(A, sbase, i, j, sDh, vol);
 }
 
 // ---------------------------------------------------------------------------
@@ -1531,7 +1383,7 @@ __device__ __forceinline__ void contract_xy(const double* s, int base, int i, in
 // state and conservative gradients (convert_derivative_to_primitive,
 // compressible_navier_stokes_2d.jl:37-57; Trixi flux(u, ∇u, orientation)).
 __device__ __forceinline__ void ns_visc_fluxes(const double* u, const double* gx, const double* gy, double gm1,
-                                               const DevConst* c, double* fx, double* fy) {
+                                               DevC c, double* fx, double* fy) {
     const double ir = rcp_nr(u[0]);
     const double v1 = u[1] * ir, v2 = u[2] * ir;
     const double p = gm1 * (u[3] - 0.5 * (u[1] * v1 + u[2] * v2));
@@ -1563,7 +1415,7 @@ __device__ __forceinline__ void ns_visc_fluxes(const double* u, const double* gx
 
 // f = f_a(u) - f_v(u, ∇u)
 __device__ __forceinline__ void ns_total_fluxes(const double* u, const double* gx, const double* gy, double gm1,
-                                                const DevConst* c, double* f, double* g) {
+                                                DevC c, double* f, double* g) {
     double fx[4], fy[4];
     euler_fluxes(u, gm1, f, g);
     ns_visc_fluxes(u, gx, gy, gm1, c, fx, fy);
@@ -1576,26 +1428,15 @@ __device__ __forceinline__ void ns_total_fluxes(const double* u, const double* g
 
 // Viscous time-step bound of one node, J⁻² max(4μ/(3ρ), μκ/(ρ Pr))
 // (compressible_navier_stokes_2d.jl:230-237), with IEEE divisions.
-__device__ __forceinline__ double lam_visc(const double* u, double invJ, const DevConst* c) {
+__device__ __forceinline__ double lam_visc(const double* u, double invJ, DevC c) {
     const double mu = c->visc_mu, rho = u[0];
     return invJ * invJ * dmax(4.0 * mu / (3.0 * rho), mu * c->visc_kappa / (rho * c->visc_Pr));
 }
 // The same with the node's J⁻¹ of a curvilinear mesh in place of J⁻² (the 2-D
 // Jacobian already scales as h²)
-__device__ __forceinline__ double lam_visc_curved(const double* u, double invJ, const DevConst* c) {
+__device__ __forceinline__ double lam_visc_curved(const double* u, double invJ, DevC c) {
     const double mu = c->visc_mu, rho = u[0];
     return invJ * dmax(4.0 * mu / (3.0 * rho), mu * c->visc_kappa / (rho * c->visc_Pr));
-}
-
-// Contravariant fluxes of a Cartesian pair: Ja¹·(f, g), Ja²·(f, g)
-// (contravariant_flux, structured/dg_2d.jl:550-556).
-__device__ __forceinline__ void to_contravariant(const double* J, const double* f, const double* g, double* fc,
-                                                 double* gc) {
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        fc[v] = fma(J[0], f[v], J[1] * g[v]);
-        gc[v] = fma(J[2], f[v], J[3] * g[v]);
-    }
 }
 
 // Reference-space gradient (w_ξ, w_η) → Cartesian with the transposed
@@ -1613,8 +1454,8 @@ __device__ __forceinline__ void grad_to_cartesian(const double* J, double invJ, 
 // BR1 gradient of the node's state: s holds the element's state (put4 before
 // the barrier), src the state array the face neighbours are read from.
 template <int N, int EB, bool CURV = false>
-__device__ __forceinline__ void br1_gradient(const double* s, const double* src, const int* nbr, const DevConst* c,
-                                             int e, int i, int j, int sbase, double invJ, const double* sDh,
+__device__ __forceinline__ void br1_gradient(const double* s, const double* src, int nbx, int nby, DevC c,
+                                             int i, int j, int sbase, double invJ, const double* sDh,
                                              const double* uown, double* gx, double* gy, const double* Jn = nullptr) {
     using G_ = VGeo<N, EB>;
     constexpr int n = G_::n, NN = G_::NN, S = G_::S;
@@ -1637,7 +1478,7 @@ __device__ __forceinline__ void br1_gradient(const double* s, const double* src,
     };
     if (i == 0 || i == n - 1) {
         const int f = (i == 0) ? 0 : 1;
-        const int nb = nbr[4 * e + f];
+        const int nb = nbx;
         const double wf = f ? c->bnd_hi : -c->bnd_lo;
         if (nb >= 0) {
             double un[4];
@@ -1653,7 +1494,7 @@ __device__ __forceinline__ void br1_gradient(const double* s, const double* src,
     }
     if (j == 0 || j == n - 1) {
         const int f = (j == 0) ? 2 : 3;
-        const int nb = nbr[4 * e + f];
+        const int nb = nby;
         const double wf = (f & 1) ? c->bnd_hi : -c->bnd_lo;
         if (nb >= 0) {
             double un[4];
@@ -1708,12 +1549,12 @@ struct ParStates {
                 y[q][v] = fma(cq[q], wy[v], y[q][v]);
             }
     }
-    __device__ __forceinline__ void flux(int q, double gm1, const DevConst* c, double* f, double* g) const {
+    __device__ __forceinline__ void flux(int q, double gm1, DevC c, double* f, double* g) const {
         ns_total_fluxes(u[q], x[q], y[q], gm1, c, f, g);
     }
     // momentum components of the viscous fluxes of state q: (fv1, fv2, gv1, gv2)
     // components 1..3 of the viscous fluxes of state q: (fx1, fx2, fx3, fy1, fy2, fy3)
-    __device__ __forceinline__ void visc6(int q, double gm1, const DevConst* c, double* out) const {
+    __device__ __forceinline__ void visc6(int q, double gm1, DevC c, double* out) const {
         double fx[4], fy[4];
         ns_visc_fluxes(u[q], x[q], y[q], gm1, c, fx, fy);
         out[0] = fx[1];
@@ -1726,11 +1567,11 @@ struct ParStates {
 };
 
 // Time derivative of the next level and its element-local gradient:
-// w = J⁻¹ (-dt D) · (dx, dy) (+ add, the level's source term dt·s) through sa,
+// w = sc D · (dx, dy), sc = -dt J⁻¹, (+ add, the level's source term dt·s) through sa,
 // then (wx, wy) = J⁻¹ D w through sg.
 template <int N, int EB, bool CURV = false>
-__device__ __forceinline__ void par_level(bool act, int sidx, int sbase, int i, int j, double invJ, double* sa,
-                                          double* sg, const double* sDm, const double* sD, const double* dx,
+__device__ __forceinline__ void par_level(bool act, int sidx, int sbase, int i, int j, double invJ, double sc,
+                                          double* sa, double* sg, const double* sD, const double* dx,
                                           const double* dy, double* w, double* wx, double* wy,
                                           const double* Jn = nullptr, const double* add = nullptr) {
     using G_ = VGeo<N, EB>;
@@ -1744,9 +1585,9 @@ __device__ __forceinline__ void par_level(bool act, int sidx, int sbase, int i, 
         if (act) put8<S>(sa, sidx, dx, dy);
     }
     __syncthreads();
-    contract<n, S>(sa, sbase, i, j, sDm, w);
+    contract<n, S>(sa, sbase, i, j, sD, w);
 #pragma unroll
-    for (int v = 0; v < 4; ++v) w[v] *= invJ;
+    for (int v = 0; v < 4; ++v) w[v] *= sc;
     if (add) {
 #pragma unroll
         for (int v = 0; v < 4; ++v) w[v] += add[v];
@@ -1766,15 +1607,15 @@ __device__ __forceinline__ void par_level(bool act, int sidx, int sbase, int i, 
 }
 
 // lw_volume_kernel_3!/4! with viscous terms (dg_2d_parabolic.jl:725-1189,
-// 1191-1860): the Euler procedure of lw3_element/lw4_element on the total
+// 1191-1860): the Euler procedure of lw3_element/lw_element on the total
 // flux, with the states of ∇u advanced by the same Taylor coefficients.
 // Buffer use: s0 keeps f(uⁿ) for the 5- and 3-point stencils, s1 takes each
 // flux derivative, s2 each time derivative; the final F̃ exchange is in s2.
 template <int N, int EB, bool CURV = false, bool WALL = false>
 __device__ __forceinline__ void lwp_element(const double* uN, const double* gxN, const double* gyN, double invJ,
-                                            double gm1, const DevConst* c, int i, int j, bool act, int sidx,
-                                            int sbase, double* s0, double* s1, double* s2, const double* sDm,
-                                            const double* sD, const double* sDh, double* Uc, double* F, double* G,
+                                            double sc, double gm1, DevC c, int i, int j, bool act, int sidx,
+                                            int sbase, double* s0, double* s1, double* s2, const double* sD,
+                                            const double* sDh, double* Uc, double* F, double* G,
                                             double* vol, const double* Jn = nullptr, double* const* wq = nullptr,
                                             double* terr = nullptr, double abstol = 0.0, double reltol = 0.0,
                                             bool has_src = false, const NsSrcPt& sp = NsSrcPt{},
@@ -1856,9 +1697,9 @@ __device__ __forceinline__ void lwp_element(const double* uN, const double* gxN,
     if constexpr (WALL) {
         double ds[4];
         src_lvl(0, 1.0, ds);
-        par_level<N, EB, CURV>(act, sidx, sbase, i, j, invJ, s0, s2, sDm, sD, F, G, w, wx, wy, Jn, ds);  // ut
+        par_level<N, EB, CURV>(act, sidx, sbase, i, j, invJ, sc, s0, s2, sD, F, G, w, wx, wy, Jn, ds);  // ut
     } else {
-        par_level<N, EB, CURV>(act, sidx, sbase, i, j, invJ, s0, s2, sDm, sD, F, G, w, wx, wy, Jn);  // ut
+        par_level<N, EB, CURV>(act, sidx, sbase, i, j, invJ, sc, s0, s2, sD, F, G, w, wx, wy, Jn);  // ut
     }
     // on a curvilinear mesh s0 took the contravariant pair; the centred stencils
     // read the node's own Cartesian f(uⁿ), written once every lane has passed
@@ -1895,9 +1736,9 @@ __device__ __forceinline__ void lwp_element(const double* uN, const double* gxN,
     if constexpr (WALL) {
         double ds[4];
         src_lvl(1, 0.5, ds);
-        par_level<N, EB, CURV>(act, sidx, sbase, i, j, invJ, s1, s2, sDm, sD, dx, dy, w, wx, wy, Jn, ds);  // utt
+        par_level<N, EB, CURV>(act, sidx, sbase, i, j, invJ, sc, s1, s2, sD, dx, dy, w, wx, wy, Jn, ds);  // utt
     } else {
-        par_level<N, EB, CURV>(act, sidx, sbase, i, j, invJ, s1, s2, sDm, sD, dx, dy, w, wx, wy, Jn);  // utt
+        par_level<N, EB, CURV>(act, sidx, sbase, i, j, invJ, sc, s1, s2, sD, dx, dy, w, wx, wy, Jn);  // utt
     }
     P.add(0.5, 0.5, 2.0, 2.0, w, wx, wy);
 #pragma unroll
@@ -1953,9 +1794,9 @@ __device__ __forceinline__ void lwp_element(const double* uN, const double* gxN,
     if constexpr (WALL) {
         double ds[4];
         src_lvl(2, 1.0 / 6.0, ds);
-        par_level<N, EB, CURV>(act, sidx, sbase, i, j, invJ, s1, s2, sDm, sD, dx, dy, w, wx, wy, Jn, ds);  // uttt
+        par_level<N, EB, CURV>(act, sidx, sbase, i, j, invJ, sc, s1, s2, sD, dx, dy, w, wx, wy, Jn, ds);  // uttt
     } else {
-        par_level<N, EB, CURV>(act, sidx, sbase, i, j, invJ, s1, s2, sDm, sD, dx, dy, w, wx, wy, Jn);  // uttt
+        par_level<N, EB, CURV>(act, sidx, sbase, i, j, invJ, sc, s1, s2, sD, dx, dy, w, wx, wy, Jn);  // uttt
     }
     P.add(1.0 / 6.0, -1.0 / 6.0, 4.0 / 3.0, -4.0 / 3.0, w, wx, wy);
 #pragma unroll
@@ -1984,9 +1825,9 @@ __device__ __forceinline__ void lwp_element(const double* uN, const double* gxN,
         if constexpr (WALL) {
             double ds[4];
             src_lvl(3, 1.0 / 24.0, ds);
-            par_level<N, EB, CURV>(act, sidx, sbase, i, j, invJ, s1, s2, sDm, sD, dx, dy, w, wx, wy, Jn, ds);
+            par_level<N, EB, CURV>(act, sidx, sbase, i, j, invJ, sc, s1, s2, sD, dx, dy, w, wx, wy, Jn, ds);
         } else {
-            par_level<N, EB, CURV>(act, sidx, sbase, i, j, invJ, s1, s2, sDm, sD, dx, dy, w, wx, wy, Jn);  // utttt
+            par_level<N, EB, CURV>(act, sidx, sbase, i, j, invJ, sc, s1, s2, sD, dx, dy, w, wx, wy, Jn);  // utttt
         }
         P.add(1.0 / 24.0, 1.0 / 24.0, 2.0 / 3.0, 2.0 / 3.0, w, wx, wy);
 #pragma unroll
@@ -2039,15 +1880,15 @@ __device__ __forceinline__ void lwp_element(const double* uN, const double* gxN,
     contract<n, S>(s2, sbase, i, j, sDh, vol);
     if (terr) {
         // temporal error of kernel 4 (dg_2d_parabolic.jl:1749-1775, 1841-1855): as in
-        // lw4_element, with the total F̃ and f_tttt
+        // lw_element, with the total F̃ and f_tttt
         double a1[4], a2[4];
-        contract<n, S>(s2, sbase, i, j, sDm, a1);  // -dt D F̃
-        contract<n, S>(s0, sbase, i, j, sDm, a2);  // -dt D f_tttt
+        contract<n, S>(s2, sbase, i, j, sD, a1);  // D F̃
+        contract<n, S>(s0, sbase, i, j, sD, a2);  // D f_tttt
         double e = 0.0;
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            const double d = invJ * ((1.0 / 120.0) * a2[v]);
-            const double hi = fma(invJ, a1[v], uN[v]);
+            const double d = sc * ((1.0 / 120.0) * a2[v]);
+            const double hi = fma(sc, a1[v], uN[v]);
             const double lo = hi - d;
             const double r = d / (abstol + reltol * dmax(fabs(hi), fabs(lo)));
             e = fma(r, r, e);
@@ -2062,7 +1903,7 @@ __device__ __forceinline__ void lwp_element(const double* uN, const double* gxN,
 // from the same evaluations
 template <bool WALL = false>
 __device__ __forceinline__ void mdrkp_ft(const double* u, const double* ut, const double* gx, const double* gtx,
-                                         const double* gy, const double* gty, double gm1, const DevConst* c,
+                                         const double* gy, const double* gty, double gm1, DevC c,
                                          double* dx, double* dy, double* v6 = nullptr) {
     const double cq[4] = {2.0, 1.0, -1.0, -2.0};
     const double wq[4] = {-1.0, 8.0, -8.0, 1.0};
@@ -2128,7 +1969,7 @@ __device__ __forceinline__ void wall_acc(double* const* wq, double w, const doub
 // components 1..3 of the viscous fluxes of a wall face node's state into its
 // wall records with weight w (the first term of the average)
 __device__ __forceinline__ void wall_first(double* const* wq, double w, const double* u, const double* gx,
-                                           const double* gy, double gm1, const DevConst* c) {
+                                           const double* gy, double gm1, DevC c) {
     if (!wq[0] && !wq[1]) return;
     double fx[4], fy[4], v6[6];
     ns_visc_fluxes(u, gx, gy, gm1, c, fx, fy);
@@ -2148,9 +1989,9 @@ __device__ __forceinline__ void wall_first(double* const* wq, double w, const do
 // its gradient, and Ssrc = s/2 + s_t/8 for the residual.
 template <int N, int EB, bool CURV = false, bool WALL = false>
 __device__ __forceinline__ void mdrkp1_element(const double* uN, const double* gxN, const double* gyN, double invJ,
-                                               double gm1, const DevConst* c, int i, int j, bool act, int sidx,
-                                               int sbase, double* s0, double* s1, double* s2, const double* sDm,
-                                               const double* sD, const double* sDh, double* Uc, double* F,
+                                               double sc, double gm1, DevC c, int i, int j, bool act, int sidx,
+                                               int sbase, double* s0, double* s1, double* s2, const double* sD,
+                                               const double* sDh, double* Uc, double* F,
                                                double* G, double* vol, const double* Jn = nullptr,
                                                double* const* wq = nullptr, bool has_src = false,
                                                const NsSrcPt& sp = NsSrcPt{}, double dt = 0.0,
@@ -2170,9 +2011,9 @@ __device__ __forceinline__ void mdrkp1_element(const double* uN, const double* g
             ds[v] = dt * s[v];
             Ssrc[v] = fma(0.125, st[v], 0.5 * s[v]);
         }
-        par_level<N, EB, CURV>(act, sidx, sbase, i, j, invJ, s0, s2, sDm, sD, f, g, ut, utx, uty, Jn, ds);
+        par_level<N, EB, CURV>(act, sidx, sbase, i, j, invJ, sc, s0, s2, sD, f, g, ut, utx, uty, Jn, ds);
     } else {
-        par_level<N, EB, CURV>(act, sidx, sbase, i, j, invJ, s0, s2, sDm, sD, f, g, ut, utx, uty, Jn);
+        par_level<N, EB, CURV>(act, sidx, sbase, i, j, invJ, sc, s0, s2, sD, f, g, ut, utx, uty, Jn);
     }
     double dx[4], dy[4];
     if constexpr (WALL) {
@@ -2210,9 +2051,9 @@ __device__ __forceinline__ void mdrkp1_element(const double* uN, const double* g
 template <int N, int EB, bool CURV = false, bool WALL = false>
 __device__ __forceinline__ void mdrkp2_element(const double* uN, const double* gxN, const double* gyN,
                                                const double* usn, const double* gxS, const double* gyS,
-                                               double invJ, double gm1, const DevConst* c, int i, int j, bool act,
+                                               double invJ, double sc, double gm1, DevC c, int i, int j, bool act,
                                                int sidx, int sbase, double* s0, double* s1, double* s2,
-                                               const double* sDm, const double* sD, const double* sDh, double* Uc,
+                                               const double* sD, const double* sDh, double* Uc,
                                                double* F, double* G, double* vol, const double* Jn = nullptr,
                                                double* const* wq = nullptr, bool has_src = false,
                                                const NsSrcPt& sp = NsSrcPt{}, double dt = 0.0,
@@ -2235,12 +2076,12 @@ __device__ __forceinline__ void mdrkp2_element(const double* uN, const double* g
     }
     __syncthreads();
     double ut[4], ust[4];
-    contract<n, S>(s0, sbase, i, j, sDm, ut);
-    contract<n, S>(s1, sbase, i, j, sDm, ust);
+    contract<n, S>(s0, sbase, i, j, sD, ut);
+    contract<n, S>(s1, sbase, i, j, sD, ust);
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-        ut[v] *= invJ;
-        ust[v] *= invJ;
+        ut[v] *= sc;
+        ust[v] *= sc;
     }
     if (has_src) {
         double s[4], st[4];
@@ -2312,337 +2153,6 @@ __device__ __forceinline__ void mdrkp2_element(const double* uN, const double* g
     contract<n, S>(s2, sbase, i, j, sDh, vol);
 }
 
-// ---------------------------------------------------------------------------
-// Curvilinear StructuredMesh (lw_volume_kernel_3!/4! for StructuredMesh,
-// src/solvers/dgsem_structured/dg_2d.jl:1379-2105): the LW procedure with the
-// node's contravariant vectors J = (Ja11, Ja12, Ja21, Ja22) and inverse
-// Jacobian.  The flux time derivatives are formed for the Cartesian fluxes
-// (their time averages F̃, G̃ feed the face records, F̃·n) and turned into
-// contravariant ones, Ja¹·(f, g) and Ja²·(f, g), for the derivative
-// contractions; the volume term is D̂ of the contravariant time average.
-// f(uⁿ) is kept in registers (f0x, f0y) for the centred stencils.
-
-// SRC: with the source terms of the StructuredMesh kernels (src_level_c; sp the
-// node's point, Ssrc the S of the residual, dtv the step).
-template <int N, int EB, bool SRC = false>
-__device__ __forceinline__ void lwc_element(const double* uN, const double* J, double invJ, double gm1, int i, int j,
-                                            bool act, int sidx, int sbase, double* s0, double* s1, double* s2,
-                                            const double* sDm, const double* sDh, double* Uc, double* F, double* G,
-                                            double* vol, double* terr = nullptr, double abstol = 0.0,
-                                            double reltol = 0.0, const SrcPt* sp = nullptr, double* Ssrc = nullptr,
-                                            double dtv = 0.0) {
-    using G_ = VGeo<N, EB>;
-    constexpr int n = G_::n, S = G_::S;
-    double f0x[4], f0y[4], cx[4], cy[4];
-    euler_fluxes(uN, gm1, f0x, f0y);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) { F[v] = f0x[v]; G[v] = f0y[v]; }
-    to_contravariant(J, f0x, f0y, cx, cy);
-    if (act) put8<S>(s0, sidx, cx, cy);
-    __syncthreads();
-    double w[4];
-    contract<n, S>(s0, sbase, i, j, sDm, w);
-    double up[4], um[4], upp[4], umm[4];
-    double sk[4] = {0.0, 0.0, 0.0, 0.0};
-    if constexpr (SRC) src_level_c(*sp, dtv, 0, N == 4, sk, Ssrc, 1.0);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        w[v] *= invJ;  // ut
-        if constexpr (SRC) w[v] = fma(dtv, sk[v], w[v]);
-        Uc[v] = fma(0.5, w[v], uN[v]);
-        up[v] = uN[v] + w[v];
-        um[v] = uN[v] - w[v];
-        upp[v] = fma(2.0, w[v], uN[v]);
-        umm[v] = fma(-2.0, w[v], uN[v]);
-    }
-    double fa[4], ga[4], dx[4], dy[4];
-    // stage 1: f_t = (-f(u++) + 8 f(u+) - 8 f(u-) + f(u--)) / 12
-    euler_fluxes(upp, gm1, fa, ga);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) { dx[v] = -fa[v]; dy[v] = -ga[v]; }
-    euler_fluxes(up, gm1, fa, ga);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) { dx[v] = fma(8.0, fa[v], dx[v]); dy[v] = fma(8.0, ga[v], dy[v]); }
-    euler_fluxes(um, gm1, fa, ga);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) { dx[v] = fma(-8.0, fa[v], dx[v]); dy[v] = fma(-8.0, ga[v], dy[v]); }
-    euler_fluxes(umm, gm1, fa, ga);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        dx[v] = (1.0 / 12.0) * (dx[v] + fa[v]);
-        dy[v] = (1.0 / 12.0) * (dy[v] + ga[v]);
-        F[v] = fma(0.5, dx[v], F[v]);
-        G[v] = fma(0.5, dy[v], G[v]);
-    }
-    to_contravariant(J, dx, dy, cx, cy);
-    if (act) put8<S>(s1, sidx, cx, cy);
-    __syncthreads();
-    contract<n, S>(s1, sbase, i, j, sDm, w);
-    if constexpr (SRC) src_level_c(*sp, dtv, 1, N == 4, sk, Ssrc, 0.5);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        w[v] *= invJ;  // utt
-        if constexpr (SRC) w[v] = fma(dtv, sk[v], w[v]);
-        Uc[v] = fma(1.0 / 6.0, w[v], Uc[v]);
-        up[v] = fma(0.5, w[v], up[v]);
-        um[v] = fma(0.5, w[v], um[v]);
-        upp[v] = fma(2.0, w[v], upp[v]);
-        umm[v] = fma(2.0, w[v], umm[v]);
-    }
-    if constexpr (N == 4) {
-        // stage 2: f_tt = (-f(u++) + 16 f(u+) - 30 f + 16 f(u-) - f(u--)) / 12
-        euler_fluxes(upp, gm1, fa, ga);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) { dx[v] = -fa[v]; dy[v] = -ga[v]; }
-        euler_fluxes(up, gm1, fa, ga);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            dx[v] = fma(16.0, fa[v], dx[v]);
-            dy[v] = fma(16.0, ga[v], dy[v]);
-            dx[v] = fma(-30.0, f0x[v], dx[v]);
-            dy[v] = fma(-30.0, f0y[v], dy[v]);
-        }
-        euler_fluxes(um, gm1, fa, ga);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) { dx[v] = fma(16.0, fa[v], dx[v]); dy[v] = fma(16.0, ga[v], dy[v]); }
-        euler_fluxes(umm, gm1, fa, ga);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            dx[v] = (1.0 / 12.0) * (dx[v] - fa[v]);
-            dy[v] = (1.0 / 12.0) * (dy[v] - ga[v]);
-        }
-    } else {
-        // stage 2: f_tt = f(u+) - 2 f + f(u-)
-        euler_fluxes(up, gm1, fa, ga);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            dx[v] = fma(-2.0, f0x[v], fa[v]);
-            dy[v] = fma(-2.0, f0y[v], ga[v]);
-        }
-        euler_fluxes(um, gm1, fa, ga);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) { dx[v] += fa[v]; dy[v] += ga[v]; }
-    }
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        F[v] = fma(1.0 / 6.0, dx[v], F[v]);
-        G[v] = fma(1.0 / 6.0, dy[v], G[v]);
-    }
-    to_contravariant(J, dx, dy, cx, cy);
-    if (act) put8<S>(s2, sidx, cx, cy);
-    __syncthreads();
-    contract<n, S>(s2, sbase, i, j, sDm, w);
-    if constexpr (SRC) src_level_c(*sp, dtv, 2, N == 4, sk, Ssrc, 1.0 / 6.0);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        w[v] *= invJ;  // uttt
-        if constexpr (SRC) w[v] = fma(dtv, sk[v], w[v]);
-        Uc[v] = fma(1.0 / 24.0, w[v], Uc[v]);
-        um[v] = fma(-1.0 / 6.0, w[v], um[v]);
-        up[v] = fma(1.0 / 6.0, w[v], up[v]);
-        umm[v] = fma(-4.0 / 3.0, w[v], umm[v]);
-        upp[v] = fma(4.0 / 3.0, w[v], upp[v]);
-    }
-    // stage 3: f_ttt = (f(u++) - 2 f(u+) + 2 f(u-) - f(u--)) / 2
-    euler_fluxes(upp, gm1, fa, ga);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) { dx[v] = fa[v]; dy[v] = ga[v]; }
-    euler_fluxes(up, gm1, fa, ga);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) { dx[v] = fma(-2.0, fa[v], dx[v]); dy[v] = fma(-2.0, ga[v], dy[v]); }
-    euler_fluxes(um, gm1, fa, ga);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) { dx[v] = fma(2.0, fa[v], dx[v]); dy[v] = fma(2.0, ga[v], dy[v]); }
-    euler_fluxes(umm, gm1, fa, ga);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        dx[v] = 0.5 * (dx[v] - fa[v]);
-        dy[v] = 0.5 * (dy[v] - ga[v]);
-        F[v] = fma(1.0 / 24.0, dx[v], F[v]);
-        G[v] = fma(1.0 / 24.0, dy[v], G[v]);
-    }
-    if constexpr (N == 4) {
-        to_contravariant(J, dx, dy, cx, cy);
-        if (act) put8<S>(s1, sidx, cx, cy);
-        __syncthreads();
-        contract<n, S>(s1, sbase, i, j, sDm, w);
-        if constexpr (SRC) src_level_c(*sp, dtv, 3, true, sk, Ssrc, 1.0 / 24.0);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            w[v] *= invJ;  // utttt
-            if constexpr (SRC) w[v] = fma(dtv, sk[v], w[v]);
-            Uc[v] = fma(1.0 / 120.0, w[v], Uc[v]);
-            um[v] = fma(1.0 / 24.0, w[v], um[v]);
-            up[v] = fma(1.0 / 24.0, w[v], up[v]);
-            umm[v] = fma(2.0 / 3.0, w[v], umm[v]);
-            upp[v] = fma(2.0 / 3.0, w[v], upp[v]);
-        }
-        // stage 4: f_tttt = 0.5 (f(u++) - 4 f(u+) + 6 f - 4 f(u-) + f(u--)), with the
-        // reference's factor 0.5 (dg_2d.jl:2018-2021)
-        euler_fluxes(upp, gm1, fa, ga);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) { dx[v] = fa[v]; dy[v] = ga[v]; }
-        euler_fluxes(up, gm1, fa, ga);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            dx[v] = fma(-4.0, fa[v], dx[v]);
-            dy[v] = fma(-4.0, ga[v], dy[v]);
-            dx[v] = fma(6.0, f0x[v], dx[v]);
-            dy[v] = fma(6.0, f0y[v], dy[v]);
-        }
-        euler_fluxes(um, gm1, fa, ga);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) { dx[v] = fma(-4.0, fa[v], dx[v]); dy[v] = fma(-4.0, ga[v], dy[v]); }
-        euler_fluxes(umm, gm1, fa, ga);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            dx[v] = 0.5 * (dx[v] + fa[v]);
-            dy[v] = 0.5 * (dy[v] + ga[v]);
-            F[v] = fma(1.0 / 120.0, dx[v], F[v]);
-            G[v] = fma(1.0 / 120.0, dy[v], G[v]);
-        }
-    }
-    // the source's last difference enters S only: s_tttt/120 (kernel 4), s_ttt/24 (kernel 3)
-    if constexpr (SRC) src_level_c(*sp, dtv, N == 4 ? 4 : 3, N == 4, sk, Ssrc, N == 4 ? 1.0 / 120.0 : 1.0 / 24.0);
-    to_contravariant(J, F, G, cx, cy);
-    // polydeg 3 read s2 in its last contraction: every thread has finished
-    // before it is reused (polydeg 4 passed a barrier since)
-    if constexpr (N == 3) __syncthreads();
-    if (act) put8<S>(s2, sidx, cx, cy);
-    // the last stage's contravariant term for the temporal error; s0 is read
-    // only by the first contraction
-    if (terr) {
-        double tx[4], ty[4];
-        to_contravariant(J, dx, dy, tx, ty);
-        if (act) put8<S>(s0, sidx, tx, ty);
-    }
-    __syncthreads();
-    contract<n, S>(s2, sbase, i, j, sDh, vol);
-    if (terr) {
-        // temporal error of the node (structured dg_2d.jl:1595-1681 at N=3, 1983-2077 at N=4):
-        // u_np1 = u + J⁻¹(-dt D)·F̃c, u_np1_low without the last stage's term, whose update
-        // itself is the numerator
-        constexpr double wlast = (N == 4) ? 1.0 / 120.0 : 1.0 / 24.0;
-        double a1[4], a2[4];
-        contract<n, S>(s2, sbase, i, j, sDm, a1);
-        contract<n, S>(s0, sbase, i, j, sDm, a2);
-        double e = 0.0;
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const double d = invJ * (wlast * a2[v]);
-            const double hi = fma(invJ, a1[v], uN[v]);
-            const double lo = hi - d;
-            const double r = d / (abstol + reltol * dmax(fabs(hi), fabs(lo)));
-            e = fma(r, r, e);
-        }
-        *terr = e;
-        __syncthreads();  // s0 is reused for the face records
-    }
-}
-
-// mdrk_kernel_1! for StructuredMesh (structured/multi_derivative_2d.jl:82-243):
-// F̃ = f/2 + f_t/8 (Cartesian, for the records), its contravariant image for
-// the D̂ contraction, Ũ = u/2 + ut/8, ut from the contravariant fluxes.  SRC
-// (146-155, 179-200): ut += dt s, Ssrc = s/2 + s_t/8.
-template <int N, int EB, bool SRC = false>
-__device__ __forceinline__ void mdrkc1_element(const double* uN, const double* J, double invJ, double gm1, int i,
-                                               int j, bool act, int sidx, int sbase, double* s0, double* s2,
-                                               const double* sDm, const double* sDh, double* Uc, double* F,
-                                               double* G, double* vol, const SrcPt* sp = nullptr,
-                                               double* Ssrc = nullptr, double dtv = 0.0) {
-    using G_ = VGeo<N, EB>;
-    constexpr int n = G_::n, S = G_::S;
-    double f[4], g[4], cx[4], cy[4];
-    euler_fluxes(uN, gm1, f, g);
-    to_contravariant(J, f, g, cx, cy);
-    if (act) put8<S>(s0, sidx, cx, cy);
-    __syncthreads();
-    double ut[4];
-    contract<n, S>(s0, sbase, i, j, sDm, ut);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) ut[v] *= invJ;
-    if constexpr (SRC) {
-        double s[4], st[4];
-        src_eval(*sp, 0.0, s);
-        src_t5(*sp, 0.0, dtv, st);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            ut[v] = fma(dtv, s[v], ut[v]);
-            Ssrc[v] = fma(0.125, st[v], 0.5 * s[v]);
-        }
-    }
-    double dx[4], dy[4];
-    mdrk_ft(uN, ut, gm1, dx, dy);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        F[v] = fma(0.125, dx[v], 0.5 * f[v]);
-        G[v] = fma(0.125, dy[v], 0.5 * g[v]);
-        Uc[v] = fma(0.125, ut[v], 0.5 * uN[v]);
-    }
-    to_contravariant(J, F, G, cx, cy);
-    if (act) put8<S>(s2, sidx, cx, cy);
-    __syncthreads();
-    contract<n, S>(s2, sbase, i, j, sDh, vol);
-}
-
-// mdrk_kernel_2! for StructuredMesh (structured/multi_derivative_2d.jl:245-445):
-// F̃ = F2 + f_t(us)/3, Ũ = U2 + ust/3, with F2 = f + f_t/6 and U2 = u + ut/6
-// recomputed from uⁿ instead of being stored by stage 1.  SRC (326-339,
-// 358-385): ut and ust += dt s(t); Ssrc = s + s_t/3 about t, the reference's
-// stage 2 overwriting the S2 it loads (stage 1's s + s_t/6) with s.
-template <int N, int EB, bool SRC = false>
-__device__ __forceinline__ void mdrkc2_element(const double* uN, const double* usn, const double* J, double invJ,
-                                               double gm1, int i, int j, bool act, int sidx, int sbase, double* s0,
-                                               double* s1, double* s2, const double* sDm, const double* sDh,
-                                               double* Uc, double* F, double* G, double* vol,
-                                               const SrcPt* sp = nullptr, double* Ssrc = nullptr, double dtv = 0.0) {
-    using G_ = VGeo<N, EB>;
-    constexpr int n = G_::n, S = G_::S;
-    double f[4], g[4], cx[4], cy[4];
-    euler_fluxes(uN, gm1, f, g);
-    to_contravariant(J, f, g, cx, cy);
-    if (act) put8<S>(s0, sidx, cx, cy);
-    euler_fluxes(usn, gm1, F, G);
-    to_contravariant(J, F, G, cx, cy);
-    if (act) put8<S>(s1, sidx, cx, cy);
-    __syncthreads();
-    double ut[4], ust[4];
-    contract<n, S>(s0, sbase, i, j, sDm, ut);
-    contract<n, S>(s1, sbase, i, j, sDm, ust);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) { ut[v] *= invJ; ust[v] *= invJ; }
-    if constexpr (SRC) {
-        double s[4], st[4];
-        src_eval(*sp, 0.0, s);
-        src_t5(*sp, 0.0, dtv, st);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            ut[v] = fma(dtv, s[v], ut[v]);
-            ust[v] = fma(dtv, s[v], ust[v]);
-            Ssrc[v] = fma(1.0 / 3.0, st[v], s[v]);
-        }
-    }
-    double dx[4], dy[4];
-    mdrk_ft(uN, ut, gm1, dx, dy);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        F[v] = fma(1.0 / 6.0, dx[v], f[v]);    // F2
-        G[v] = fma(1.0 / 6.0, dy[v], g[v]);
-        Uc[v] = fma(1.0 / 6.0, ut[v], uN[v]);  // U2
-    }
-    mdrk_ft(usn, ust, gm1, dx, dy);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        F[v] = fma(1.0 / 3.0, dx[v], F[v]);
-        G[v] = fma(1.0 / 3.0, dy[v], G[v]);
-        Uc[v] = fma(1.0 / 3.0, ust[v], Uc[v]);
-    }
-    to_contravariant(J, F, G, cx, cy);
-    if (act) put8<S>(s2, sidx, cx, cy);
-    __syncthreads();
-    contract<n, S>(s2, sbase, i, j, sDh, vol);
-}
-
 // Curvilinear CFL speeds of a node (Trixi max_dt for curvilinear meshes): the
 // speeds transformed to the reference element, |Ja^k · (λ1, λ2)| |J⁻¹|.
 __device__ __forceinline__ void curved_speeds(const double* u, const double* J, double invJ, double gamma, double& m1,
@@ -2669,15 +2179,27 @@ __device__ __forceinline__ void curved_speeds(const double* u, const double* J, 
 #define TLW_VOL_WAVES 3
 #endif
 template <bool TWO> constexpr int kVolWaves = TWO ? 2 : TLW_VOL_WAVES;
+template <bool SC, bool PAR> constexpr bool vol_two_buffers = !SC && !PAR;
+
+// What a lane of a volume workgroup reads of its tile before the element procedure.
+template <bool CURV, bool US> struct TileIn {
+    double u[4];               // uⁿ of the lane's node
+    double us[US ? 4 : 1];     // the MDRK stage state
+    double J[CURV ? 4 : 1];    // Ja11, Ja12, Ja21, Ja22 of the node
+    double invJ;               // per element on a TreeMesh, per node on a curvilinear mesh
+    int nbx, nby;              // neighbours across the node's x and y face (where it lies on one)
+    int slot;                  // neighbour across the lane's face slot (element, face, node)
+};
 
 // PAR: hyperbolic-parabolic (compressible Navier-Stokes) element procedures,
 // same register budget as shock capturing.
-// The volume workgroup `bid` of a's table, with its LDS: lds [G_::LDS], sDm,
-// sDh, sD [G_::M] (-dt D, D̂ and D, rows of G_::MS) and s_alpha [EB] (smoothed blending
-// factors of the curvilinear interfaces).
+// One tile (blk) of a's table, number bid, with its LDS: lds [G_::LDS2 or LDS],
+// sDh and sD [G_::M] (D̂ and D, rows of G_::MS) and s_alpha [EB] (smoothed
+// blending factors of the curvilinear interfaces).
 template <int N, int EB, int KIND, bool SC, bool PAR, bool CURV>
-__device__ __forceinline__ void volume_body(const KArgs& a, int bid, double* lds, double* sDm, double* sDh, double* sD,
-                                            double* s_alpha) {
+__device__ __forceinline__ void volume_tile(const KArgs& a, int bid, const int4& blk,
+                                            const TileIn<CURV, vol_base(KIND) == VOL_MDRK2>& in, double* lds,
+                                            double* sDh, double* sD, double* s_alpha) {
     static_assert(!(SC && PAR), "shock capturing has no hyperbolic-parabolic form");
     static_assert(!CURV || !PAR || KIND != VOL_LW_ADAPT, "adaptive steps: Euler LW, or Navier-Stokes LW on a TreeMesh");
     static_assert(!PAR || vol_base(KIND) != VOL_LW_ADAPT || N == 4, "the parabolic temporal error is kernel 4's");
@@ -2685,11 +2207,20 @@ __device__ __forceinline__ void volume_body(const KArgs& a, int bid, double* lds
     static_assert(!(CURV && PAR && SC), "no shock capturing with parabolic terms");
     using G_ = VGeo<N, EB>;
     constexpr int n = G_::n, NN = G_::NN, S = G_::S, NT = G_::NT;
+    // The plain Euler kernels exchange through two buffers: F̃ last in the first of
+    // them, where the interface fluxes go later, and the face records in the
+    // second.  Shock capturing and the Navier-Stokes kernels use three: s2 takes
+    // F̃ and the interface fluxes, s0 and s1 the records.
+    constexpr bool TWO = vol_two_buffers<SC, PAR>;
     double* s0 = lds;
     double* s1 = lds + 8 * S;
-    double* s2 = lds + 16 * S;
-    const int4 blk = load_blk_at(a.vblk, bid);
-    DevState* st = a.st + blk.z;
+    double* s2 = TWO ? lds : lds + 16 * S;
+    constexpr int KB = vol_base(KIND);
+    // (A, B) of the element procedures, whose last exchange goes to s2
+    constexpr bool last_is_a = KB == VOL_MDRK2 || (N == 4 && (KB == VOL_LW || KB == VOL_LW_ADAPT));
+    double* bufA = last_is_a ? s2 : s1;
+    double* bufB = last_is_a ? s1 : s2;
+    const DevS st = dev_state(a.st + blk.z);
     if (a.use_state_dt && st->finished) return;
     const int tid = threadIdx.x;
     const int le = tid / NN, node = tid - (tid / NN) * NN;
@@ -2704,17 +2235,16 @@ __device__ __forceinline__ void volume_body(const KArgs& a, int bid, double* lds
     const double* uin = sel_in(a, cur);
     double* out = sel_out(a, cur);
     const double dt = a.use_state_dt ? st->dt : a.dt_arg;
-    const DevConst* c = a.c;
+    const DevC c = dev_const(a.c);
     const double gamma = c->gamma, gm1 = gamma - 1.0;
-    // inverse Jacobian: per element on a TreeMesh, per node on a curvilinear mesh
-    const double invJ = CURV ? a.ijn[(size_t)e * NN + node] : a.inv_jac[e];
+    const double invJ = in.invJ;
+    const double sc = -dt * invJ;
     const size_t off = ((size_t)e * NN + node) * 4;
     // source terms: separate instantiations (KIND = VOL_LW_SRC + the plain kind);
     // the node's coordinates from the element's centre and edge length, the
     // time of the call; Ssrc = S, added to the residual at the end
     constexpr bool SRC = vol_is_src(KIND);
     constexpr bool WALL = vol_is_wall(KIND);
-    constexpr int KB = vol_base(KIND);
     static_assert(!SRC || (!SC && !PAR), "source terms: the Euler kernels");
     double Ssrc[4] = {0.0, 0.0, 0.0, 0.0};
     SrcPt sp{0.0, 0.0, 0.0, gamma};
@@ -2729,48 +2259,29 @@ __device__ __forceinline__ void volume_body(const KArgs& a, int bid, double* lds
         sp.t = a.use_state_dt ? st->t : a.t_arg;
     }
 
-    if (tid < NN) {  // published by the first barrier of the element computation
-        const int q = (tid / n) * G_::MS + tid % n;
-        sDm[q] = -dt * c->D[tid / n][tid % n];
-        sDh[q] = c->Dhat[tid / n][tid % n];
-        if constexpr (PAR) sD[q] = c->D[tid / n][tid % n];
-    }
-    double uN[4], Uc[4], F[4], G[4], vol[4];
+    double Uc[4], F[4], G[4], vol[4];
     double terr = 0.0;  // temporal error of the node (adaptive steps, LW N=4)
-    load4(uin + off, uN);
-    double Jn[4] = {0.0, 0.0, 0.0, 0.0};  // Ja11, Ja12, Ja21, Ja22 of the node: same layout as the state
+    const double* uN = in.u;
+    const double* Jn = in.J;
     // walls: the node's wall records (its x face, its y face; null where that face is no wall)
     double* wq[2] = {nullptr, nullptr};
     if constexpr (WALL) {
         const int wfx = (i == 0) ? 0 : ((i == n - 1) ? 1 : -1), wfy = (j == 0) ? 2 : ((j == n - 1) ? 3 : -1);
-        if (act && wfx >= 0 && a.nbr[4 * e + wfx] == -1) wq[0] = a.fvb + (((size_t)e * 4 + wfx) * n + j) * 6;
-        if (act && wfy >= 0 && a.nbr[4 * e + wfy] == -1) wq[1] = a.fvb + (((size_t)e * 4 + wfy) * n + i) * 6;
+        if (act && wfx >= 0 && in.nbx == -1) wq[0] = a.fvb + (((size_t)e * 4 + wfx) * n + j) * 6;
+        if (act && wfy >= 0 && in.nby == -1) wq[1] = a.fvb + (((size_t)e * 4 + wfy) * n + i) * 6;
     }
-    if constexpr (CURV) load4(a.Ja + off, Jn);
-    if constexpr (CURV && !PAR) {
-        if constexpr (KIND == VOL_LW) {
-            lwc_element<N, EB>(uN, Jn, invJ, gm1, i, j, act, sidx, sbase, s0, s1, s2, sDm, sDh, Uc, F, G, vol);
-        } else if constexpr (KIND == VOL_LW_SRC) {
-            lwc_element<N, EB, true>(uN, Jn, invJ, gm1, i, j, act, sidx, sbase, s0, s1, s2, sDm, sDh, Uc, F, G, vol,
-                                     nullptr, 0.0, 0.0, &sp, Ssrc, dt);
-        } else if constexpr (KIND == VOL_MDRK1_SRC) {
-            mdrkc1_element<N, EB, true>(uN, Jn, invJ, gm1, i, j, act, sidx, sbase, s0, s2, sDm, sDh, Uc, F, G, vol,
-                                        &sp, Ssrc, dt);
-        } else if constexpr (KIND == VOL_MDRK2_SRC) {
-            double usn[4];
-            load4(a.us + off, usn);
-            mdrkc2_element<N, EB, true>(uN, usn, Jn, invJ, gm1, i, j, act, sidx, sbase, s0, s1, s2, sDm, sDh, Uc, F,
-                                        G, vol, &sp, Ssrc, dt);
-        } else if constexpr (KIND == VOL_LW_ADAPT) {
-            lwc_element<N, EB>(uN, Jn, invJ, gm1, i, j, act, sidx, sbase, s0, s1, s2, sDm, sDh, Uc, F, G, vol,
-                               &terr, st->abstol, st->reltol);
-        } else if constexpr (KIND == VOL_MDRK1) {
-            mdrkc1_element<N, EB>(uN, Jn, invJ, gm1, i, j, act, sidx, sbase, s0, s2, sDm, sDh, Uc, F, G, vol);
+    if constexpr (!PAR) {
+        const bool adapt = KB == VOL_LW_ADAPT;
+        if constexpr (KB == VOL_LW || KB == VOL_LW_ADAPT) {
+            lw_element<N, EB, CURV, false, SRC>(uN, Jn, dt, sc, gamma, i, j, act, sidx, sbase, bufA, bufB, sD, sDh,
+                                                Uc, F, G, vol, nullptr, adapt ? &terr : nullptr,
+                                                adapt ? st->abstol : 0.0, adapt ? st->reltol : 0.0, &sp, Ssrc);
+        } else if constexpr (KB == VOL_MDRK1) {
+            mdrk1_element<N, EB, CURV, SRC>(uN, Jn, dt, sc, gamma, i, j, act, sidx, sbase, bufA, bufB, sD, sDh, Uc,
+                                            F, G, vol, &sp, Ssrc);
         } else {
-            double usn[4];
-            load4(a.us + off, usn);
-            mdrkc2_element<N, EB>(uN, usn, Jn, invJ, gm1, i, j, act, sidx, sbase, s0, s1, s2, sDm, sDh, Uc, F, G,
-                                  vol);
+            mdrk2_element<N, EB, CURV, SRC>(uN, in.us, Jn, dt, sc, gamma, i, j, act, sidx, sbase, bufA, bufB, sD,
+                                            sDh, Uc, F, G, vol, &sp, Ssrc);
         }
     } else if constexpr (PAR) {
         // BR1 gradients of uⁿ (and of us in MDRK stage 2), exchanged through a
@@ -2791,46 +2302,28 @@ __device__ __forceinline__ void volume_body(const KArgs& a, int bid, double* lds
             }
         }
         if constexpr (KB == VOL_MDRK2) {
-            double usn[4], gxS[4], gyS[4];
-            load4(a.us + off, usn);
+            const double* usn = in.us;
+            double gxS[4], gyS[4];
             if (act) put4<S>(sg + 4 * S, sidx, usn);
             __syncthreads();
-            br1_gradient<N, EB, CURV>(sg, uin, a.nbr, c, e, i, j, sbase, invJ, sDh, uN, gxN, gyN, Jn);
-            br1_gradient<N, EB, CURV>(sg + 4 * S, a.us, a.nbr, c, e, i, j, sbase, invJ, sDh, usn, gxS, gyS, Jn);
-            mdrkp2_element<N, EB, CURV, WALL>(uN, gxN, gyN, usn, gxS, gyS, invJ, gm1, c, i, j, act, sidx, sbase, s0,
-                                              s1, s2, sDm, sD, sDh, Uc, F, G, vol, Jn, wq, nsrc, nsp, dt, Ssrc);
+            br1_gradient<N, EB, CURV>(sg, uin, in.nbx, in.nby, c, i, j, sbase, invJ, sDh, uN, gxN, gyN, Jn);
+            br1_gradient<N, EB, CURV>(sg + 4 * S, a.us, in.nbx, in.nby, c, i, j, sbase, invJ, sDh, usn, gxS, gyS, Jn);
+            mdrkp2_element<N, EB, CURV, WALL>(uN, gxN, gyN, usn, gxS, gyS, invJ, sc, gm1, c, i, j, act, sidx, sbase, s0,
+                                              s1, s2, sD, sDh, Uc, F, G, vol, Jn, wq, nsrc, nsp, dt, Ssrc);
         } else {
             __syncthreads();
-            br1_gradient<N, EB, CURV>(sg, uin, a.nbr, c, e, i, j, sbase, invJ, sDh, uN, gxN, gyN, Jn);
+            br1_gradient<N, EB, CURV>(sg, uin, in.nbx, in.nby, c, i, j, sbase, invJ, sDh, uN, gxN, gyN, Jn);
             if constexpr (KB == VOL_LW)
-                lwp_element<N, EB, CURV, WALL>(uN, gxN, gyN, invJ, gm1, c, i, j, act, sidx, sbase, s0, s1, s2, sDm,
-                                               sD, sDh, Uc, F, G, vol, Jn, wq, nullptr, 0.0, 0.0, nsrc, nsp, Ssrc,
+                lwp_element<N, EB, CURV, WALL>(uN, gxN, gyN, invJ, sc, gm1, c, i, j, act, sidx, sbase, s0, s1, s2, sD,
+                                               sDh, Uc, F, G, vol, Jn, wq, nullptr, 0.0, 0.0, nsrc, nsp, Ssrc,
                                                dt);
             else if constexpr (KB == VOL_LW_ADAPT)
-                lwp_element<N, EB, CURV, WALL>(uN, gxN, gyN, invJ, gm1, c, i, j, act, sidx, sbase, s0, s1, s2, sDm,
-                                               sD, sDh, Uc, F, G, vol, Jn, wq, &terr, st->abstol, st->reltol);
+                lwp_element<N, EB, CURV, WALL>(uN, gxN, gyN, invJ, sc, gm1, c, i, j, act, sidx, sbase, s0, s1, s2, sD,
+                                               sDh, Uc, F, G, vol, Jn, wq, &terr, st->abstol, st->reltol);
             else
-                mdrkp1_element<N, EB, CURV, WALL>(uN, gxN, gyN, invJ, gm1, c, i, j, act, sidx, sbase, s0, s1, s2, sDm,
-                                                  sD, sDh, Uc, F, G, vol, Jn, wq, nsrc, nsp, dt, Ssrc);
+                mdrkp1_element<N, EB, CURV, WALL>(uN, gxN, gyN, invJ, sc, gm1, c, i, j, act, sidx, sbase, s0, s1, s2, sD,
+                                                  sDh, Uc, F, G, vol, Jn, wq, nsrc, nsp, dt, Ssrc);
         }
-    } else if (KB == VOL_LW || KB == VOL_LW_ADAPT) {
-        if constexpr (N == 4 && KB == VOL_LW_ADAPT)
-            lw4_element<N, EB>(uN, dt, invJ, gm1, c, i, j, act, sidx, sbase, s0, s1, s2, sDm, sDh, Uc, F, G, vol,
-                               nullptr, &terr, st->abstol, st->reltol);
-        else if constexpr (N == 4)
-            lw4_element<N, EB, false, SRC>(uN, dt, invJ, gm1, c, i, j, act, sidx, sbase, s0, s1, s2, sDm, sDh, Uc, F,
-                                           G, vol, nullptr, nullptr, 0.0, 0.0, &sp, Ssrc);
-        else
-            lw3_element<N, EB, false, SRC>(uN, dt, invJ, gm1, c, i, j, act, sidx, sbase, s0, s1, s2, sDm, sDh, Uc, F,
-                                           G, vol, nullptr, &sp, Ssrc);
-    } else if (KB == VOL_MDRK1) {
-        mdrk1_element<N, EB, SRC>(uN, dt, invJ, gm1, c, i, j, act, sidx, sbase, s0, s1, s2, sDm, sDh, Uc, F, G, vol,
-                                  &sp, Ssrc);
-    } else {
-        double usn[4];
-        load4(a.us + off, usn);
-        mdrk2_element<N, EB, SRC>(uN, usn, dt, invJ, gm1, c, i, j, act, sidx, sbase, s0, s1, s2, sDm, sDh, Uc, F, G,
-                                  vol, &sp, Ssrc);
     }
     if (act && a.auxU) {
         store4(a.auxU + off, Uc);
@@ -2918,12 +2411,11 @@ __device__ __forceinline__ void volume_body(const KArgs& a, int bid, double* lds
     }
     // --- face records into LDS (s0, s1 are free), one per face the node lies on.
     // λ ingredients: |v1|, |v2| and c of the λ state, once per node.
-    double* rec = lds;  // [EB][4][n][RQ]
+    double* rec = TWO ? s1 : lds;  // [EB][4][n][RQ]
     const bool tree = c->flux_order == 0;
     const double* jump = tree ? uN : Uc;
     const double* lamst = tree ? Uc : uN;
-    const int nbx = fx >= 0 ? a.nbr[4 * e + fx] : -1;
-    const int nby = fy >= 0 ? a.nbr[4 * e + fy] : -1;
+    const int nbx = in.nbx, nby = in.nby;
     if constexpr (CURV) {
         // structured order with the interface's normal n (shared by both
         // elements): F̃·n, |v(uⁿ)·n| and c(uⁿ)|n| (dg_2d.jl:2229-2264)
@@ -2985,16 +2477,16 @@ __device__ __forceinline__ void volume_body(const KArgs& a, int bid, double* lds
     // workgroup is evaluated once, by the slot of its left element's + face, and
     // its flux goes to both adjacent nodes (accx for x faces, accy for y faces);
     // the record of a face leaving the workgroup goes to HBM for the surface kernel.
-    double* accx = lds + 16 * S;  // pairs of variables (put4), in s2 (free after the last contraction)
+    double* accx = s2;  // pairs of variables (put4); s2 is free after the last contraction
     double* accy = accx + 4 * S;
     constexpr int NSLOT = EB * 4 * n;
     static_assert(NSLOT <= NT, "one face slot per lane");
-    static_assert(EB * 4 * n * RQ <= 16 * S, "records fit in s0 and s1");
+    static_assert(TWO || EB * 4 * n * RQ <= 16 * S, "records fit in s0 and s1");
     if (tid < NSLOT) {
         const int ls = tid / (4 * n), f = (tid / n) % 4, l = tid % n;
         if (ls < nel) {
             const int es = e0 + ls;
-            const int ne = a.nbr[4 * es + f];
+            const int ne = in.slot;
             const double* own = rec + tid * RQ;
             if (!(ne >= e0 && ne < e0 + nel)) {
                 double r[RQ];
@@ -3084,6 +2576,39 @@ __device__ __forceinline__ void volume_body(const KArgs& a, int bid, double* lds
     // kernel's: it reads every node once after the last correction
 }
 
+// The volume workgroup `bid` of a's table.  The loads of a lane's tile data go
+// out together at the start, the neighbours among them, which are first needed
+// after the element procedure (the Navier-Stokes kernels: for the BR1 gradient).
+template <int N, int EB, int KIND, bool SC, bool PAR, bool CURV>
+__device__ __forceinline__ void volume_body(const KArgs& a, int bid, double* lds, double* sDh, double* sD,
+                                            double* s_alpha) {
+    using G_ = VGeo<N, EB>;
+    constexpr int n = G_::n, NN = G_::NN, NSLOT = EB * 4 * n;
+    const int4 blk = load_blk_at(a.vblk, bid);
+    const int tid = threadIdx.x;
+    const int le = tid / NN, node = tid - (tid / NN) * NN;
+    const int i = node % n, j = node / n;
+    const int lec = le < blk.y ? le : blk.y - 1;
+    const int e = blk.x + lec;
+    const size_t off = ((size_t)e * NN + node) * 4;
+    TileIn<CURV, vol_base(KIND) == VOL_MDRK2> in;
+    load4(sel_in(a, a.use_state_dt ? dev_state(a.st + blk.z)->cur : 0) + off, in.u);
+    if constexpr (vol_base(KIND) == VOL_MDRK2) load4(a.us + off, in.us);
+    if constexpr (CURV) load4(a.Ja + off, in.J);
+    in.invJ = CURV ? a.ijn[(size_t)e * NN + node] : a.inv_jac[e];
+    in.nbx = in.nby = in.slot = -1;
+    if (i == 0 || i == n - 1) in.nbx = a.nbr[4 * e + (i == 0 ? 0 : 1)];
+    if (j == 0 || j == n - 1) in.nby = a.nbr[4 * e + (j == 0 ? 2 : 3)];
+    const int ls = tid / (4 * n);
+    if (tid < NSLOT && ls < blk.y) in.slot = a.nbr[4 * (blk.x + ls) + (tid / n) % 4];
+    if (tid < NN) {  // published by the first barrier of the element procedure
+        const int q = (tid / n) * G_::MS + tid % n;
+        sDh[q] = dev_const(a.c)->Dhat[tid / n][tid % n];
+        sD[q] = dev_const(a.c)->D[tid / n][tid % n];
+    }
+    volume_tile<N, EB, KIND, SC, PAR, CURV>(a, bid, blk, in, lds, sDh, sD, s_alpha);
+}
+
 // the Navier-Stokes LW and MDRK stage-2 wall kernels (a rarely used
 // configuration: the lid-driven cavity's walls) run at one wave per SIMD, so
 // their extra wall terms live in the accumulation registers instead of private
@@ -3096,10 +2621,10 @@ constexpr int kVolWavesOf =
 template <int N, int EB, int KIND, bool SC, bool PAR = false, bool CURV = false>
 __global__ __launch_bounds__((VGeo<N, EB>::NT), (kVolWavesOf<KIND, SC, PAR>)) void k_volume(KArgs a) {
     using G_ = VGeo<N, EB>;
-    __shared__ alignas(16) double lds[G_::LDS];
-    __shared__ alignas(16) double sDm[G_::M], sDh[G_::M], sD[G_::M];
+    __shared__ alignas(16) double lds[vol_two_buffers<SC, PAR> ? G_::LDS2 : G_::LDS];
+    __shared__ alignas(16) double sDh[G_::M], sD[G_::M];
     __shared__ double s_alpha[(SC && CURV) ? EB : 1];
-    volume_body<N, EB, KIND, SC, PAR, CURV>(a, blockIdx.x, lds, sDm, sDh, sD, s_alpha);
+    volume_body<N, EB, KIND, SC, PAR, CURV>(a, blockIdx.x, lds, sDh, sD, s_alpha);
 }
 
 // Outer record of a domain-boundary face node: time average of the boundary
@@ -3107,7 +2632,7 @@ __global__ __launch_bounds__((VGeo<N, EB>::NT), (kVolWavesOf<KIND, SC, PAR>)) vo
 template <int N>
 __device__ inline void boundary_record(const KArgs& a, int e, int face, int l, double t, double dt, double* r) {
     constexpr int n = N + 1;
-    const DevConst* c = a.c;
+    const DevC c = dev_const(a.c);
     const int orientation = face < 2 ? 1 : 2;
     const double half = 0.5 * a.length[e];
     double x, y;
@@ -3153,7 +2678,7 @@ template <int N>
 __device__ inline void boundary_record_curved(const KArgs& a, int e, int face, int l, double t, double dt, double* r,
                                               bool p4est_form = false) {
     constexpr int n = N + 1;
-    const DevConst* c = a.c;
+    const DevC c = dev_const(a.c);
     const size_t fo = ((size_t)e * 4 + face) * n + l;
     const double x = a.fxy[2 * fo], y = a.fxy[2 * fo + 1];
     double nf[4];
@@ -3194,7 +2719,7 @@ __device__ __forceinline__ void surface_body(const KArgs& a, int bid) {
     constexpr int n = G_::n, NN = G_::NN, EB = G_::EB, S = G_::S;
     __shared__ double s_l1[S], s_l2[S], s_m[EB], s_lv[S], s_mv[EB];
     const int4 blk = load_blk_at(a.sblk, bid);
-    DevState* st = a.st + blk.z;
+    const DevS st = dev_state(a.st + blk.z);
     if (a.use_state_dt && st->finished) return;
     const int tid = threadIdx.x;
     const int le = tid / NN, node = tid - (tid / NN) * NN;
@@ -3208,7 +2733,7 @@ __device__ __forceinline__ void surface_body(const KArgs& a, int bid) {
     double* out = sel_out(a, cur);
     const double dt = a.use_state_dt ? st->dt : a.dt_arg;
     const double t = a.use_state_dt ? st->t : a.t_arg;
-    const DevConst* c = a.c;
+    const DevC c = dev_const(a.c);
     const double invJ = CURV ? a.ijn[(size_t)e * NN + node] : a.inv_jac[e];
     const int eblk = a.etile[e];
     const int fx = (i == 0) ? 0 : ((i == n - 1) ? 1 : -1);
@@ -3417,7 +2942,7 @@ __device__ __forceinline__ void surface_body(const KArgs& a, int bid) {
     // admissibility test of the updated state cover all nodes here.
     if (act && !any_ext) load4(out + ((size_t)e * NN + node) * 4, val);
     if (a.reduce == RED_ADAPT) {  // test_updated_solution (adaptive.jl:30-46)
-        if (act && !admissible(val, c->gamma)) st->bad_state = 1;
+        if (act && !admissible(val, c->gamma)) a.st[blk.z].bad_state = 1;
         return;
     }
     const bool par = a.pv_off > 0;
@@ -3431,7 +2956,7 @@ __device__ __forceinline__ void surface_body(const KArgs& a, int bid) {
         } else {
             node_speeds(val, c->gamma, l1, l2, bad);
         }
-        if (bad) st->bad_state = 1;
+        if (bad) a.st[blk.z].bad_state = 1;
         s_l1[lec * NN + node] = l1;
         s_l2[lec * NN + node] = l2;
         s_lv[lec * NN + node] = par ? (CURV ? lam_visc_curved(val, invJ, c) : lam_visc(val, invJ, c)) : 0.0;
@@ -3476,7 +3001,9 @@ __global__ __launch_bounds__(kSurfBlock) void k_surface(KArgs a) {
 constexpr int kTransferBlock = 256;
 template <int N>
 __global__ __launch_bounds__(kTransferBlock) void k_transfer(const double* __restrict__ uold, double* __restrict__ unew,
-                                                            const int* __restrict__ plan, int E_new, const DevConst* c) {
+                                                            const int* __restrict__ plan, int E_new,
+                                                            const DevConst* dc) {
+    const DevC c = dev_const(dc);
     constexpr int n = N + 1, NN = n * n;
     const long long gid = (long long)blockIdx.x * kTransferBlock + threadIdx.x;
     if (gid >= (long long)E_new * NN) return;
@@ -3491,8 +3018,8 @@ __global__ __launch_bounds__(kTransferBlock) void k_transfer(const double* __res
         for (int q = 0; q < nsrc; ++q) {
             const int src = (p[0] == 1) ? p[1] : p[1 + q];
             const int child = (p[0] == 1) ? p[2] : q;
-            const double* Mx = (p[0] == 1) ? c->mfwd[child & 1][i] : c->mrev[child & 1][i];
-            const double* My = (p[0] == 1) ? c->mfwd[child >> 1][j] : c->mrev[child >> 1][j];
+            const auto* Mx = (p[0] == 1) ? c->mfwd[child & 1][i] : c->mrev[child & 1][i];
+            const auto* My = (p[0] == 1) ? c->mfwd[child >> 1][j] : c->mrev[child >> 1][j];
             const double* us = uold + (size_t)src * NN * 4;
             for (int l = 0; l < n; ++l) {
                 double t[4] = {0.0, 0.0, 0.0, 0.0};
@@ -3523,7 +3050,7 @@ __global__ __launch_bounds__(kMortarBlock) void k_mortar(KArgs a) {
     constexpr int n = N + 1, MPB = kMortarBlock / n;
     __shared__ double fs[MPB][2][n][4];
     if (a.use_state_dt && a.st[0].finished) return;
-    const DevConst* c = a.c;
+    const DevC c = dev_const(a.c);
     const int tid = threadIdx.x, lm = tid / n, l = tid - lm * n;
     const int m = blockIdx.x * MPB + lm;
     const bool act = lm < MPB && m < a.n_mortars;
@@ -3597,17 +3124,17 @@ __global__ __launch_bounds__(kSurfBlock) void k_max_speed(KArgs a) {
     if (a.Ja) {  // curvilinear mesh: speeds in reference space, |J⁻¹| included
         double Jn[4];
         load4(a.Ja + ((size_t)e * NN + node) * 4, Jn);
-        curved_speeds(val, Jn, a.ijn[(size_t)e * NN + node], a.c->gamma, l1, l2, bad);
+        curved_speeds(val, Jn, a.ijn[(size_t)e * NN + node], dev_const(a.c)->gamma, l1, l2, bad);
     } else {
-        node_speeds(val, a.c->gamma, l1, l2, bad);
+        node_speeds(val, dev_const(a.c)->gamma, l1, l2, bad);
     }
     if (act && bad) st->bad_state = 1;
     const bool par = a.pv_off > 0;
     if (act) {
         s_l1[lec * NN + node] = l1;
         s_l2[lec * NN + node] = l2;
-        s_lv[lec * NN + node] = par ? (a.Ja ? lam_visc_curved(val, a.ijn[(size_t)e * NN + node], a.c)
-                                            : lam_visc(val, a.inv_jac[e], a.c))
+        s_lv[lec * NN + node] = par ? (a.Ja ? lam_visc_curved(val, a.ijn[(size_t)e * NN + node], dev_const(a.c))
+                                            : lam_visc(val, a.inv_jac[e], dev_const(a.c)))
                                     : 0.0;
     }
     __syncthreads();
@@ -3653,7 +3180,7 @@ __global__ __launch_bounds__(kSurfBlock) void k_indicator(KArgs a, double* alpha
     const bool act = le < nel;
     const int lec = le < nel ? le : nel - 1;
     const int e = e0 + lec;
-    const DevConst* c = a.c;
+    const DevC c = dev_const(a.c);
     const double* uin = sel_in(a, a.use_state_dt ? st->cur : 0);
     if (a.use_state_dt && st->finished) return;
     double un[4];
@@ -3724,7 +3251,7 @@ __global__ __launch_bounds__(kSurfBlock) void k_limiter(KArgs a) {
     const int sidx = lec * NN + node, sbase = lec * NN;
     const int cur = a.use_state_dt ? st->cur : 0;
     double* u = sel_out(a, cur);
-    const DevConst* c = a.c;
+    const DevC c = dev_const(a.c);
     const double gm1 = c->gamma - 1.0;
     const size_t off = ((size_t)e * NN + node) * 4;
     double un[4];
@@ -3980,16 +3507,16 @@ __global__ __launch_bounds__(kFinalizeBlock) void k_finalize(FinArgs f) {
 template <int EB3, int EB4>
 __global__ __launch_bounds__((VGeo<4, EB4>::NT), kVolWaves<false>) void k_volume_pair(KArgs a3, KArgs a4, int g3) {
     static_assert(VGeo<3, EB3>::NT == VGeo<4, EB4>::NT, "one block size for both halves");
-    constexpr int L = VGeo<3, EB3>::LDS > VGeo<4, EB4>::LDS ? VGeo<3, EB3>::LDS : VGeo<4, EB4>::LDS;
+    constexpr int L = VGeo<3, EB3>::LDS2 > VGeo<4, EB4>::LDS2 ? VGeo<3, EB3>::LDS2 : VGeo<4, EB4>::LDS2;
     constexpr int M = VGeo<4, EB4>::M;
     static_assert(M >= VGeo<3, EB3>::M, "operators of both degrees");
     __shared__ alignas(16) double lds[L];
-    __shared__ alignas(16) double sDm[M], sDh[M], sD[M];
+    __shared__ alignas(16) double sDh[M], sD[M];
     __shared__ double s_alpha[1];
     if ((int)blockIdx.x < g3)
-        volume_body<3, EB3, VOL_LW, false, false, false>(a3, blockIdx.x, lds, sDm, sDh, sD, s_alpha);
+        volume_body<3, EB3, VOL_LW, false, false, false>(a3, blockIdx.x, lds, sDh, sD, s_alpha);
     else
-        volume_body<4, EB4, VOL_LW, false, false, false>(a4, blockIdx.x - g3, lds, sDm, sDh, sD, s_alpha);
+        volume_body<4, EB4, VOL_LW, false, false, false>(a4, blockIdx.x - g3, lds, sDh, sD, s_alpha);
 }
 
 __global__ __launch_bounds__(kSurfBlock) void k_surface_pair(KArgs a3, KArgs a4, int g3) {
