@@ -61,10 +61,11 @@ struct tlw_ctx {
     double* d_partial = nullptr;
     double* d_alpha_tmp = nullptr;
     double* d_alpha = nullptr;
-    // workgroup tables (KArgs::vblk, sblk, etile) and per-instance partial ranges
+    // workgroup tables (KArgs::vblk, sblk, link) and per-instance partial ranges
     int4* d_vblk = nullptr;
     int4* d_sblk = nullptr;
-    int* d_etile = nullptr;
+    int* d_link = nullptr;
+    std::vector<int> h_nbr;  // the neighbour table, for the links of a new tile
     int4* d_rng = nullptr;
     int vgrid = 0, sgrid = 0, vcap = 0;
     bool sc = false;
@@ -173,7 +174,7 @@ void free_mesh(tlw_ctx* c) {
     drop_graphs(c);
     void* ptrs[] = {c->d_nbr,       c->d_invj,  c->d_center, c->d_length, c->d_trace,   c->d_buf[0],    c->d_buf[1],
                     c->d_us,        c->d_auxU,  c->d_auxF,   c->d_partial, c->d_alpha_tmp, c->d_alpha,
-                    c->d_vblk,      c->d_sblk,  c->d_etile,  c->d_rng,    c->d_state,   c->d_cur,
+                    c->d_vblk,      c->d_sblk,  c->d_link,  c->d_rng,    c->d_state,   c->d_cur,
                     c->d_Ja,        c->d_ijn,   c->d_fnorm,  c->d_fxy,     c->d_snrm,      c->d_sqrk,
                     c->d_fvb,       c->d_bidx,  c->d_btab,   c->d_mort,   c->d_mrec,    c->d_mflux,
                     c->d_plink,     c->d_nxy};
@@ -184,7 +185,7 @@ void free_mesh(tlw_ctx* c) {
     c->d_buf[0] = c->d_buf[1] = nullptr;
     c->d_partial = c->d_alpha_tmp = c->d_alpha = nullptr;
     c->d_vblk = c->d_sblk = c->d_rng = nullptr;
-    c->d_etile = nullptr;
+    c->d_link = nullptr;
     c->d_state = nullptr;
     c->h_state = nullptr;
     c->d_cur = nullptr;
@@ -204,8 +205,8 @@ void free_mesh(tlw_ctx* c) {
 
 // Workgroup tables for the current tile: volume workgroups of ebv elements and
 // node-per-lane workgroups of the surface size, both restarted at every
-// instance boundary, the element -> volume workgroup map and each instance's
-// range of partials (volume workgroups, then the node-per-lane grid after them).
+// instance boundary, the faces that leave a volume workgroup (KArgs::link) and each
+// instance's range of partials (volume workgroups, then the node-per-lane grid after them).
 int build_tables(tlw_ctx* c) {
     std::vector<int4> vb, sb, rng(c->ninst);
     std::vector<int> et(c->E);
@@ -226,6 +227,9 @@ int build_tables(tlw_ctx* c) {
     if ((int)vb.size() > c->vcap) return fail(c, TLW_EINVAL, "volume workgroup table exceeds its allocation");
     c->vgrid = (int)vb.size();
     c->sgrid = (int)sb.size();
+    std::vector<int> link(c->h_nbr);
+    for (size_t q = 0; q < link.size(); ++q)
+        if (link[q] >= 0 && et[link[q]] == et[q / 4]) link[q] = kResolved;
     for (auto& r : rng) {  // surface partials follow the volume ones
         r.z += c->vgrid;
         r.w += c->vgrid;
@@ -233,7 +237,7 @@ int build_tables(tlw_ctx* c) {
     HIPCHK(c, hipStreamSynchronize(c->stream));
     HIPCHK(c, hipMemcpy(c->d_vblk, vb.data(), sizeof(int4) * vb.size(), hipMemcpyHostToDevice));
     HIPCHK(c, hipMemcpy(c->d_sblk, sb.data(), sizeof(int4) * sb.size(), hipMemcpyHostToDevice));
-    HIPCHK(c, hipMemcpy(c->d_etile, et.data(), sizeof(int) * et.size(), hipMemcpyHostToDevice));
+    HIPCHK(c, hipMemcpy(c->d_link, link.data(), sizeof(int) * link.size(), hipMemcpyHostToDevice));
     HIPCHK(c, hipMemcpy(c->d_rng, rng.data(), sizeof(int4) * rng.size(), hipMemcpyHostToDevice));
     drop_graphs(c);
     return TLW_OK;
@@ -508,7 +512,7 @@ int upload_meshes(tlw_ctx* c, const tlw_mesh_desc* ms, int ninst, const tlw_curv
     HIPCHK(c, hipMemset(c->d_partial, 0, sizeof(double) * npart));
     HIPCHK(c, hipMalloc(&c->d_vblk, sizeof(int4) * (size_t)c->vcap));
     HIPCHK(c, hipMalloc(&c->d_sblk, sizeof(int4) * (size_t)scap));
-    HIPCHK(c, hipMalloc(&c->d_etile, sizeof(int) * (size_t)E));
+    HIPCHK(c, hipMalloc(&c->d_link, sizeof(int) * 4 * (size_t)E));
     HIPCHK(c, hipMalloc(&c->d_rng, sizeof(int4) * (size_t)ninst));
     if (c->hconst.ns_walls) HIPCHK(c, hipMalloc(&c->d_fvb, sizeof(double) * (size_t)E * 4 * c->n * 6));
     if (pd) {
@@ -541,6 +545,7 @@ int upload_meshes(tlw_ctx* c, const tlw_mesh_desc* ms, int ninst, const tlw_curv
     }
     HIPCHK(c, hipMemcpy(c->d_state, c->h_state, sizeof(DevState) * ninst, hipMemcpyHostToDevice));
     HIPCHK(c, hipMemcpy(c->d_nbr, nbr.data(), sizeof(int) * 4 * E, hipMemcpyHostToDevice));
+    c->h_nbr.assign(nbr.begin(), nbr.end());
     HIPCHK(c, hipMemcpy(c->d_invj, invj.data(), sizeof(double) * E, hipMemcpyHostToDevice));
     HIPCHK(c, hipMemcpy(c->d_center, center.data(), sizeof(double) * 2 * E, hipMemcpyHostToDevice));
     HIPCHK(c, hipMemcpy(c->d_length, length.data(), sizeof(double) * E, hipMemcpyHostToDevice));
@@ -625,7 +630,7 @@ KArgs base_args(tlw_ctx* c) {
     a.ebv = c->ebv;
     a.vblk = c->d_vblk;
     a.sblk = c->d_sblk;
-    a.etile = c->d_etile;
+    a.link = c->d_link;
     a.alpha_tmp = c->d_alpha_tmp;
     a.alpha_out = c->d_alpha;
     a.bc_scale = 1.0;

@@ -138,6 +138,9 @@ __device__ __forceinline__ DevS dev_state(const DevState* p) { return (DevS)(uin
 template <class T> using ConstArr = const __attribute__((address_space(4))) T*;
 template <class T> __device__ __forceinline__ ConstArr<T> const_arr(const T* p) { return (ConstArr<T>)(uintptr_t)p; }
 
+// a face whose two elements share a volume workgroup (KArgs::link)
+constexpr int kResolved = -0x7fffffff;
+
 enum BufSel { SEL_EXPLICIT = 0, SEL_CUR = 1, SEL_OTHER = 2 };
 // RED_ADAPT: adaptive step (per-workgroup sums of the temporal errors and the
 // admissibility test of the updated state instead of CFL maxima)
@@ -196,7 +199,7 @@ struct KArgs {
     // straddle two instances of a batch, so each reads one instance's state.
     const int4* vblk;
     const int4* sblk;
-    const int* etile;  // [E] volume workgroup of each element
+    const int* link;   // [E][4] nbr for the faces that leave a volume workgroup, kResolved for the others
     const double* alpha_tmp;  // indicator values before smoothing [E]
     double* alpha_out;        // smoothed blending factors [E] (optional)
     // hyperbolic-parabolic CFL reduction: the per-workgroup maxima of the
@@ -562,6 +565,76 @@ __device__ __forceinline__ void slot_max(double* slots, int inst, int which, dou
         atomicMax(reinterpret_cast<unsigned long long*>(slots + ((size_t)inst * 2 + which) * kSlots +
                                                         (blockIdx.x & (kSlots - 1))),
                   (unsigned long long)__double_as_longlong(v));
+}
+
+// v of the lane that the DPP control picks (a lane of the same row of 16).
+template <int CTRL> __device__ __forceinline__ double dpp_f64(double v) {
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double readlane_f64(double v, int lane) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                            __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+// maximum over the 8 lanes of a group, over a row's two groups, over the rows
+// (non-negative operands; a NaN loses against any of them, as in dmax(m, NaN))
+__device__ __forceinline__ double max_group8(double v) {
+    v = fmax(v, dpp_f64<0xB1>(v));   // quad_perm 1 0 3 2
+    v = fmax(v, dpp_f64<0x4E>(v));   // quad_perm 2 3 0 1
+    return fmax(v, dpp_f64<0x141>(v));  // row_half_mirror
+}
+__device__ __forceinline__ double max_groups(double v) {
+    v = fmax(v, dpp_f64<0x128>(v));  // row_ror 8
+    return fmax(fmax(readlane_f64(v, 0), readlane_f64(v, 16)), fmax(readlane_f64(v, 32), readlane_f64(v, 48)));
+}
+
+// The CFL maxima of a node-per-lane workgroup of nel elements into its slots:
+// J⁻¹ (max λ1 + max λ2) over its elements (with `scaled`, a curvilinear mesh,
+// the speeds carry the node's |J⁻¹| and invJ is not used), and with par the
+// maximum of the viscous bounds lv.  Every lane of the workgroup calls it, with
+// the node's values where act.  One barrier, then the first wave takes eight
+// lanes per element.  One lane per element walking its 25 nodes was most of the
+// instructions of the kernels that end with it: at 1024², N=4, the surface
+// kernel went from 548 to 411 us (2.7 GB, now at HBM speed), the initial dt's
+// k_max_speed from 415 to 169 us (0.84 GB).
+template <int N>
+__device__ __forceinline__ void cfl_maxima(double* slots, int inst, int tid, int nel, int sidx, bool act, bool first,
+                                           double l1, double l2, double lv, double invJ, bool scaled, bool par) {
+    using G_ = SGeo<N>;
+    constexpr int NN = G_::NN, EB = G_::EB;
+    static_assert(EB <= 8, "eight lanes per element in one wave");
+    __shared__ double2 s_l[G_::S];
+    __shared__ double s_v[G_::S], s_j[EB];
+    if (act) {
+        s_l[sidx] = make_double2(l1, l2);
+        if (par) s_v[sidx] = lv;
+        if (first) s_j[sidx / NN] = invJ;
+    }
+    __syncthreads();
+    if (tid >= 64) return;
+    const int el = tid >> 3, q = tid & 7;
+    double m1 = 0.0, m2 = 0.0, mv = 0.0;
+    if (el < nel) {
+#pragma unroll
+        for (int k = 0; k < NN; k += 8) {
+            if (k + q >= NN) continue;
+            const double2 x = s_l[el * NN + k + q];
+            m1 = fmax(m1, x.x);
+            m2 = fmax(m2, x.y);
+            if (par) mv = fmax(mv, s_v[el * NN + k + q]);
+        }
+    }
+    m1 = max_group8(m1);
+    m2 = max_group8(m2);
+    double bm = 0.0;
+    if (el < nel) bm = scaled ? m1 + m2 : s_j[el] * (m1 + m2);
+    bm = max_groups(bm);
+    if (par) mv = max_groups(max_group8(mv));
+    if (tid == 0) {
+        slot_max(slots, inst, 0, bm);
+        if (par) slot_max(slots, inst, 1, mv);
+    }
 }
 
 // Square root of a positive normal argument: the hardware reciprocal
@@ -2717,7 +2790,6 @@ template <int N, bool BC, bool SC, bool CURV = false, bool MORT = false>
 __device__ __forceinline__ void surface_body(const KArgs& a, int bid) {
     using G_ = SGeo<N>;
     constexpr int n = G_::n, NN = G_::NN, EB = G_::EB, S = G_::S;
-    __shared__ double s_l1[S], s_l2[S], s_m[EB], s_lv[S], s_mv[EB];
     const int4 blk = load_blk_at(a.sblk, bid);
     const DevS st = dev_state(a.st + blk.z);
     if (a.use_state_dt && st->finished) return;
@@ -2735,18 +2807,17 @@ __device__ __forceinline__ void surface_body(const KArgs& a, int bid) {
     const double t = a.use_state_dt ? st->t : a.t_arg;
     const DevC c = dev_const(a.c);
     const double invJ = CURV ? a.ijn[(size_t)e * NN + node] : a.inv_jac[e];
-    const int eblk = a.etile[e];
     const int fx = (i == 0) ? 0 : ((i == n - 1) ? 1 : -1);
     const int fy = (j == 0) ? 2 : ((j == n - 1) ? 3 : -1);
-    const int nbx = fx >= 0 ? a.nbr[4 * e + fx] : 0;
-    const int nby = fy >= 0 ? a.nbr[4 * e + fy] : 0;
-    const bool extx = fx >= 0 && (nbx < 0 || a.etile[nbx] != eblk);
-    const bool exty = fy >= 0 && (nby < 0 || a.etile[nby] != eblk);
-    const bool any_ext = extx || exty;
+    // the node's value and its faces' links go out together
+    const size_t off = ((size_t)e * NN + node) * 4;
+    int nbx = kResolved, nby = kResolved;
+    if (fx >= 0) nbx = a.link[4 * e + fx];
+    if (fy >= 0) nby = a.link[4 * e + fy];
     double val[4];
-    if (act && any_ext) {
-        const size_t off = ((size_t)e * NN + node) * 4;
-        load4(out + off, val);
+    load4(out + off, val);
+    const bool extx = nbx != kResolved, exty = nby != kResolved;
+    if (act && (extx || exty)) {
         double surf[4] = {0.0, 0.0, 0.0, 0.0};
         constexpr int RQ = kRQ<SC>;
         auto do_face = [&](int f, int l, int nb) {
@@ -2937,52 +3008,26 @@ __device__ __forceinline__ void surface_body(const KArgs& a, int bid) {
         store4(out + off, val);
     }
     if (a.reduce == RED_NONE) return;
-    // Every node's final value: the corrected ones are in registers, the volume
-    // kernel finalised the others.  CFL maxima (Trixi max_dt) and the
-    // admissibility test of the updated state cover all nodes here.
-    if (act && !any_ext) load4(out + ((size_t)e * NN + node) * 4, val);
+    // Every node's final value, corrected here or finalised by the volume kernel:
+    // CFL maxima (Trixi max_dt) and the admissibility test of the updated state
+    // cover all nodes here.
     if (a.reduce == RED_ADAPT) {  // test_updated_solution (adaptive.jl:30-46)
         if (act && !admissible(val, c->gamma)) a.st[blk.z].bad_state = 1;
         return;
     }
     const bool par = a.pv_off > 0;
-    if (act) {
-        double l1, l2;
-        bool bad;
-        if constexpr (CURV) {
-            double Jn[4];
-            load4(a.Ja + ((size_t)e * NN + node) * 4, Jn);
-            curved_speeds(val, Jn, invJ, c->gamma, l1, l2, bad);
-        } else {
-            node_speeds(val, c->gamma, l1, l2, bad);
-        }
-        if (bad) a.st[blk.z].bad_state = 1;
-        s_l1[lec * NN + node] = l1;
-        s_l2[lec * NN + node] = l2;
-        s_lv[lec * NN + node] = par ? (CURV ? lam_visc_curved(val, invJ, c) : lam_visc(val, invJ, c)) : 0.0;
+    double l1, l2;
+    bool bad;
+    if constexpr (CURV) {
+        double Jn[4];
+        load4(a.Ja + off, Jn);
+        curved_speeds(val, Jn, invJ, c->gamma, l1, l2, bad);
+    } else {
+        node_speeds(val, c->gamma, l1, l2, bad);
     }
-    __syncthreads();
-    if (act && node == 0) {
-        double m1 = 0.0, m2 = 0.0, mv = 0.0;
-        for (int k = 0; k < NN; ++k) {
-            m1 = dmax(m1, s_l1[lec * NN + k]);
-            m2 = dmax(m2, s_l2[lec * NN + k]);
-            mv = dmax(mv, s_lv[lec * NN + k]);
-        }
-        // curvilinear speeds carry the node's |J⁻¹| already
-        s_m[lec] = CURV ? m1 + m2 : invJ * (m1 + m2);
-        s_mv[lec] = mv;
-    }
-    __syncthreads();
-    if (tid == 0) {
-        double bm = 0.0, bv = 0.0;
-        for (int k = 0; k < nel; ++k) {
-            bm = dmax(bm, s_m[k]);
-            bv = dmax(bv, s_mv[k]);
-        }
-        slot_max(a.slots, blk.z, 0, bm);
-        if (par) slot_max(a.slots, blk.z, 1, bv);
-    }
+    if (act && bad) a.st[blk.z].bad_state = 1;
+    const double lv = par ? (CURV ? lam_visc_curved(val, invJ, c) : lam_visc(val, invJ, c)) : 0.0;
+    cfl_maxima<N>(a.slots, blk.z, tid, nel, lec * NN + node, act, node == 0, l1, l2, lv, invJ, CURV, par);
 }
 
 template <int N, bool BC, bool SC, bool CURV = false, bool MORT = false>
@@ -3105,59 +3150,34 @@ __global__ __launch_bounds__(kMortarBlock) void k_mortar(KArgs a) {
 template <int N>
 __global__ __launch_bounds__(kSurfBlock) void k_max_speed(KArgs a) {
     using G_ = SGeo<N>;
-    constexpr int NN = G_::NN, EB = G_::EB, S = G_::S;
-    __shared__ double s_l1[S], s_l2[S], s_m[EB], s_lv[S], s_mv[EB];
+    constexpr int NN = G_::NN;
     const int4 blk = load_blk(a.sblk);
-    DevState* st = a.st + blk.z;
     const int tid = threadIdx.x;
     const int le = tid / NN, node = tid - (tid / NN) * NN;
-    const int e0 = blk.x;
     const int nel = blk.y;
     const bool act = le < nel;
     const int lec = le < nel ? le : nel - 1;
-    const int e = e0 + lec;
-    const double* uin = sel_in(a, st->cur);
+    const int e = blk.x + lec;
+    const DevC c = dev_const(a.c);
+    const size_t off = ((size_t)e * NN + node) * 4;
+    const double* uin = sel_in(a, dev_state(a.st + blk.z)->cur);
     double val[4];
-    load4(uin + ((size_t)e * NN + node) * 4, val);
+    load4(uin + off, val);
+    const bool curv = a.Ja != nullptr;  // speeds in reference space, |J⁻¹| included
+    const double invJ = curv ? a.ijn[(size_t)e * NN + node] : a.inv_jac[e];
     double l1, l2;
     bool bad;
-    if (a.Ja) {  // curvilinear mesh: speeds in reference space, |J⁻¹| included
+    if (curv) {
         double Jn[4];
-        load4(a.Ja + ((size_t)e * NN + node) * 4, Jn);
-        curved_speeds(val, Jn, a.ijn[(size_t)e * NN + node], dev_const(a.c)->gamma, l1, l2, bad);
+        load4(a.Ja + off, Jn);
+        curved_speeds(val, Jn, invJ, c->gamma, l1, l2, bad);
     } else {
-        node_speeds(val, dev_const(a.c)->gamma, l1, l2, bad);
+        node_speeds(val, c->gamma, l1, l2, bad);
     }
-    if (act && bad) st->bad_state = 1;
+    if (act && bad) a.st[blk.z].bad_state = 1;
     const bool par = a.pv_off > 0;
-    if (act) {
-        s_l1[lec * NN + node] = l1;
-        s_l2[lec * NN + node] = l2;
-        s_lv[lec * NN + node] = par ? (a.Ja ? lam_visc_curved(val, a.ijn[(size_t)e * NN + node], dev_const(a.c))
-                                            : lam_visc(val, a.inv_jac[e], dev_const(a.c)))
-                                    : 0.0;
-    }
-    __syncthreads();
-    if (act && node == 0) {
-        double m1 = 0.0, m2 = 0.0, mv = 0.0;
-        for (int k = 0; k < NN; ++k) {
-            m1 = dmax(m1, s_l1[lec * NN + k]);
-            m2 = dmax(m2, s_l2[lec * NN + k]);
-            mv = dmax(mv, s_lv[lec * NN + k]);
-        }
-        s_m[lec] = a.Ja ? m1 + m2 : a.inv_jac[e] * (m1 + m2);
-        s_mv[lec] = mv;
-    }
-    __syncthreads();
-    if (tid == 0) {
-        double bm = 0.0, bv = 0.0;
-        for (int k = 0; k < nel; ++k) {
-            bm = dmax(bm, s_m[k]);
-            bv = dmax(bv, s_mv[k]);
-        }
-        slot_max(a.slots, blk.z, 0, bm);
-        if (par) slot_max(a.slots, blk.z, 1, bv);
-    }
+    const double lv = par ? (curv ? lam_visc_curved(val, invJ, c) : lam_visc(val, invJ, c)) : 0.0;
+    cfl_maxima<N>(a.slots, blk.z, tid, nel, lec * NN + node, act, node == 0, l1, l2, lv, invJ, curv, par);
 }
 
 // Hennemann-Gassner indicator (Trixi IndicatorHennemannGassner, Hennemann et
@@ -3296,50 +3316,22 @@ __global__ __launch_bounds__(kSurfBlock) void k_limiter(KArgs a) {
     }
     if (act && changed) store4(u + off, un);
     if (a.reduce == RED_NONE) return;
-    // per-element max of λ1, λ2 of the limited state (curvilinear speeds carry the
-    // node's |J⁻¹|; Navier-Stokes adds the viscous bound), one partial per workgroup
+    // CFL maxima of the limited state (curvilinear speeds carry the node's |J⁻¹|;
+    // Navier-Stokes adds the viscous bound)
+    const bool curv = a.Ja != nullptr, par = a.pv_off > 0;
+    const double invJ = curv ? a.ijn[(size_t)e * NN + node] : a.inv_jac[e];
     double l1, l2;
     bool bad;
-    if (a.Ja) {
+    if (curv) {
         double Jn[4];
         load4(a.Ja + off, Jn);
-        curved_speeds(un, Jn, a.ijn[(size_t)e * NN + node], c->gamma, l1, l2, bad);
+        curved_speeds(un, Jn, invJ, c->gamma, l1, l2, bad);
     } else {
         node_speeds(un, c->gamma, l1, l2, bad);
     }
     if (act && bad) st->bad_state = 1;
-    const bool par = a.pv_off > 0;
-    double* s_l1 = s_var;
-    double* s_l2 = s_q[0];
-    double* s_lv = s_q[1];
-    double* s_mv = s_q[2];
-    if (act) {
-        s_l1[sidx] = l1;
-        s_l2[sidx] = l2;
-        s_lv[sidx] = par ? (a.Ja ? lam_visc_curved(un, a.ijn[(size_t)e * NN + node], c) : lam_visc(un, a.inv_jac[e], c))
-                         : 0.0;
-    }
-    __syncthreads();
-    if (act && node == 0) {
-        double m1 = 0.0, m2 = 0.0, mv = 0.0;
-        for (int k = 0; k < NN; ++k) {
-            m1 = dmax(m1, s_l1[sbase + k]);
-            m2 = dmax(m2, s_l2[sbase + k]);
-            mv = dmax(mv, s_lv[sbase + k]);
-        }
-        s_theta[lec] = a.Ja ? m1 + m2 : a.inv_jac[e] * (m1 + m2);
-        s_mv[lec] = mv;
-    }
-    __syncthreads();
-    if (tid == 0) {
-        double bm = 0.0, bv = 0.0;
-        for (int k = 0; k < nel; ++k) {
-            bm = dmax(bm, s_theta[k]);
-            bv = dmax(bv, s_mv[k]);
-        }
-        slot_max(a.slots, blk.z, 0, bm);
-        if (par) slot_max(a.slots, blk.z, 1, bv);
-    }
+    const double lv = par ? (curv ? lam_visc_curved(un, invJ, c) : lam_visc(un, invJ, c)) : 0.0;
+    cfl_maxima<N>(a.slots, blk.z, tid, nel, sidx, act, node == 0, l1, l2, lv, invJ, curv, par);
 }
 
 // Step control of the adaptive LW loop (perform_step! for Adaptive and LW,
