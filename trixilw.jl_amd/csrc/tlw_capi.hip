@@ -10,6 +10,7 @@
 // own time, dt and CFL reduction, advanced by the same launches.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -68,6 +69,7 @@ struct tlw_ctx {
     std::vector<int> h_nbr;  // the neighbour table, for the links of a new tile
     int4* d_rng = nullptr;
     int vgrid = 0, sgrid = 0, vcap = 0;
+    int sbnd = 0;  // the first sbnd node-per-lane workgroups hold the elements with a boundary face (0: mixed)
     bool sc = false;
     bool parabolic = false;   // compressible Navier-Stokes (tlw_create_parabolic)
     // curvilinear StructuredMesh (tlw_create_curved): per node Ja [E][n²][4] and
@@ -165,6 +167,8 @@ bool eb_supported(int N, int eb) {
 }
 int surf_eb(int N) { return N == 4 ? SGeo<4>::EB : SGeo<3>::EB; }
 
+constexpr int kSplitSurface = 4096;  // workgroups (build_tables)
+
 void drop_graphs(tlw_ctx* c) {
     for (auto& kv : c->graph_cache) (void)hipGraphExecDestroy(kv.second);
     c->graph_cache.clear();
@@ -223,6 +227,20 @@ int build_tables(tlw_ctx* c) {
         rng[k].z = (int)sb.size();
         for (int e = f0; e < f1; e += seb) sb.push_back(make_int4(e, std::min(seb, f1 - e), k, 0));
         rng[k].w = (int)sb.size();
+    }
+    // The boundary code holds the surface kernel to two waves per SIMD (181 VGPRs
+    // against 78): on a large mesh the workgroups without a boundary face come last
+    // and run in a launch of their own without it.  The Riemann problem with shock
+    // capturing, N=4: at 128² (3277 workgroups) a step takes 99.0 us split and 97.6
+    // whole, at 256² (13108) the surface part 57 us split and 71 whole.
+    c->sbnd = 0;
+    if (c->bc_faces && !c->p4est && (int)sb.size() >= kSplitSurface) {
+        auto mid = std::stable_partition(sb.begin(), sb.end(), [&](const int4& w) {
+            for (int q = 4 * w.x; q < 4 * (w.x + w.y); ++q)
+                if (c->h_nbr[q] == -1) return true;
+            return false;
+        });
+        c->sbnd = (int)(mid - sb.begin());
     }
     if ((int)vb.size() > c->vcap) return fail(c, TLW_EINVAL, "volume workgroup table exceeds its allocation");
     c->vgrid = (int)vb.size();
@@ -793,7 +811,6 @@ void launch_finalize(tlw_ctx* c, int reduce, int use_vol) {
         hipLaunchKernelGGL(k_finalize<3>, dim3(c->ninst), dim3(kFinalizeBlock), 0, c->stream, f);
 }
 template <int N> void launch_surface_t(tlw_ctx* c, const KArgs& a) {
-    dim3 g(c->sgrid), b(kSurfBlock);
     if (c->curved && c->has_boundary && a.in_sel == SEL_EXPLICIT && !a.u) {
         // the curvilinear boundary faces read uⁿ: never launch without it
         c->bad_launch = true;
@@ -804,27 +821,33 @@ template <int N> void launch_surface_t(tlw_ctx* c, const KArgs& a) {
         hipLaunchKernelGGL(HIP_KERNEL_NAME(k_mortar<N>), dim3((c->n_mortars + MPB - 1) / MPB), dim3(kMortarBlock), 0,
                            c->stream, a);
     }
-    if (c->curved) {
-        if (c->sc) {
-            if (c->has_boundary) hipLaunchKernelGGL(HIP_KERNEL_NAME(k_surface<N, true, true, true>), g, b, 0, c->stream, a);
-            else hipLaunchKernelGGL(HIP_KERNEL_NAME(k_surface<N, false, true, true>), g, b, 0, c->stream, a);
-        } else if (c->has_boundary) {
-            hipLaunchKernelGGL(HIP_KERNEL_NAME(k_surface<N, true, false, true>), g, b, 0, c->stream, a);
+    // the instantiation with boundary code, then (sbnd > 0) without it for the rest
+    auto launch = [&](bool bc, int first, int count) {
+        if (count <= 0) return;
+        KArgs q = a;
+        q.sblk += first;
+        const dim3 g(count), b(kSurfBlock);
+        if (c->curved && c->sc) {
+            if (bc) hipLaunchKernelGGL(HIP_KERNEL_NAME(k_surface<N, true, true, true>), g, b, 0, c->stream, q);
+            else hipLaunchKernelGGL(HIP_KERNEL_NAME(k_surface<N, false, true, true>), g, b, 0, c->stream, q);
+        } else if (c->curved) {
+            if (bc) hipLaunchKernelGGL(HIP_KERNEL_NAME(k_surface<N, true, false, true>), g, b, 0, c->stream, q);
+            else hipLaunchKernelGGL(HIP_KERNEL_NAME(k_surface<N, false, false, true>), g, b, 0, c->stream, q);
+        } else if (c->n_mortars > 0) {  // plain FR on a TreeMesh with refined cells
+            if (bc) hipLaunchKernelGGL(HIP_KERNEL_NAME(k_surface<N, true, false, false, true>), g, b, 0, c->stream, q);
+            else hipLaunchKernelGGL(HIP_KERNEL_NAME(k_surface<N, false, false, false, true>), g, b, 0, c->stream, q);
+        } else if (c->sc) {
+            if (bc) hipLaunchKernelGGL(HIP_KERNEL_NAME(k_surface<N, true, true>), g, b, 0, c->stream, q);
+            else hipLaunchKernelGGL(HIP_KERNEL_NAME(k_surface<N, false, true>), g, b, 0, c->stream, q);
         } else {
-            hipLaunchKernelGGL(HIP_KERNEL_NAME(k_surface<N, false, false, true>), g, b, 0, c->stream, a);
+            if (bc) hipLaunchKernelGGL(HIP_KERNEL_NAME(k_surface<N, true, false>), g, b, 0, c->stream, q);
+            else hipLaunchKernelGGL(HIP_KERNEL_NAME(k_surface<N, false, false>), g, b, 0, c->stream, q);
         }
-    } else if (c->n_mortars > 0) {  // plain FR on a TreeMesh with refined cells
-        if (c->bc_faces)
-            hipLaunchKernelGGL(HIP_KERNEL_NAME(k_surface<N, true, false, false, true>), g, b, 0, c->stream, a);
-        else
-            hipLaunchKernelGGL(HIP_KERNEL_NAME(k_surface<N, false, false, false, true>), g, b, 0, c->stream, a);
-    } else if (c->sc) {
-        if (c->has_boundary) hipLaunchKernelGGL(HIP_KERNEL_NAME(k_surface<N, true, true>), g, b, 0, c->stream, a);
-        else hipLaunchKernelGGL(HIP_KERNEL_NAME(k_surface<N, false, true>), g, b, 0, c->stream, a);
-    } else {
-        if (c->has_boundary) hipLaunchKernelGGL(HIP_KERNEL_NAME(k_surface<N, true, false>), g, b, 0, c->stream, a);
-        else hipLaunchKernelGGL(HIP_KERNEL_NAME(k_surface<N, false, false>), g, b, 0, c->stream, a);
-    }
+    };
+    const bool bc = c->n_mortars > 0 ? c->bc_faces : c->has_boundary;
+    const int nb = !bc ? 0 : c->sbnd > 0 ? c->sbnd : c->sgrid;
+    launch(true, 0, nb);
+    launch(false, nb, c->sgrid - nb);
     // the step's CFL partials come from the surface kernel alone; with adaptive
     // steps the volume kernel's temporal-error sums are read by the finalize kernel
     if (a.reduce != RED_NONE) launch_finalize(c, a.reduce == RED_ADAPT ? RED_STEP : a.reduce, 0);
@@ -2044,6 +2067,8 @@ int create_common(int ninst, const tlw_mesh_desc* meshes, const tlw_basis_desc* 
             for (int k = 0; k < n; ++k) h.Vinv[i][k] = solver->inverse_vandermonde_host[i + n * k];
         h.alpha_max = solver->alpha_max;
         h.alpha_min = solver->alpha_min;
+        h.hg_threshold = 0.5 * std::pow(10.0, -1.8 * std::pow((double)c->n, 0.25));
+        h.hg_sharpness = std::log((1.0 - 0.0001) / 0.0001);
         h.alpha_smooth = solver->alpha_smooth;
         if (solver->reconstruction != TLW_RECON_FIRST_ORDER && solver->reconstruction != TLW_RECON_MUSCL_HANCOCK) {
             delete c;
