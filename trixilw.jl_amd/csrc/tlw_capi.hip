@@ -87,6 +87,7 @@ struct tlw_ctx {
     size_t slot_off = 0;      // offset of the CFL maxima slots in d_partial
     int pv_off = 0;           // offset of the viscous CFL partials (0: none)
     int ebv = 0;              // elements per volume workgroup
+    bool ebv_given = false;   // by tlw_set_elements_per_workgroup or tlw_autotune; else default_eb of the mesh
     bool positivity = false;  // Zhang-Shu limiter in the device loop
     bool adaptive = false;    // error-controlled steps (tlw_solve_init_adaptive)
     bool has_boundary = false;  // a face with neighbour -1, or a mortar (paths that refuse both test this)
@@ -159,7 +160,17 @@ size_t inst_len(const tlw_ctx* c, int k) {
 constexpr int kEbChoices4[3] = {5, 10, 15};
 constexpr int kEbChoices3[3] = {4, 8, 16};
 const int* eb_choices(int N) { return N == 4 ? kEbChoices4 : kEbChoices3; }
-int default_eb(int N) { return N == 4 ? 15 : 16; }
+// The tile of a context that has not been given one, by its number of elements:
+// small tiles spread a small mesh over the chip, large ones keep more faces inside
+// a workgroup.  Steps of the device loop in us, Euler LW in Z-order, tiles as
+// above: polydeg 4 32² 15.1 / 16.2 / 17.2, 128² 40.7 / 40.6 / 50.7, 256² 118 / 110 / 151
+// (15 elements are six waves, a workgroup and a half on four SIMDs); polydeg 3 32²
+// 14.6 / 14.8 / 15.5, 64² 17.9 / 16.1 / 16.9, 128² 28.3 / 26.4 / 26.9, 256² 70.9 / 65.9 / 62.8.
+// MDRK and Navier-Stokes cross over at the same sizes.
+int default_eb(int N, int E) {
+    if (N == 4) return E <= 16384 ? 5 : 10;
+    return E <= 2048 ? 4 : E <= 32768 ? 8 : 16;
+}
 int min_eb(int N) { return N == 4 ? 5 : 4; }
 bool eb_supported(int N, int eb) {
     const int* ch = eb_choices(N);
@@ -520,6 +531,7 @@ int upload_meshes(tlw_ctx* c, const tlw_mesh_desc* ms, int ninst, const tlw_curv
     HIPCHK(c, hipMalloc(&c->d_us, sizeof(double) * nd));
     // tables and partials sized for the smallest tile, so the tile can change freely
     c->vcap = (E + min_eb(c->N) - 1) / min_eb(c->N) + ninst;
+    if (!c->ebv_given) c->ebv = default_eb(c->N, E);  // at most 256 nodes, as Navier-Stokes walls need
     const int scap = (E + surf_eb(c->N) - 1) / surf_eb(c->N) + ninst;
     // hyperbolic-parabolic: the viscous partials follow in a second block of the same size
     c->pv_off = c->parabolic ? c->vcap + scap : 0;
@@ -1647,6 +1659,7 @@ int tlw_set_elements_per_workgroup(tlw_ctx* c, int32_t elements) {
                                              : "elements per workgroup must be 4, 8 or 16 for polydeg 3");
     if (c->hconst.ns_walls && elements * c->n * c->n > 256)
         return fail(c, TLW_EINVAL, "Navier-Stokes walls: at most 256 nodes per workgroup (polydeg 4: 5 or 10)");
+    c->ebv_given = true;
     if (elements == c->ebv) return TLW_OK;
     HIPCHK(c, hipStreamSynchronize(c->stream));
     c->ebv = elements;
@@ -2034,7 +2047,6 @@ int create_common(int ninst, const tlw_mesh_desc* meshes, const tlw_basis_desc* 
     tlw_ctx* c = new tlw_ctx;
     c->N = basis->polydeg;
     c->n = c->N + 1;
-    c->ebv = default_eb(c->N);
     c->p4est = pd != nullptr;
     c->time_disc = solver->time_discretization;
     c->flags = solver->flags;
@@ -2131,8 +2143,6 @@ int create_common(int ninst, const tlw_mesh_desc* meshes, const tlw_basis_desc* 
         h.visc_Pr = par->prandtl;
         h.visc_kappa = solver->gamma * (1.0 / (solver->gamma - 1.0)) / par->prandtl;
         h.ns_walls = par->walls ? 1 : 0;
-        // the wall kernel runs at one wave per SIMD: a tile of at most 4 waves
-        if (h.ns_walls && c->ebv * c->n * c->n > 256) c->ebv = 10;  // polydeg 4 (polydeg 3 tiles fit)
         for (int k = 0; k < 8; ++k) h.wall_v[k] = par->walls ? par->wall_velocity[k] : 0.0;
         for (int k = 0; k < 4; ++k) {
             h.wall_iso[k] = (par->walls && par->wall_isothermal[k]) ? 1 : 0;

@@ -2609,13 +2609,16 @@ __device__ __forceinline__ void volume_tile(const KArgs& a, int bid, const int4&
 #pragma unroll
         for (int v = 0; v < 4; ++v) surf[v] = fma(Fs[v], wf, surf[v]);
     }
+    // du = -J⁻¹ (vol + surf) + S, or u + dt du rounded once
+    constexpr bool ADD_SRC =
+        SRC || (PAR && !CURV && (KB == VOL_MDRK1 || KB == VOL_MDRK2 || (WALL && KB == VOL_LW)));
+    const double fac = a.step_mode ? sc : -invJ;
     double val[4];
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-        double d = (-invJ) * (vol[v] + surf[v]);
-        if constexpr (SRC || (PAR && !CURV && (KB == VOL_MDRK1 || KB == VOL_MDRK2 || (WALL && KB == VOL_LW))))
-            d += Ssrc[v];
-        val[v] = a.step_mode ? fma(dt, d, uN[v]) : d;
+        val[v] = a.step_mode ? uN[v] : 0.0;
+        if constexpr (ADD_SRC) val[v] = fma(a.step_mode ? dt : 1.0, Ssrc[v], val[v]);
+        val[v] = fma(fac, vol[v] + surf[v], val[v]);
     }
     if (act) store4(out + off, val);
     if constexpr (KB == VOL_LW_ADAPT) {
@@ -3001,11 +3004,9 @@ __device__ __forceinline__ void surface_body(const KArgs& a, int bid) {
         };
         if (extx) do_face(fx, j, nbx);
         if (exty) do_face(fy, i, nby);
+        const double fac = a.step_mode ? -dt * invJ : -invJ;
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const double d = (-invJ) * surf[v];
-            val[v] = a.step_mode ? fma(dt, d, val[v]) : val[v] + d;
-        }
+        for (int v = 0; v < 4; ++v) val[v] = fma(fac, surf[v], val[v]);
         store4(out + off, val);
     }
     if (a.reduce == RED_NONE) return;
