@@ -1487,17 +1487,50 @@ __device__ __forceinline__ void ns_visc_fluxes(const double* u, const double* gx
     fy[3] = (v1 * t12 + v2 * t22 + kappa * Ty) * mu;
 }
 
-// f = f_a(u) - f_v(u, ∇u)
-__device__ __forceinline__ void ns_total_fluxes(const double* u, const double* gx, const double* gy, double gm1,
-                                                DevC c, double* f, double* g) {
-    double fx[4], fy[4];
-    euler_fluxes(u, gm1, f, g);
-    ns_visc_fluxes(u, gx, gy, gm1, c, fx, fy);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        f[v] -= fx[v];
-        g[v] -= fy[v];
-    }
+// The total flux pair f_a(u) - f_v(u, ∇u) as the five values the stencils sum:
+// q = (f2, f3 = g2, f4, g3, g4), the mass fluxes ρv1, ρv2 being linear and
+// without a viscous part (euler_q keeps p out of its sums; here the stresses sit
+// on top of it).  The primitive gradients stay multiplied by ρ and 1/ρ enters
+// the viscosity once: 52 instructions against 77 for the two flux vectors.
+__device__ __forceinline__ void ns_q(const double* u, const double* gx, const double* gy, double gm1, DevC c,
+                                     double* q) {
+    const double ir = rcp_nr(u[0]);
+    const double v1 = u[1] * ir, v2 = u[2] * ir;
+    const double q11 = u[1] * v1, q12 = u[1] * v2, q22 = u[2] * v2;
+    const double hk = 0.5 * (q11 + q22);
+    const double p = gm1 * (u[3] - hk);
+    const double T = p * ir, hv = hk * ir;
+    // ρ ∂v1, ρ ∂v2 and ρ ∂T of one direction
+    auto prim = [&](const double* W, double& a1, double& a2, double& rT) {
+        a1 = fma(-W[0], v1, W[1]);
+        a2 = fma(-W[0], v2, W[2]);
+        const double pd = fma(-v2, a2, fma(-v1, a1, fma(-W[0], hv, W[3])));
+        rT = fma(gm1, pd, -(W[0] * T));
+    };
+    double a1x, a2x, Tx, a1y, a2y, Ty;
+    prim(gx, a1x, a2x, Tx);
+    prim(gy, a1y, a2y, Ty);
+    const double mi = c->visc_mu * ir, ki = mi * c->visc_kappa;
+    const double t11 = mi * fma(4.0 / 3.0, a1x, (-2.0 / 3.0) * a2y);
+    const double t12 = mi * (a1y + a2x);
+    const double t22 = mi * fma(4.0 / 3.0, a2y, (-2.0 / 3.0) * a1x);
+    const double H = u[3] + p;
+    q[0] = (q11 + p) - t11;
+    q[1] = q12 - t12;
+    q[2] = fma(H, v1, -fma(v1, t11, fma(v2, t12, ki * Tx)));
+    q[3] = (q22 + p) - t22;
+    q[4] = fma(H, v2, -fma(v1, t12, fma(v2, t22, ki * Ty)));
+}
+// the flux pair of the sums q and the linear parts of the mass fluxes
+__device__ __forceinline__ void ns_join(const double* q, double l1, double l2, double* f, double* g) {
+    f[0] = l1;
+    f[1] = q[0];
+    f[2] = q[1];
+    f[3] = q[2];
+    g[0] = l2;
+    g[1] = q[1];
+    g[2] = q[3];
+    g[3] = q[4];
 }
 
 // Viscous time-step bound of one node, J⁻² max(4μ/(3ρ), μκ/(ρ Pr))
@@ -1623,10 +1656,9 @@ struct ParStates {
                 y[q][v] = fma(cq[q], wy[v], y[q][v]);
             }
     }
-    __device__ __forceinline__ void flux(int q, double gm1, DevC c, double* f, double* g) const {
-        ns_total_fluxes(u[q], x[q], y[q], gm1, c, f, g);
+    __device__ __forceinline__ void flux(int s, double gm1, DevC c, double* q) const {
+        ns_q(u[s], x[s], y[s], gm1, c, q);
     }
-    // momentum components of the viscous fluxes of state q: (fv1, fv2, gv1, gv2)
     // components 1..3 of the viscous fluxes of state q: (fx1, fx2, fx3, fy1, fy2, fy3)
     __device__ __forceinline__ void visc6(int q, double gm1, DevC c, double* out) const {
         double fx[4], fy[4];
@@ -1696,7 +1728,11 @@ __device__ __forceinline__ void lwp_element(const double* uN, const double* gxN,
                                             double* Ssrc = nullptr, double dtv = 0.0) {
     using G_ = VGeo<N, EB>;
     constexpr int n = G_::n, S = G_::S;
-    ns_total_fluxes(uN, gxN, gyN, gm1, c, F, G);
+    double q0[5], sum[5];
+    ns_q(uN, gxN, gyN, gm1, c, q0);
+    ns_join(q0, uN[1], uN[2], F, G);
+#pragma unroll
+    for (int m = 0; m < 5; ++m) sum[m] = q0[m];
     // the Navier-Stokes convergence source (the wall instantiation, has_src;
     // dg_2d_parabolic.jl:725-1860): level k of the Taylor procedure gets dt·s^(k)
     // before its gradient is formed, S the same weights as F̃ (s^(k) the time
@@ -1768,180 +1804,68 @@ __device__ __forceinline__ void lwp_element(const double* uN, const double* gxN,
         }
     };
     double w[4], wx[4], wy[4];
-    if constexpr (WALL) {
-        double ds[4];
-        src_lvl(0, 1.0, ds);
-        par_level<N, EB, CURV>(act, sidx, sbase, i, j, invJ, sc, s0, s2, sD, F, G, w, wx, wy, Jn, ds);  // ut
-    } else {
-        par_level<N, EB, CURV>(act, sidx, sbase, i, j, invJ, sc, s0, s2, sD, F, G, w, wx, wy, Jn);  // ut
-    }
-    // on a curvilinear mesh s0 took the contravariant pair; the centred stencils
-    // read the node's own Cartesian f(uⁿ), written once every lane has passed
-    // the contraction of s0
-    if constexpr (CURV) {
-        if (act) put8<S>(s0, sidx, F, G);
-    }
     ParStates P;
     P.init(uN, gxN, gyN);
-    P.add(1.0, -1.0, 2.0, -2.0, w, wx, wy);
 #pragma unroll
-    for (int v = 0; v < 4; ++v) Uc[v] = fma(0.5, w[v], uN[v]);
-    double fa[4], ga[4], dx[4], dy[4];
-    // stage 1: f_t = (-f(u++) + 8 f(u+) - 8 f(u-) + f(u--)) / 12
-    P.flux(2, gm1, c, fa, ga);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) { dx[v] = -fa[v]; dy[v] = -ga[v]; }
-    P.flux(0, gm1, c, fa, ga);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) { dx[v] = fma(8.0, fa[v], dx[v]); dy[v] = fma(8.0, ga[v], dy[v]); }
-    P.flux(1, gm1, c, fa, ga);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) { dx[v] = fma(-8.0, fa[v], dx[v]); dy[v] = fma(-8.0, ga[v], dy[v]); }
-    P.flux(3, gm1, c, fa, ga);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        dx[v] = (1.0 / 12.0) * (dx[v] + fa[v]);
-        dy[v] = (1.0 / 12.0) * (dy[v] + ga[v]);
-        F[v] = fma(0.5, dx[v], F[v]);
-        G[v] = fma(0.5, dy[v], G[v]);
-    }
-    // f_t of the viscous part, weight 1/2
-    wall_stage(P, 8.0, -8.0, -1.0, 1.0, 0.0, 1.0 / 12.0, 0.5, true);
-    if constexpr (WALL) {
-        double ds[4];
-        src_lvl(1, 0.5, ds);
-        par_level<N, EB, CURV>(act, sidx, sbase, i, j, invJ, sc, s1, s2, sD, dx, dy, w, wx, wy, Jn, ds);  // utt
-    } else {
-        par_level<N, EB, CURV>(act, sidx, sbase, i, j, invJ, sc, s1, s2, sD, dx, dy, w, wx, wy, Jn);  // utt
-    }
-    P.add(0.5, 0.5, 2.0, 2.0, w, wx, wy);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) Uc[v] = fma(1.0 / 6.0, w[v], Uc[v]);
-    if constexpr (N == 4) {
-        // stage 2: f_tt = (-f(u++) + 16 f(u+) - 30 f + 16 f(u-) - f(u--)) / 12
-        P.flux(2, gm1, c, fa, ga);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) { dx[v] = -fa[v]; dy[v] = -ga[v]; }
-        P.flux(0, gm1, c, fa, ga);
-        double f0[4], g0[4];
-        get4<S>(s0, sidx, f0);
-        get4<S>(s0 + 4 * S, sidx, g0);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            dx[v] = fma(16.0, fa[v], dx[v]);
-            dy[v] = fma(16.0, ga[v], dy[v]);
-            dx[v] = fma(-30.0, f0[v], dx[v]);
-            dy[v] = fma(-30.0, g0[v], dy[v]);
-        }
-        P.flux(1, gm1, c, fa, ga);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) { dx[v] = fma(16.0, fa[v], dx[v]); dy[v] = fma(16.0, ga[v], dy[v]); }
-        P.flux(3, gm1, c, fa, ga);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            dx[v] = (1.0 / 12.0) * (dx[v] - fa[v]);
-            dy[v] = (1.0 / 12.0) * (dy[v] - ga[v]);
-        }
-    } else {
-        // stage 2: f_tt = f(u+) - 2 f + f(u-)
-        P.flux(0, gm1, c, fa, ga);
-        double f0[4], g0[4];
-        get4<S>(s0, sidx, f0);
-        get4<S>(s0 + 4 * S, sidx, g0);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            dx[v] = fma(-2.0, f0[v], fa[v]);
-            dy[v] = fma(-2.0, g0[v], ga[v]);
-        }
-        P.flux(1, gm1, c, fa, ga);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) { dx[v] += fa[v]; dy[v] += ga[v]; }
-    }
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        F[v] = fma(1.0 / 6.0, dx[v], F[v]);
-        G[v] = fma(1.0 / 6.0, dy[v], G[v]);
-    }
-    // f_tt of the viscous part, weight 1/6 (five points at N = 4, three at N = 3)
-    if constexpr (N == 4) wall_stage(P, 16.0, 16.0, -1.0, -1.0, -30.0, 1.0 / 12.0, 1.0 / 6.0, true);
-    else wall_stage(P, 1.0, 1.0, 0.0, 0.0, -2.0, 1.0, 1.0 / 6.0, false);
-    if constexpr (WALL) {
-        double ds[4];
-        src_lvl(2, 1.0 / 6.0, ds);
-        par_level<N, EB, CURV>(act, sidx, sbase, i, j, invJ, sc, s1, s2, sD, dx, dy, w, wx, wy, Jn, ds);  // uttt
-    } else {
-        par_level<N, EB, CURV>(act, sidx, sbase, i, j, invJ, sc, s1, s2, sD, dx, dy, w, wx, wy, Jn);  // uttt
-    }
-    P.add(1.0 / 6.0, -1.0 / 6.0, 4.0 / 3.0, -4.0 / 3.0, w, wx, wy);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) Uc[v] = fma(1.0 / 24.0, w[v], Uc[v]);
-    // stage 3: f_ttt = (f(u++) - 2 f(u+) + 2 f(u-) - f(u--)) / 2
-    P.flux(2, gm1, c, fa, ga);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) { dx[v] = fa[v]; dy[v] = ga[v]; }
-    P.flux(0, gm1, c, fa, ga);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) { dx[v] = fma(-2.0, fa[v], dx[v]); dy[v] = fma(-2.0, ga[v], dy[v]); }
-    P.flux(1, gm1, c, fa, ga);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) { dx[v] = fma(2.0, fa[v], dx[v]); dy[v] = fma(2.0, ga[v], dy[v]); }
-    P.flux(3, gm1, c, fa, ga);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        dx[v] = 0.5 * (dx[v] - fa[v]);
-        dy[v] = 0.5 * (dy[v] - ga[v]);
-        F[v] = fma(1.0 / 24.0, dx[v], F[v]);
-        G[v] = fma(1.0 / 24.0, dy[v], G[v]);
-    }
-    // f_ttt of the viscous part, weight 1/24
-    wall_stage(P, -2.0, 2.0, 1.0, -1.0, 0.0, 0.5, 1.0 / 24.0, true);
-    if constexpr (N == 4) {
+    for (int k = 1; k <= N; ++k) {
+        // F, G: the (k-1)-th time difference of the total flux pair
+        double* sa = k == 1 ? s0 : s1;
         if constexpr (WALL) {
             double ds[4];
-            src_lvl(3, 1.0 / 24.0, ds);
-            par_level<N, EB, CURV>(act, sidx, sbase, i, j, invJ, sc, s1, s2, sD, dx, dy, w, wx, wy, Jn, ds);
+            src_lvl(k - 1, lw_weight(k - 1), ds);
+            par_level<N, EB, CURV>(act, sidx, sbase, i, j, invJ, sc, sa, s2, sD, F, G, w, wx, wy, Jn, ds);
         } else {
-            par_level<N, EB, CURV>(act, sidx, sbase, i, j, invJ, sc, s1, s2, sD, dx, dy, w, wx, wy, Jn);  // utttt
+            par_level<N, EB, CURV>(act, sidx, sbase, i, j, invJ, sc, sa, s2, sD, F, G, w, wx, wy, Jn);
         }
-        P.add(1.0 / 24.0, 1.0 / 24.0, 2.0 / 3.0, 2.0 / 3.0, w, wx, wy);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) Uc[v] = fma(1.0 / 120.0, w[v], Uc[v]);
-        // stage 4: f_tttt = 0.5 (f(u++) - 4 f(u+) + 6 f - 4 f(u-) + f(u--)), with
-        // the reference's factor 0.5 (dg_2d_parabolic.jl:1746-1747)
-        P.flux(2, gm1, c, fa, ga);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) { dx[v] = fa[v]; dy[v] = ga[v]; }
-        P.flux(0, gm1, c, fa, ga);
-        double f0[4], g0[4];
-        get4<S>(s0, sidx, f0);
-        get4<S>(s0 + 4 * S, sidx, g0);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            dx[v] = fma(-4.0, fa[v], dx[v]);
-            dy[v] = fma(-4.0, ga[v], dy[v]);
-            dx[v] = fma(6.0, f0[v], dx[v]);
-            dy[v] = fma(6.0, g0[v], dy[v]);
+        // s0 keeps the node's own Cartesian f(uⁿ) for the centred stencils: on a
+        // curvilinear mesh written once every lane has passed its contraction
+        if constexpr (CURV) {
+            if (k == 1 && act) put8<S>(s0, sidx, F, G);
         }
-        P.flux(1, gm1, c, fa, ga);
+        P.add(kTaylor[0][k - 1], kTaylor[1][k - 1], kTaylor[2][k - 1], kTaylor[3][k - 1], w, wx, wy);
 #pragma unroll
-        for (int v = 0; v < 4; ++v) { dx[v] = fma(-4.0, fa[v], dx[v]); dy[v] = fma(-4.0, ga[v], dy[v]); }
-        P.flux(3, gm1, c, fa, ga);
+        for (int v = 0; v < 4; ++v) Uc[v] = fma(lw_weight(k), w[v], k == 1 ? uN[v] : Uc[v]);
+        constexpr TimeDiff tds[5] = {{}, time_diff<N>(1), time_diff<N>(2), time_diff<N>(3), time_diff<N>(4)};
+        const TimeDiff td = tds[k];
+        double d[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, q[5];
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            dx[v] = 0.5 * (dx[v] + fa[v]);
-            dy[v] = 0.5 * (dy[v] + ga[v]);
-            F[v] = fma(1.0 / 120.0, dx[v], F[v]);
-            G[v] = fma(1.0 / 120.0, dy[v], G[v]);
+        for (int r = 0; r < 5; ++r) {
+            const int s = r == 0 ? 2 : r == 1 ? 0 : r == 2 ? 4 : r == 3 ? 1 : 3;
+            if (td.c[s] == 0.0) continue;
+            if (s < 4) {
+                P.flux(s & 3, gm1, c, q);
+            } else {
+                double f0[4], g0[4];
+                get4<S>(s0, sidx, f0);
+                get4<S>(s0 + 4 * S, sidx, g0);
+                q[0] = f0[1];
+                q[1] = f0[2];
+                q[2] = f0[3];
+                q[3] = g0[2];
+                q[4] = g0[3];
+            }
+#pragma unroll
+            for (int m = 0; m < 5; ++m) d[m] = fma(td.c[s], q[m], d[m]);
         }
-        // s0 is read only at the own node since the first contraction: it takes
-        // the total f_tttt for the temporal error
-        if (terr && act) put8<S>(s0, sidx, dx, dy);
+#pragma unroll
+        for (int m = 0; m < 5; ++m) {
+            if (td.scale != 1.0) d[m] *= td.scale;
+            sum[m] = fma(lw_weight(k), d[m], sum[m]);
+        }
+        ns_join(d, td.linear * w[1], td.linear * w[2], F, G);
+        // the viscous part of this difference into the wall records
+        wall_stage(P, td.c[0], td.c[1], td.c[2], td.c[3], td.c[4], td.scale, lw_weight(k), td.c[2] != 0.0);
     }
-    // f_tttt of the viscous part (with the 0.5), weight 1/120
-    if constexpr (N == 4) wall_stage(P, -4.0, -4.0, 1.0, 1.0, 6.0, 0.5, 1.0 / 120.0, true);
+    // s0 is read only at the own node since the first contraction: it takes
+    // the total f_tttt for the temporal error
+    if constexpr (N == 4) {
+        if (terr && act) put8<S>(s0, sidx, F, G);
+    }
     // the source's last difference enters S only: s_tttt/120 (kernel 4), s_ttt/24 (kernel 3)
-    if constexpr (N == 4) src_lvl(4, 1.0 / 120.0, nullptr);
-    else src_lvl(3, 1.0 / 24.0, nullptr);
+    src_lvl(N, lw_weight(N), nullptr);
+    // the linear parts of F̃: those of Ũ, up to the factor the last stencil puts on them
+    constexpr double miss = lw_weight(N) * (1.0 - time_diff<N>(N).linear);
+    ns_join(sum, fma(-miss, w[1], Uc[1]), fma(-miss, w[2], Uc[2]), F, G);
     __syncthreads();  // every thread has finished reading s2 before it is reused
     if constexpr (CURV) {
         double Fc[4], Gc[4];
@@ -1972,58 +1896,43 @@ __device__ __forceinline__ void lwp_element(const double* uN, const double* gxN,
     }
 }
 
-// f_t of the states w ± wt, w ± 2wt (and their gradients) for the MDRK stages;
-// WALL: also f_t of components 1..3 of the viscous fluxes in v6 (x, then y),
-// from the same evaluations
+// acc += weight · f_t of the states w ± wt, w ± 2wt (and their gradients) for
+// the MDRK stages (the five ns_q sums; the mass fluxes' part of f_t is ut);
+// WALL: also f_t of components 1..3 of the viscous fluxes in v6 (x, then y)
 template <bool WALL = false>
 __device__ __forceinline__ void mdrkp_ft(const double* u, const double* ut, const double* gx, const double* gtx,
-                                         const double* gy, const double* gty, double gm1, DevC c,
-                                         double* dx, double* dy, double* v6 = nullptr) {
-    const double cq[4] = {2.0, 1.0, -1.0, -2.0};
-    const double wq[4] = {-1.0, 8.0, -8.0, 1.0};
-    double a6[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+                                         const double* gy, const double* gty, double gm1, DevC c, double weight,
+                                         double* acc, double* v6 = nullptr) {
+    constexpr TimeDiff td = time_diff<4>(1);
+    double d[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, a6[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-    for (int v = 0; v < 4; ++v) dx[v] = dy[v] = 0.0;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        double s[4], sx[4], sy[4], fa[4], ga[4];
+    for (int r = 0; r < 4; ++r) {
+        const int k = r == 0 ? 2 : r == 1 ? 0 : r == 2 ? 1 : 3;
+        double s[4], sx[4], sy[4], q[5];
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            s[v] = fma(cq[q], ut[v], u[v]);
-            sx[v] = fma(cq[q], gtx[v], gx[v]);
-            sy[v] = fma(cq[q], gty[v], gy[v]);
+            s[v] = fma(kTaylor[k][0], ut[v], u[v]);
+            sx[v] = fma(kTaylor[k][0], gtx[v], gx[v]);
+            sy[v] = fma(kTaylor[k][0], gty[v], gy[v]);
         }
+        ns_q(s, sx, sy, gm1, c, q);
+#pragma unroll
+        for (int m = 0; m < 5; ++m) d[m] = fma(td.c[k], q[m], d[m]);
         if constexpr (WALL) {
             double fx[4], fy[4];
-            euler_fluxes(s, gm1, fa, ga);
             ns_visc_fluxes(s, sx, sy, gm1, c, fx, fy);
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                fa[v] -= fx[v];
-                ga[v] -= fy[v];
+            for (int m = 0; m < 3; ++m) {
+                a6[m] = fma(td.c[k], fx[1 + m], a6[m]);
+                a6[3 + m] = fma(td.c[k], fy[1 + m], a6[3 + m]);
             }
-#pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                a6[k] = fma(wq[q], fx[1 + k], a6[k]);
-                a6[3 + k] = fma(wq[q], fy[1 + k], a6[3 + k]);
-            }
-        } else {
-            ns_total_fluxes(s, sx, sy, gm1, c, fa, ga);
-        }
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            dx[v] = fma(wq[q], fa[v], dx[v]);
-            dy[v] = fma(wq[q], ga[v], dy[v]);
         }
     }
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        dx[v] *= 1.0 / 12.0;
-        dy[v] *= 1.0 / 12.0;
-    }
+    for (int m = 0; m < 5; ++m) acc[m] = fma(weight * td.scale, d[m], acc[m]);
     if constexpr (WALL) {
 #pragma unroll
-        for (int k = 0; k < 6; ++k) v6[k] = a6[k] * (1.0 / 12.0);
+        for (int m = 0; m < 6; ++m) v6[m] = a6[m] * td.scale;
     }
 }
 
@@ -2072,8 +1981,9 @@ __device__ __forceinline__ void mdrkp1_element(const double* uN, const double* g
                                                double* Ssrc = nullptr) {
     using G_ = VGeo<N, EB>;
     constexpr int n = G_::n, S = G_::S;
-    double f[4], g[4];
-    ns_total_fluxes(uN, gxN, gyN, gm1, c, f, g);
+    double f[4], g[4], q[5];
+    ns_q(uN, gxN, gyN, gm1, c, q);
+    ns_join(q, uN[1], uN[2], f, g);
     if constexpr (WALL) wall_first(wq, 0.5, uN, gxN, gyN, gm1, c);
     double ut[4], utx[4], uty[4];
     if (has_src) {
@@ -2089,20 +1999,18 @@ __device__ __forceinline__ void mdrkp1_element(const double* uN, const double* g
     } else {
         par_level<N, EB, CURV>(act, sidx, sbase, i, j, invJ, sc, s0, s2, sD, f, g, ut, utx, uty, Jn);
     }
-    double dx[4], dy[4];
+#pragma unroll
+    for (int m = 0; m < 5; ++m) q[m] *= 0.5;
     if constexpr (WALL) {
         double v6[6];
-        mdrkp_ft<true>(uN, ut, gxN, utx, gyN, uty, gm1, c, dx, dy, v6);
+        mdrkp_ft<true>(uN, ut, gxN, utx, gyN, uty, gm1, c, 0.125, q, v6);
         wall_acc(wq, 0.125, v6, false);
     } else {
-        mdrkp_ft(uN, ut, gxN, utx, gyN, uty, gm1, c, dx, dy);
+        mdrkp_ft(uN, ut, gxN, utx, gyN, uty, gm1, c, 0.125, q);
     }
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        F[v] = fma(0.125, dx[v], 0.5 * f[v]);
-        G[v] = fma(0.125, dy[v], 0.5 * g[v]);
-        Uc[v] = fma(0.125, ut[v], 0.5 * uN[v]);
-    }
+    for (int v = 0; v < 4; ++v) Uc[v] = fma(0.125, ut[v], 0.5 * uN[v]);
+    ns_join(q, Uc[1], Uc[2], F, G);
     __syncthreads();  // every thread has finished reading s2 before it is reused
     if constexpr (CURV) {
         double Fc[4], Gc[4];
@@ -2134,10 +2042,12 @@ __device__ __forceinline__ void mdrkp2_element(const double* uN, const double* g
                                                double* Ssrc = nullptr) {
     using G_ = VGeo<N, EB>;
     constexpr int n = G_::n, S = G_::S;
-    double f[4], g[4], fs[4], gs[4];
-    ns_total_fluxes(uN, gxN, gyN, gm1, c, f, g);
+    double f[4], g[4], fs[4], gs[4], q[5], qs[5];
+    ns_q(uN, gxN, gyN, gm1, c, q);
+    ns_join(q, uN[1], uN[2], f, g);
     if constexpr (WALL) wall_first(wq, 1.0, uN, gxN, gyN, gm1, c);
-    ns_total_fluxes(usn, gxS, gyS, gm1, c, fs, gs);
+    ns_q(usn, gxS, gyS, gm1, c, qs);
+    ns_join(qs, usn[1], usn[2], fs, gs);
     if constexpr (CURV) {
         double cx[4], cy[4];
         to_contravariant(Jn, f, g, cx, cy);
@@ -2188,33 +2098,19 @@ __device__ __forceinline__ void mdrkp2_element(const double* uN, const double* g
             sty[v] *= invJ;
         }
     }
-    double dx[4], dy[4];
     if constexpr (WALL) {
         double v6[6];
-        mdrkp_ft<true>(uN, ut, gxN, utx, gyN, uty, gm1, c, dx, dy, v6);
+        mdrkp_ft<true>(uN, ut, gxN, utx, gyN, uty, gm1, c, 1.0 / 6.0, q, v6);
         wall_acc(wq, 1.0 / 6.0, v6, false);
-    } else {
-        mdrkp_ft(uN, ut, gxN, utx, gyN, uty, gm1, c, dx, dy);
-    }
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        F[v] = fma(1.0 / 6.0, dx[v], f[v]);
-        G[v] = fma(1.0 / 6.0, dy[v], g[v]);
-        Uc[v] = fma(1.0 / 6.0, ut[v], uN[v]);
-    }
-    if constexpr (WALL) {
-        double v6[6];
-        mdrkp_ft<true>(usn, ust, gxS, stx, gyS, sty, gm1, c, dx, dy, v6);
+        mdrkp_ft<true>(usn, ust, gxS, stx, gyS, sty, gm1, c, 1.0 / 3.0, q, v6);
         wall_acc(wq, 1.0 / 3.0, v6, false);
     } else {
-        mdrkp_ft(usn, ust, gxS, stx, gyS, sty, gm1, c, dx, dy);
+        mdrkp_ft(uN, ut, gxN, utx, gyN, uty, gm1, c, 1.0 / 6.0, q);
+        mdrkp_ft(usn, ust, gxS, stx, gyS, sty, gm1, c, 1.0 / 3.0, q);
     }
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        F[v] = fma(1.0 / 3.0, dx[v], F[v]);
-        G[v] = fma(1.0 / 3.0, dy[v], G[v]);
-        Uc[v] = fma(1.0 / 3.0, ust[v], Uc[v]);
-    }
+    for (int v = 0; v < 4; ++v) Uc[v] = fma(1.0 / 3.0, ust[v], fma(1.0 / 6.0, ut[v], uN[v]));
+    ns_join(q, Uc[1], Uc[2], F, G);
     __syncthreads();  // every thread has finished reading s2 before it is reused
     if constexpr (CURV) {
         double Fc[4], Gc[4];
