@@ -767,10 +767,8 @@ template <int n> __device__ __forceinline__ void op_row(const double* M, int i, 
 // with f and g of every node of the workgroup in s (put8) and M (n x n, rows
 // of op_stride(n)) in LDS.
 template <int n, int S>
-__device__ __forceinline__ void contract(const double* s, int base, int i, int j, const double* M, double* out) {
-    double Di[n], Dj[n];
-    op_row<n>(M, i, Di);
-    op_row<n>(M, j, Dj);
+__device__ __forceinline__ void contract_rows(const double* s, int base, int i, int j, const double* Di,
+                                              const double* Dj, double* out) {
     const double2* p = reinterpret_cast<const double2*>(s);
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
@@ -796,6 +794,14 @@ __device__ __forceinline__ void load4(const double* p, double* u) {
     const double2* p2 = reinterpret_cast<const double2*>(p);
     const double2 a = p2[0], b = p2[1];
     u[0] = a.x; u[1] = a.y; u[2] = b.x; u[3] = b.y;
+}
+
+template <int n, int S>
+__device__ __forceinline__ void contract(const double* s, int base, int i, int j, const double* M, double* out) {
+    double Di[n], Dj[n];
+    op_row<n>(M, i, Di);
+    op_row<n>(M, j, Dj);
+    contract_rows<n, S>(s, base, i, j, Di, Dj, out);
 }
 
 // Boundary state of face node l of element e's face at GLL time level q (q = n:
@@ -1177,7 +1183,7 @@ __device__ __forceinline__ void put_fluxes(double* s, int sidx, bool act, const 
 // feed the face records.  The last exchange is in A (N = 4) or B (N = 3).
 // Bound by FP64 issue with the LDS contractions beside it: per node and level
 // four euler_q with five sums each (22 issue slots + 4 for the estimate of 1/ρ),
-// 26 LDS loads and 4 stores.  LW N=4 1024², 10 elements per workgroup: whole
+// 20 LDS loads and 4 stores.  LW N=4 1024², 10 elements per workgroup: whole
 // flux vectors, three buffers and plain loads of the constants 1283 us, this form
 // with the early loads of volume_body 1138 us.
 // With KEEP, tder receives the time derivatives ut, utt, ... (4 per order),
@@ -1203,6 +1209,7 @@ __device__ __forceinline__ void lw_element(const double* uN, const double* J, do
     constexpr int n = G_::n, S = G_::S;
     const double gm1 = gamma - 1.0, kh = -0.5 * gm1;
     double q0[5], sum[5], st[4][4], w[4], sk[4] = {0.0, 0.0, 0.0, 0.0};
+    double Di[n], Dj[n];
     euler_q(uN, gamma, kh, q0);
     euler_join(q0, uN[1], uN[2], uN[3], gm1, kh, F, G);
 #pragma unroll
@@ -1213,7 +1220,11 @@ __device__ __forceinline__ void lw_element(const double* uN, const double* J, do
         double* buf = (k & 1) ? A : B;
         put_fluxes<S, CURV>(buf, sidx, act, J, F, G);
         __syncthreads();
-        contract<n, S>(buf, sbase, i, j, sD, w);
+        if (k == 1) {  // read once: 20 LDS loads a level instead of 26 (1.3% of a step at 1024², N=4)
+            op_row<n>(sD, i, Di);
+            op_row<n>(sD, j, Dj);
+        }
+        contract_rows<n, S>(buf, sbase, i, j, Di, Dj, w);
         if constexpr (SRC) src_level_c(*sp, dt, k - 1, CURV && N == 4, sk, Ssrc, lw_weight(k - 1));
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
@@ -1905,26 +1916,29 @@ __device__ __forceinline__ void mdrkp_ft(const double* u, const double* ut, cons
                                          double* acc, double* v6 = nullptr) {
     constexpr TimeDiff td = time_diff<4>(1);
     double d[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, a6[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-#pragma unroll
+    constexpr int kUnroll = WALL ? 1 : 4;  // the wall kernels spill the interleaved states
+#pragma unroll kUnroll
     for (int r = 0; r < 4; ++r) {
-        const int k = r == 0 ? 2 : r == 1 ? 0 : r == 2 ? 1 : 3;
+        // the states u + 2ut, u + ut, u - ut, u - 2ut (selects, as the loop may stay one)
+        const double off = r == 0 ? 2.0 : r == 1 ? 1.0 : r == 2 ? -1.0 : -2.0;
+        const double ck = r == 0 ? td.c[2] : r == 1 ? td.c[0] : r == 2 ? td.c[1] : td.c[3];
         double s[4], sx[4], sy[4], q[5];
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            s[v] = fma(kTaylor[k][0], ut[v], u[v]);
-            sx[v] = fma(kTaylor[k][0], gtx[v], gx[v]);
-            sy[v] = fma(kTaylor[k][0], gty[v], gy[v]);
+            s[v] = fma(off, ut[v], u[v]);
+            sx[v] = fma(off, gtx[v], gx[v]);
+            sy[v] = fma(off, gty[v], gy[v]);
         }
         ns_q(s, sx, sy, gm1, c, q);
 #pragma unroll
-        for (int m = 0; m < 5; ++m) d[m] = fma(td.c[k], q[m], d[m]);
+        for (int m = 0; m < 5; ++m) d[m] = fma(ck, q[m], d[m]);
         if constexpr (WALL) {
             double fx[4], fy[4];
             ns_visc_fluxes(s, sx, sy, gm1, c, fx, fy);
 #pragma unroll
             for (int m = 0; m < 3; ++m) {
-                a6[m] = fma(td.c[k], fx[1 + m], a6[m]);
-                a6[3 + m] = fma(td.c[k], fy[1 + m], a6[3 + m]);
+                a6[m] = fma(ck, fx[1 + m], a6[m]);
+                a6[3 + m] = fma(ck, fy[1 + m], a6[3 + m]);
             }
         }
     }
