@@ -2533,9 +2533,10 @@ __device__ __forceinline__ void volume_tile(const KArgs& a, int bid, const int4&
     if (act) store4(out + off, val);
     if constexpr (KB == VOL_LW_ADAPT) {
         if (a.reduce != RED_ADAPT) return;
-        // the workgroup's sum of its elements' temporal errors (adaptive.jl:48-64)
-        double* se = lds;
-        double* rs = lds + S;
+        // the workgroup's sum of its elements' temporal errors (adaptive.jl:48-64), in
+        // the records' place: the interface fluxes may still be read by other lanes
+        double* se = rec;
+        double* rs = se + S;
         double* es = rs + EB * n;
         if (act) se[sidx] = terr;
         __syncthreads();
