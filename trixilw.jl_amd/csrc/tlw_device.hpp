@@ -839,6 +839,28 @@ template <int RQ = kTraceQ> __device__ __forceinline__ void store_record(double*
     for (int k = 0; k < RQ / 2; ++k) p2[k] = make_double2(r[2 * k], r[2 * k + 1]);
 }
 
+// Pair p of variables of face record `slot` in LDS.  The shock-capturing records
+// are 128 bytes apart, half a cycle of the banks: their pairs are permuted by the
+// slot, so that neighbouring lanes reading one pair meet different banks.
+template <int RQ> __device__ __forceinline__ double2* rec_pair(double* rec, int slot, int p) {
+    double2* q = reinterpret_cast<double2*>(rec + slot * RQ);
+    return q + (RQ == kTraceQSC ? (p ^ ((slot >> 1) & 7)) : p);
+}
+template <int RQ> __device__ __forceinline__ void get_record(double* rec, int slot, double* r) {
+#pragma unroll
+    for (int k = 0; k < RQ / 2; ++k) {
+        const double2 x = *rec_pair<RQ>(rec, slot, k);
+        r[2 * k] = x.x;
+        r[2 * k + 1] = x.y;
+    }
+}
+// pairs [first, last) of the record
+template <int RQ, int first = 0, int last = RQ / 2>
+__device__ __forceinline__ void put_record(double* rec, int slot, const double* r) {
+#pragma unroll
+    for (int k = first; k < last; ++k) *rec_pair<RQ>(rec, slot, k) = make_double2(r[2 * k], r[2 * k + 1]);
+}
+
 // Buffer selection by integer arithmetic on the loaded pointers: a select
 // between fields of the argument struct would be folded into a load from a
 // computed offset, which moves the whole struct to private memory.
@@ -2157,13 +2179,17 @@ __device__ __forceinline__ void curved_speeds(const double* u, const double* J, 
 // reduction here costs barriers and LDS passes worth 15% of this kernel).
 // Waves per SIMD the register budget is sized for: 3 (168 VGPRs) for the
 // plain scheme (TLW_VOL_WAVES at build time); 2 (256 VGPRs) with shock
-// capturing, whose subcell FV and blended face fluxes would otherwise spill,
-// and with source terms (the source's time differences at every stage).
+// capturing, which takes 157 on a TreeMesh (and so runs 3 waves all the same)
+// but 172 on a curvilinear mesh, and with source terms (the source's time
+// differences at every stage).
 #ifndef TLW_VOL_WAVES
 #define TLW_VOL_WAVES 3
 #endif
 template <bool TWO> constexpr int kVolWaves = TWO ? 2 : TLW_VOL_WAVES;
 template <bool SC, bool PAR> constexpr bool vol_two_buffers = !SC && !PAR;
+
+// pure_and_blended_element_ids!: an element without subcell FV
+__device__ __forceinline__ bool pure_dg(double alpha) { return fabs(alpha) <= 1e-12; }
 
 // What a lane of a volume workgroup reads of its tile before the element procedure.
 template <bool CURV, bool US> struct TileIn {
@@ -2178,8 +2204,8 @@ template <bool CURV, bool US> struct TileIn {
 // PAR: hyperbolic-parabolic (compressible Navier-Stokes) element procedures,
 // same register budget as shock capturing.
 // One tile (blk) of a's table, number bid, with its LDS: lds [G_::LDS2 or LDS],
-// sDh and sD [G_::M] (D̂ and D, rows of G_::MS) and s_alpha [EB] (smoothed
-// blending factors of the curvilinear interfaces).
+// sDh and sD [G_::M] (D̂ and D, rows of G_::MS) and s_alpha [EB + 1] (smoothed
+// blending factors, and whether any of them blends).
 template <int N, int EB, int KIND, bool SC, bool PAR, bool CURV>
 __device__ __forceinline__ void volume_tile(const KArgs& a, int bid, const int4& blk,
                                             const TileIn<CURV, vol_base(KIND) == VOL_MDRK2>& in, double* lds,
@@ -2193,8 +2219,9 @@ __device__ __forceinline__ void volume_tile(const KArgs& a, int bid, const int4&
     constexpr int n = G_::n, NN = G_::NN, S = G_::S, NT = G_::NT;
     // The plain Euler kernels exchange through two buffers: F̃ last in the first of
     // them, where the interface fluxes go later, and the face records in the
-    // second.  Shock capturing and the Navier-Stokes kernels use three: s2 takes
-    // F̃ and the interface fluxes, s0 and s1 the records.
+    // second.  Shock capturing and the Navier-Stokes kernels use three: s2 takes F̃;
+    // then s0 and s1 the records and s2 the interface fluxes, or with shock capturing
+    // s1 and s2 the records and s0, which holds uⁿ before, the fluxes.
     constexpr bool TWO = vol_two_buffers<SC, PAR>;
     double* s0 = lds;
     double* s1 = lds + 8 * S;
@@ -2207,6 +2234,30 @@ __device__ __forceinline__ void volume_tile(const KArgs& a, int bid, const int4&
     const DevS st = dev_state(a.st + blk.z);
     if (a.use_state_dt && st->finished) return;
     const int tid = threadIdx.x;
+    if constexpr (SC) {
+        // the tile's blending factors, smoothed over the face neighbours (Trixi
+        // apply_smoothing!), by one lane an element of the first wave: read early,
+        // and published by the first barrier of the element procedure
+        static_assert(EB < 64, "one wave's lanes");
+        if (tid < 64) {
+            double al = 0.0;
+            if (tid < blk.y) {
+                const int es = blk.x + tid;
+                al = a.alpha_tmp[es];
+                if (dev_const(a.c)->alpha_smooth) {
+                    const int4 nb = *reinterpret_cast<const int4*>(a.nbr + 4 * es);
+                    if (nb.x >= 0) al = dmax(al, 0.5 * a.alpha_tmp[nb.x]);
+                    if (nb.y >= 0) al = dmax(al, 0.5 * a.alpha_tmp[nb.y]);
+                    if (nb.z >= 0) al = dmax(al, 0.5 * a.alpha_tmp[nb.z]);
+                    if (nb.w >= 0) al = dmax(al, 0.5 * a.alpha_tmp[nb.w]);
+                }
+                s_alpha[tid] = al;
+                if (a.alpha_out) a.alpha_out[es] = al;
+            }
+            const bool any = __any(!pure_dg(al));
+            if (tid == 0) s_alpha[EB] = any ? 1.0 : 0.0;
+        }
+    }
     const int le = tid / NN, node = tid - (tid / NN) * NN;
     const int i = node % n, j = node / n;
     const int e0 = blk.x;
@@ -2320,86 +2371,121 @@ __device__ __forceinline__ void volume_tile(const KArgs& a, int bid, const int4&
     constexpr int RQ = kRQ<SC>;
     double fnlx[4] = {0, 0, 0, 0}, fnly[4] = {0, 0, 0, 0};
     double alpha_e = 0.0;
+    bool subcells = false;  // the workgroup has a blended element
     if constexpr (SC) {
-        // blending factor, smoothed over the face neighbours (Trixi apply_smoothing!)
-        alpha_e = a.alpha_tmp[e];
-        if (c->alpha_smooth) {
+        // Away from shocks a workgroup has no blended element, and what is left of
+        // the subcell FV is one Rusanov flux a face node (below) in place of two a
+        // node and two barriers fewer.  256², N=4, tile 10, one workgroup in ten
+        // blended: 168 us (234 VGPRs) with the subcell FV of every element and the
+        // blending factors read here, now 130 (157 VGPRs).
+        alpha_e = s_alpha[lec];
+        subcells = __builtin_amdgcn_readfirstlane(s_alpha[EB] != 0.0);
+        if (subcells) {
+            const bool blended = !pure_dg(alpha_e);
+            // subcell FV (fv_kernel!, dg_2d.jl:251-324): Rusanov fluxes between the
+            // face values of neighbouring subcells, zero at the element faces.  First
+            // order (Trixi calcflux_fv!): the face values are the node values.  A
+            // blended element away from the domain boundary with MUSCL-Hancock takes
+            // the reconstructed, half-step-evolved face values (mh_faces).
+            if (act) put4<S>(s1, sidx, uN);
+            __syncthreads();
+            double ql[4], qr[4], qd[4], qu[4];
 #pragma unroll
-            for (int f = 0; f < 4; ++f) {
-                const int nb = a.nbr[4 * e + f];
-                if (nb >= 0) alpha_e = dmax(alpha_e, 0.5 * a.alpha_tmp[nb]);
+            for (int v = 0; v < 4; ++v) ql[v] = qr[v] = qd[v] = qu[v] = uN[v];
+            if (!CURV && c->recon == 1 && blended && a.nbr[4 * e] >= 0 && a.nbr[4 * e + 1] >= 0 && a.nbr[4 * e + 2] >= 0 &&
+                a.nbr[4 * e + 3] >= 0) {
+                const double dtmh = (KIND == VOL_MDRK1) ? 0.5 * dt : dt;  // tree/multi_derivative_2d.jl:199
+                mh_faces<N, S>(s1, sidx, i, j, uN, c, 2.0 - alpha_e, dtmh, invJ, gm1, ql, qr, qd, qu);
             }
-        }
-        if (act && node == 0 && a.alpha_out) a.alpha_out[e] = alpha_e;
-        if constexpr (CURV) {
-            if (act && node == 0) s_alpha[lec] = alpha_e;
-        }
-        // subcell FV (fv_kernel!, dg_2d.jl:251-324): Rusanov fluxes between the
-        // face values of neighbouring subcells, zero at the element faces.  First
-        // order (Trixi calcflux_fv!): the face values are the node values.  A
-        // blended element away from the domain boundary with MUSCL-Hancock takes
-        // the reconstructed, half-step-evolved face values (mh_faces).
-        if (act) put4<S>(s1, sidx, uN);
-        __syncthreads();
-        const bool blended = !(fabs(alpha_e) <= 1e-12);  // pure_and_blended_element_ids!
-        double ql[4], qr[4], qd[4], qu[4];
+            // the right and upper face values go to the neighbouring subcells
+            if (act) put8<S>(s0, sidx, qr, qu);
+            __syncthreads();
+            double fxl[4] = {0, 0, 0, 0}, gyl[4] = {0, 0, 0, 0}, w[4];
+            if (i > 0) {
+                get4<S>(s0, sidx - 1, w);
+                if constexpr (CURV) {
+                    // Trixi's subcell normal, or for a pure-DG element at subcell face n-1 the
+                    // normal of the reference's calc_fn_low! (structured/dg_2d.jl:111-173)
+                    const double* nq = (!blended && i == n - 1) ? a.sqrk + ((size_t)e * n + j) * 4
+                                                                 : a.snrm + ((size_t)e * NN + node) * 4;
+                    rusanov_normal(w, ql, gamma, nq[0], nq[1], sqrt(fma(nq[0], nq[0], nq[1] * nq[1])), fxl);
+                } else {
+                    rusanov(w, ql, gamma, 1, fxl);
+                }
+            }
+            if (j > 0) {
+                get4<S>(s0 + 4 * S, sidx - n, w);
+                if constexpr (CURV) {
+                    const double* nq = (!blended && j == n - 1) ? a.sqrk + ((size_t)e * n + i) * 4 + 2
+                                                                 : a.snrm + ((size_t)e * NN + node) * 4 + 2;
+                    rusanov_normal(w, qd, gamma, nq[0], nq[1], sqrt(fma(nq[0], nq[0], nq[1] * nq[1])), gyl);
+                } else {
+                    rusanov(w, qd, gamma, 2, gyl);
+                }
+            }
+            if (act) put8<S>(s2, sidx, fxl, gyl);
+            __syncthreads();
+            const double iwi = 1.0 / c->weights[i], iwj = 1.0 / c->weights[j];
+            double fxr4[4] = {0.0, 0.0, 0.0, 0.0}, gyr4[4] = {0.0, 0.0, 0.0, 0.0};
+            if (i < n - 1) get4<S>(s2, sidx + 1, fxr4);
+            if (j < n - 1) get4<S>(s2 + 4 * S, sidx + n, gyr4);
 #pragma unroll
-        for (int v = 0; v < 4; ++v) ql[v] = qr[v] = qd[v] = qu[v] = uN[v];
-        if (!CURV && c->recon == 1 && blended && a.nbr[4 * e] >= 0 && a.nbr[4 * e + 1] >= 0 && a.nbr[4 * e + 2] >= 0 &&
-            a.nbr[4 * e + 3] >= 0) {
-            const double dtmh = (KIND == VOL_MDRK1) ? 0.5 * dt : dt;  // tree/multi_derivative_2d.jl:199
-            mh_faces<N, S>(s1, sidx, i, j, uN, c, 2.0 - alpha_e, dtmh, invJ, gm1, ql, qr, qd, qu);
-        }
-        // the right and upper face values go to the neighbouring subcells
-        if (act) put8<S>(s0, sidx, qr, qu);
-        __syncthreads();
-        double fxl[4] = {0, 0, 0, 0}, gyl[4] = {0, 0, 0, 0}, w[4];
-        if (i > 0) {
-            get4<S>(s0, sidx - 1, w);
-            if constexpr (CURV) {
-                // Trixi's subcell normal, or for a pure-DG element at subcell face n-1 the
-                // normal of the reference's calc_fn_low! (structured/dg_2d.jl:111-173)
-                const double* nq = (!blended && i == n - 1) ? a.sqrk + ((size_t)e * n + j) * 4
-                                                             : a.snrm + ((size_t)e * NN + node) * 4;
-                rusanov_normal(w, ql, gamma, nq[0], nq[1], sqrt(fma(nq[0], nq[0], nq[1] * nq[1])), fxl);
-            } else {
-                rusanov(w, ql, gamma, 1, fxl);
+            for (int v = 0; v < 4; ++v) {
+                const double fxr = fxr4[v], gyr = gyr4[v];
+                const double fv = iwi * (fxr - fxl[v]) + iwj * (gyr - gyl[v]);
+                vol[v] = (1.0 - alpha_e) * vol[v] + (blended ? alpha_e * fv : 0.0);
+                // fn_low: the subcell fluxes next to the element faces (load_fn_low!)
+                fnlx[v] = (fx == 0) ? fxr : fxl[v];
+                fnly[v] = (fy == 2) ? gyr : gyl[v];
             }
-        }
-        if (j > 0) {
-            get4<S>(s0 + 4 * S, sidx - n, w);
-            if constexpr (CURV) {
-                const double* nq = (!blended && j == n - 1) ? a.sqrk + ((size_t)e * n + i) * 4 + 2
-                                                             : a.snrm + ((size_t)e * NN + node) * 4 + 2;
-                rusanov_normal(w, qd, gamma, nq[0], nq[1], sqrt(fma(nq[0], nq[0], nq[1] * nq[1])), gyl);
-            } else {
-                rusanov(w, qd, gamma, 2, gyl);
-            }
-        }
-        if (act) put8<S>(s2, sidx, fxl, gyl);
-        __syncthreads();
-        const double iwi = 1.0 / c->weights[i], iwj = 1.0 / c->weights[j];
-        double fxr4[4] = {0.0, 0.0, 0.0, 0.0}, gyr4[4] = {0.0, 0.0, 0.0, 0.0};
-        if (i < n - 1) get4<S>(s2, sidx + 1, fxr4);
-        if (j < n - 1) get4<S>(s2 + 4 * S, sidx + n, gyr4);
+            __syncthreads();  // s1 and s2 are reused for the face records
+        } else {
+            if (act) put4<S>(s0, sidx, uN);
+            __syncthreads();
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const double fxr = fxr4[v], gyr = gyr4[v];
-            const double fv = iwi * (fxr - fxl[v]) + iwj * (gyr - gyl[v]);
-            vol[v] = (1.0 - alpha_e) * vol[v] + (blended ? alpha_e * fv : 0.0);
-            // fn_low: the subcell fluxes next to the element faces (load_fn_low!)
-            fnlx[v] = (fx == 0) ? fxr : fxl[v];
-            fnly[v] = (fy == 2) ? gyr : gyl[v];
+            for (int v = 0; v < 4; ++v) vol[v] = (1.0 - alpha_e) * vol[v];
         }
-        __syncthreads();  // s0, s1 and s2 are reused for the face records and interface sums
     }
     // --- face records into LDS (s0, s1 are free), one per face the node lies on.
     // λ ingredients: |v1|, |v2| and c of the λ state, once per node.
-    double* rec = TWO ? s1 : lds;  // [EB][4][n][RQ]
+    double* rec = (TWO || SC) ? s1 : lds;  // [EB][4][n][RQ]
     const bool tree = c->flux_order == 0;
     const double* jump = tree ? uN : Uc;
     const double* lamst = tree ? Uc : uN;
     const int nbx = in.nbx, nby = in.nby;
+    constexpr int NSLOT = EB * 4 * n;
+    static_assert(NSLOT <= NT, "one face slot per lane");
+    constexpr int FN = CURV ? 12 : 10;  // fn_low in a record: variables [FN, FN + 4)
+    auto put_face = [&](int f, int l, const double* r) {
+        const int slot = (lec * 4 + f) * n + l;
+        if constexpr (SC) {
+            put_record<RQ, 0, FN / 2>(rec, slot, r);
+            if (subcells) put_record<RQ, FN / 2, FN / 2 + 2>(rec, slot, r);
+            put_record<RQ, FN / 2 + 2>(rec, slot, r);
+        } else {
+            put_record<RQ>(rec, slot, r);
+        }
+    };
+    if constexpr (SC) {
+        // without a blended element only fn_low is left of the subcell FV: the flux
+        // between the face's node and the next one inwards, by the lane of the slot
+        if (!subcells && tid < NSLOT && tid / (4 * n) < nel) {
+            const int ls = tid / (4 * n), f = (tid / n) % 4, l = tid % n;
+            const int k = (f & 1) ? n - 1 : 1;  // upper node of the two, along the face's direction
+            const int hi = (f < 2) ? l * n + k : k * n + l;
+            double ul[4], ur[4], r[RQ];
+            get4<S>(s0, ls * NN + hi - (f < 2 ? 1 : n), ul);
+            get4<S>(s0, ls * NN + hi, ur);
+            if constexpr (CURV) {
+                const size_t es = e0 + ls;
+                const double* nq = ((f & 1) ? a.sqrk + (es * n + l) * 4 : a.snrm + (es * NN + hi) * 4) + (f < 2 ? 0 : 2);
+                rusanov_normal(ul, ur, gamma, nq[0], nq[1], sqrt(fma(nq[0], nq[0], nq[1] * nq[1])), r + FN);
+            } else {
+                rusanov(ul, ur, gamma, f < 2 ? 1 : 2, r + FN);
+            }
+            put_record<RQ, FN / 2, FN / 2 + 2>(rec, tid, r);
+        }
+    }
     if constexpr (CURV) {
         // structured order with the interface's normal n (shared by both
         // elements): F̃·n, |v(uⁿ)·n| and c(uⁿ)|n| (dg_2d.jl:2229-2264)
@@ -2426,7 +2512,7 @@ __device__ __forceinline__ void volume_tile(const KArgs& a, int bid, const int4&
             } else {
                 make_record(r, Uc, Fn, fabs(fma(v1, nf[0], v2 * nf[1])), cs * nf[2]);
             }
-            store_record<RQ>(rec + ((lec * 4 + f) * n + l) * RQ, r);
+            put_face(f, l, r);
         };
         if (act && fx >= 0) face(fx, j, fnlx);
         if (act && fy >= 0) face(fy, i, fnly);
@@ -2445,14 +2531,14 @@ __device__ __forceinline__ void volume_tile(const KArgs& a, int bid, const int4&
             double r[RQ];
             make_record(r, jump, F, av1, cs);
             fill(r, fnlx);
-            store_record<RQ>(rec + ((lec * 4 + fx) * n + j) * RQ, r);
+            put_face(fx, j, r);
             if (nbx <= -2) mortar_side(a, nbx, n, j, jump, F, lamst);
         }
         if (act && fy >= 0) {
             double r[RQ];
             make_record(r, jump, G, av2, cs);
             fill(r, fnly);
-            store_record<RQ>(rec + ((lec * 4 + fy) * n + i) * RQ, r);
+            put_face(fy, i, r);
             if (nby <= -2) mortar_side(a, nby, n, i, jump, G, lamst);
         }
     }
@@ -2461,25 +2547,22 @@ __device__ __forceinline__ void volume_tile(const KArgs& a, int bid, const int4&
     // workgroup is evaluated once, by the slot of its left element's + face, and
     // its flux goes to both adjacent nodes (accx for x faces, accy for y faces);
     // the record of a face leaving the workgroup goes to HBM for the surface kernel.
-    double* accx = s2;  // pairs of variables (put4); s2 is free after the last contraction
+    double* accx = SC ? s0 : s2;  // pairs of variables (put4); free after the last contraction
     double* accy = accx + 4 * S;
-    constexpr int NSLOT = EB * 4 * n;
-    static_assert(NSLOT <= NT, "one face slot per lane");
-    static_assert(TWO || EB * 4 * n * RQ <= 16 * S, "records fit in s0 and s1");
+    static_assert(TWO || EB * 4 * n * RQ <= 16 * S, "records fit in two buffers");
     if (tid < NSLOT) {
         const int ls = tid / (4 * n), f = (tid / n) % 4, l = tid % n;
         if (ls < nel) {
             const int es = e0 + ls;
             const int ne = in.slot;
-            const double* own = rec + tid * RQ;
             if (!(ne >= e0 && ne < e0 + nel)) {
                 double r[RQ];
-                load_record<RQ>(own, r);
+                get_record<RQ>(rec, tid, r);
                 store_record<RQ>(a.trace + ((size_t)es * 4 * n + f * n + l) * RQ, r);
             } else if (f & 1) {
                 double Lr[RQ], Rr[RQ], Fs[4];
-                load_record<RQ>(own, Lr);
-                load_record<RQ>(rec + (((ne - e0) * 4 + (f ^ 1)) * n + l) * RQ, Rr);
+                get_record<RQ>(rec, tid, Lr);
+                get_record<RQ>(rec, ((ne - e0) * 4 + (f ^ 1)) * n + l, Rr);
                 // + face of ls: node (n-1, l) or (l, n-1); - face of ne: node (0, l) or (l, 0)
                 const int nodeL = (f == 1) ? l * n + (n - 1) : (n - 1) * n + l;
                 const int nodeR = (f == 1) ? l * n : l;
@@ -2611,7 +2694,7 @@ __global__ __launch_bounds__((VGeo<N, EB>::NT), (kVolWavesOf<KIND, SC, PAR>)) vo
     using G_ = VGeo<N, EB>;
     __shared__ alignas(16) double lds[vol_two_buffers<SC, PAR> ? G_::LDS2 : G_::LDS];
     __shared__ alignas(16) double sDh[G_::M], sD[G_::M];
-    __shared__ double s_alpha[(SC && CURV) ? EB : 1];
+    __shared__ double s_alpha[SC ? EB + 1 : 1];
     volume_body<N, EB, KIND, SC, PAR, CURV>(a, blockIdx.x, lds, sDh, sD, s_alpha);
 }
 
