@@ -811,16 +811,20 @@ void launch_volume(tlw_ctx* c, const KArgs& a, int kind) {
     if (c->N == 4) launch_volume_t<4>(c, a, kind);
     else launch_volume_t<3>(c, a, kind);
 }
-FinArgs fin_args(tlw_ctx* c, int reduce, int use_vol) {
-    return FinArgs{c->d_state, c->d_partial, c->d_rng, use_vol, reduce, c->pv_off, c->d_partial + c->slot_off,
+FinArgs fin_args(tlw_ctx* c, int reduce) {
+    return FinArgs{c->d_state, c->d_partial, c->d_rng, reduce, c->pv_off, c->d_partial + c->slot_off,
                    DtLog{c->d_dtlog, c->dtlog_cap, c->d_dtpresc, c->dtpresc_n}};
 }
-void launch_finalize(tlw_ctx* c, int reduce, int use_vol) {
-    const FinArgs f = fin_args(c, reduce, use_vol);
-    if (c->N == 4)
-        hipLaunchKernelGGL(k_finalize<4>, dim3(c->ninst), dim3(kFinalizeBlock), 0, c->stream, f);
+template <int N> void launch_finalize_t(tlw_ctx* c, int reduce) {
+    if (reduce == RED_ADAPT)
+        hipLaunchKernelGGL(k_finalize_adaptive<N>, dim3(c->ninst), dim3(kFinalizeBlock), 0, c->stream,
+                           fin_args(c, reduce));
     else
-        hipLaunchKernelGGL(k_finalize<3>, dim3(c->ninst), dim3(kFinalizeBlock), 0, c->stream, f);
+        hipLaunchKernelGGL(k_finalize<N>, dim3(c->ninst), dim3(kFinalizeWave), 0, c->stream, fin_args(c, reduce));
+}
+void launch_finalize(tlw_ctx* c, int reduce) {
+    if (c->N == 4) launch_finalize_t<4>(c, reduce);
+    else launch_finalize_t<3>(c, reduce);
 }
 template <int N> void launch_surface_t(tlw_ctx* c, const KArgs& a) {
     if (c->curved && c->has_boundary && a.in_sel == SEL_EXPLICIT && !a.u) {
@@ -862,7 +866,7 @@ template <int N> void launch_surface_t(tlw_ctx* c, const KArgs& a) {
     launch(false, nb, c->sgrid - nb);
     // the step's CFL partials come from the surface kernel alone; with adaptive
     // steps the volume kernel's temporal-error sums are read by the finalize kernel
-    if (a.reduce != RED_NONE) launch_finalize(c, a.reduce == RED_ADAPT ? RED_STEP : a.reduce, 0);
+    if (a.reduce != RED_NONE) launch_finalize(c, a.reduce);
 }
 void launch_surface(tlw_ctx* c, const KArgs& a) {
     if (c->N == 4) launch_surface_t<4>(c, a);
@@ -871,12 +875,12 @@ void launch_surface(tlw_ctx* c, const KArgs& a) {
 void launch_limiter(tlw_ctx* c, const KArgs& a) {
     if (c->N == 4) hipLaunchKernelGGL(k_limiter<4>, dim3(c->sgrid), dim3(kSurfBlock), 0, c->stream, a);
     else hipLaunchKernelGGL(k_limiter<3>, dim3(c->sgrid), dim3(kSurfBlock), 0, c->stream, a);
-    if (a.reduce != RED_NONE) launch_finalize(c, a.reduce, 0);
+    if (a.reduce != RED_NONE) launch_finalize(c, a.reduce);
 }
 void launch_max_speed(tlw_ctx* c, const KArgs& a) {
     if (c->N == 4) hipLaunchKernelGGL(k_max_speed<4>, dim3(c->sgrid), dim3(kSurfBlock), 0, c->stream, a);
     else hipLaunchKernelGGL(k_max_speed<3>, dim3(c->sgrid), dim3(kSurfBlock), 0, c->stream, a);
-    launch_finalize(c, a.reduce, 0);
+    launch_finalize(c, a.reduce);
 }
 
 int check_launch(tlw_ctx* c) {
@@ -1913,8 +1917,8 @@ void enqueue_pair_step(tlw_ensemble* e) {
                            c3->vgrid);
     hipLaunchKernelGGL(k_surface_pair, dim3(c3->sgrid + c4->sgrid), dim3(kSurfBlock), 0, e->stream, a3, a4,
                        c3->sgrid);
-    hipLaunchKernelGGL(k_finalize_pair, dim3(c3->ninst + c4->ninst), dim3(kFinalizeBlock), 0, e->stream,
-                       fin_args(c3, RED_STEP, 0), fin_args(c4, RED_STEP, 0), c3->ninst);
+    hipLaunchKernelGGL(k_finalize_pair, dim3(c3->ninst + c4->ninst), dim3(kFinalizeWave), 0, e->stream,
+                       fin_args(c3, RED_STEP), fin_args(c4, RED_STEP), c3->ninst);
 }
 
 }  // namespace

@@ -3378,12 +3378,8 @@ __device__ inline void adaptive_control(DevState* st, double total, double k) {
     st->finished = julia_isapprox(t1, tf);
 }
 
-// Final reduction of the per-workgroup partial maxima of J⁻¹(max λ1 + max λ2),
-// one workgroup per instance over that instance's partials (rng[inst] = volume
-// begin/end, surface begin/end; the volume range is skipped when use_vol is 0),
-// then compute_dt / set_dt! / set_t_and_iter! / isfinished on the instance's
-// state (lwfr.jl:76-103, 146-148, 176-190; Trixi max_dt).
-constexpr int kFinalizeBlock = 1024;
+constexpr int kFinalizeBlock = 1024;  // adaptive steps
+constexpr int kFinalizeWave = 64;
 // Per-step dt record and prescription of a single-instance device loop: the dt
 // of step k (k = the iteration count since the last solve_init) is written to
 // log[k] while k < log_cap, and taken from presc[k] instead of cfl · max_dt
@@ -3394,95 +3390,102 @@ struct DtLog {
     const double* presc;
     long long presc_n;
 };
-// With pv_off > 0 the viscous maxima (pv_off entries further on) give the
-// parabolic bound 1/((λa + λv)·2(2N+1)), λv = 2(2N+1)·max J⁻² max(4μ/(3ρ), μκ/(ρPr)),
-// and max_dt is the smaller of the two (compute_dt for
-// SemidiscretizationHyperbolicParabolic, lwfr.jl:192-210).
-// The arguments of one context's finalize launch.
+// The arguments of one context's finalize launch; reduce is RED_QUERY, RED_INIT or
+// RED_STEP, pv_off > 0 with parabolic terms.
 struct FinArgs {
     DevState* st_all;
     const double* partial;
     const int4* rng;
-    int use_vol, reduce, pv_off;
+    int reduce, pv_off;
     double* slots;
     DtLog dl;
 };
 
-// Instance `bid` of the context, with LDS s, sv [kFinalizeBlock].
+// The end of an adaptive step, one workgroup per instance: the sum of the volume
+// workgroups' temporal-error partials (rng[inst].x to .y), then the controller.
 template <int N>
-__device__ __forceinline__ void finalize_body(const FinArgs& f, int bid, double* s, double* sv) {
-    constexpr int n = N + 1;
+__global__ __launch_bounds__(kFinalizeBlock) void k_finalize_adaptive(FinArgs f) {
+    __shared__ double s[kFinalizeBlock];
     const double* partial = f.partial;
-    const int reduce = f.reduce, pv_off = f.pv_off;
-    double* slots = f.slots;
-    const DtLog& dl = f.dl;
-    DevState* st = f.st_all + bid;
-    const int4 r = f.rng[bid];
-    if (reduce == RED_STEP && st->finished) return;
-    if (reduce == RED_STEP && st->adaptive) {
-        // sum of the volume workgroups' temporal-error partials, then the controller
-        double m[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-        int k = r.x + (int)threadIdx.x;
-        for (; k + 7 * kFinalizeBlock < r.y; k += 8 * kFinalizeBlock) {
+    DevState* st = f.st_all + blockIdx.x;
+    const int4 r = f.rng[blockIdx.x];
+    if (st->finished) return;
+    double m[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    int k = r.x + (int)threadIdx.x;
+    for (; k + 7 * kFinalizeBlock < r.y; k += 8 * kFinalizeBlock) {
 #pragma unroll
-            for (int q = 0; q < 8; ++q) m[q] += partial[k + q * kFinalizeBlock];
-        }
-        for (; k < r.y; k += kFinalizeBlock) m[0] += partial[k];
-        s[threadIdx.x] = ((m[0] + m[1]) + (m[2] + m[3])) + ((m[4] + m[5]) + (m[6] + m[7]));
-        __syncthreads();
-        for (int w = kFinalizeBlock / 2; w > 0; w >>= 1) {
-            if ((int)threadIdx.x < w) s[threadIdx.x] += s[threadIdx.x + w];
-            __syncthreads();
-        }
-        if (threadIdx.x == 0) adaptive_control(st, s[0], (double)n);
-        return;
+        for (int q = 0; q < 8; ++q) m[q] += partial[k + q * kFinalizeBlock];
     }
-    // the instance's CFL (and viscous) slots, reset for the next reduction
-    {
-        const int t = (int)threadIdx.x;
-        double* sl = slots + (size_t)bid * 2 * kSlots;
-        s[t] = 0.0;
-        sv[t] = 0.0;
-        if (t < kSlots) {
-            s[t] = sl[t];
-            sl[t] = 0.0;
-            if (pv_off > 0) {
-                sv[t] = sl[kSlots + t];
-                sl[kSlots + t] = 0.0;
-            }
-        }
-    }
+    for (; k < r.y; k += kFinalizeBlock) m[0] += partial[k];
+    s[threadIdx.x] = ((m[0] + m[1]) + (m[2] + m[3])) + ((m[4] + m[5]) + (m[6] + m[7]));
     __syncthreads();
-    for (int w = kSlots / 2; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) {
-            s[threadIdx.x] = dmax(s[threadIdx.x], s[threadIdx.x + w]);
-            if (pv_off > 0) sv[threadIdx.x] = dmax(sv[threadIdx.x], sv[threadIdx.x + w]);
-        }
+    for (int w = kFinalizeBlock / 2; w > 0; w >>= 1) {
+        if ((int)threadIdx.x < w) s[threadIdx.x] += s[threadIdx.x + w];
         __syncthreads();
     }
-    if (threadIdx.x != 0) return;
+    if (threadIdx.x == 0) adaptive_control(st, s[0], N + 1.0);
+}
+
+// The maximum over the CFL slots of instance `bid` (reset for the next reduction),
+// then compute_dt / set_dt! / set_t_and_iter! / isfinished on the instance's state
+// (lwfr.jl:76-103, 146-148, 176-190; Trixi max_dt).  The viscous maxima give the
+// parabolic bound 1/((λa + λv)·2(2N+1)), λv = 2(2N+1)·max J⁻² max(4μ/(3ρ), μκ/(ρPr)),
+// and max_dt is the smaller of the two (compute_dt for
+// SemidiscretizationHyperbolicParabolic, lwfr.jl:192-210).
+// A step of a small mesh waits for this kernel's chain of memory latencies, so one
+// wave does it, four slots a lane, with every load sent out at the start and the
+// maximum taken across lanes: 1.76 us of a 32² step of 13.7 us (N=4), where 1024
+// lanes and a tree in LDS took 2.96.
+template <int N> __device__ __forceinline__ void finalize_body(const FinArgs& f, int bid) {
+    constexpr int n = N + 1, Q = kSlots / kFinalizeWave;
+    const int lane = threadIdx.x;
+    DevState* st = f.st_all + bid;
+    double* sl = f.slots + (size_t)bid * 2 * kSlots + lane;
+    const bool par = f.pv_off > 0;
+    double m[Q], mv[Q];
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        m[q] = sl[q * kFinalizeWave];
+        mv[q] = par ? sl[kSlots + q * kFinalizeWave] : 0.0;
+    }
+    double t = st->t;
+    const double dt_step = st->dt, tf = st->t_final, cfl = st->cfl;
+    const int cur = st->cur;
+    long long it = st->iter;
+    if (f.reduce == RED_STEP && st->finished) return;
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        sl[q * kFinalizeWave] = 0.0;
+        if (par) sl[kSlots + q * kFinalizeWave] = 0.0;
+    }
+    auto wave_max = [](const double* x) {
+        double v = x[0];
+#pragma unroll
+        for (int q = 1; q < Q; ++q) v = fmax(v, x[q]);
+        return max_groups(max_group8(v));
+    };
     const double tiny = 4.9406564584124654e-324;  // nextfloat(0.0), Trixi's start value
-    const double M = dmax(tiny, s[0]);
+    const double M = dmax(tiny, wave_max(m));
     double max_dt = 2.0 / (n * M);
-    if (pv_off > 0) {
-        const double lam_v = dmax(tiny, sv[0]) * (2.0 * (2.0 * N + 1.0));
+    if (par) {
+        const double lam_v = dmax(tiny, wave_max(mv)) * (2.0 * (2.0 * N + 1.0));
         const double dtv = 1.0 / ((M + lam_v) * (2 * (2.0 * N + 1.0)));
         if (dtv < max_dt) max_dt = dtv;
     }
-    if (reduce == RED_QUERY) {
+    if (lane != 0) return;
+    if (f.reduce == RED_QUERY) {
         st->query = max_dt;
         return;
     }
-    double t = st->t;
-    if (reduce == RED_STEP) {
-        t = t + st->dt;  // set_t_and_iter!
+    if (f.reduce == RED_STEP) {
+        t = t + dt_step;  // set_t_and_iter!
+        it = it + 1;
         st->t = t;
-        st->iter = st->iter + 1;
-        st->cur = 1 - st->cur;
+        st->iter = it;
+        st->cur = 1 - cur;
     }
-    const double tf = st->t_final;
-    double dt = st->cfl * max_dt;  // compute_dt
-    const long long it = st->iter;
+    const DtLog& dl = f.dl;
+    double dt = cfl * max_dt;  // compute_dt
     if (dl.presc && it < dl.presc_n) dt = dl.presc[it];  // prescribed dt of step `it`
     if (t + dt > tf) dt = tf - t;  // set_dt!
     st->dt = dt;
@@ -3490,10 +3493,8 @@ __device__ __forceinline__ void finalize_body(const FinArgs& f, int bid, double*
     st->finished = julia_isapprox(t, tf);
 }
 
-template <int N>
-__global__ __launch_bounds__(kFinalizeBlock) void k_finalize(FinArgs f) {
-    __shared__ double s[kFinalizeBlock], sv[kFinalizeBlock];
-    finalize_body<N>(f, blockIdx.x, s, sv);
+template <int N> __global__ __launch_bounds__(kFinalizeWave) void k_finalize(FinArgs f) {
+    finalize_body<N>(f, blockIdx.x);
 }
 
 // Two contexts advanced by the same launches (tlw_create_ensemble): one of
@@ -3522,12 +3523,11 @@ __global__ __launch_bounds__(kSurfBlock) void k_surface_pair(KArgs a3, KArgs a4,
         surface_body<4, false, false, false>(a4, blockIdx.x - g3);
 }
 
-__global__ __launch_bounds__(kFinalizeBlock) void k_finalize_pair(FinArgs f3, FinArgs f4, int n3) {
-    __shared__ double s[kFinalizeBlock], sv[kFinalizeBlock];
+__global__ __launch_bounds__(kFinalizeWave) void k_finalize_pair(FinArgs f3, FinArgs f4, int n3) {
     if ((int)blockIdx.x < n3)
-        finalize_body<3>(f3, blockIdx.x, s, sv);
+        finalize_body<3>(f3, blockIdx.x);
     else
-        finalize_body<4>(f4, blockIdx.x - n3, s, sv);
+        finalize_body<4>(f4, blockIdx.x - n3);
 }
 
 // Initialisation of the device integrator state of every instance.
