@@ -1220,7 +1220,9 @@ __device__ __forceinline__ void put_fluxes(double* s, int sidx, bool act, const 
 // dt times the source's own difference (dg_2d.jl:980-987, 1033-1045, 1093-1103,
 // 1148-1160; five-point s_tt in the curvilinear kernel 4) and Ssrc receives
 // S = s + s_t/2 + s_tt/6 + ... (1228-1247), which the caller adds to the residual.
-template <int N, int EB, bool CURV = false, bool KEEP = false, bool SRC = false>
+// Without FLUXES it ends with Ũ and tder, which need neither the last level's
+// stencil nor F̃.
+template <int N, int EB, bool CURV = false, bool KEEP = false, bool SRC = false, bool FLUXES = true>
 __device__ __forceinline__ void lw_element(const double* uN, const double* J, double dt, double sc, double gamma,
                                            int i, int j, bool act, int sidx, int sbase, double* A, double* B,
                                            const double* sD, const double* sDh, double* Uc, double* F, double* G,
@@ -1257,6 +1259,7 @@ __device__ __forceinline__ void lw_element(const double* uN, const double* J, do
 #pragma unroll
             for (int s = 0; s < 4; ++s) st[s][v] = fma(kTaylor[s][k - 1], w[v], k == 1 ? uN[v] : st[s][v]);
         }
+        if (!FLUXES && k == N) return;
         constexpr TimeDiff tds[5] = {{}, time_diff<N>(1), time_diff<N>(2), time_diff<N>(3), time_diff<N>(4)};
         const TimeDiff td = tds[k];
         double d[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, q[5];
