@@ -224,14 +224,12 @@ void free_mesh(tlw_ctx* c) {
 // instance's range of partials (volume workgroups, then the node-per-lane grid after them).
 int build_tables(tlw_ctx* c) {
     std::vector<int4> vb, sb, rng(c->ninst);
-    std::vector<int> et(c->E);
     const int seb = surf_eb(c->N);
     for (int k = 0; k < c->ninst; ++k) {
         const int f0 = c->inst_first[k], f1 = c->inst_first[k + 1];
         rng[k].x = (int)vb.size();
         for (int e = f0; e < f1; e += c->ebv) {
             const int nel = std::min(c->ebv, f1 - e);
-            for (int q = 0; q < nel; ++q) et[e + q] = (int)vb.size();
             vb.push_back(make_int4(e, nel, k, 0));
         }
         rng[k].y = (int)vb.size();
@@ -256,9 +254,6 @@ int build_tables(tlw_ctx* c) {
     if ((int)vb.size() > c->vcap) return fail(c, TLW_EINVAL, "volume workgroup table exceeds its allocation");
     c->vgrid = (int)vb.size();
     c->sgrid = (int)sb.size();
-    std::vector<int> link(c->h_nbr);
-    for (size_t q = 0; q < link.size(); ++q)
-        if (link[q] >= 0 && et[link[q]] == et[q / 4]) link[q] = kResolved;
     for (auto& r : rng) {  // surface partials follow the volume ones
         r.z += c->vgrid;
         r.w += c->vgrid;
@@ -266,8 +261,10 @@ int build_tables(tlw_ctx* c) {
     HIPCHK(c, hipStreamSynchronize(c->stream));
     HIPCHK(c, hipMemcpy(c->d_vblk, vb.data(), sizeof(int4) * vb.size(), hipMemcpyHostToDevice));
     HIPCHK(c, hipMemcpy(c->d_sblk, sb.data(), sizeof(int4) * sb.size(), hipMemcpyHostToDevice));
-    HIPCHK(c, hipMemcpy(c->d_link, link.data(), sizeof(int) * link.size(), hipMemcpyHostToDevice));
     HIPCHK(c, hipMemcpy(c->d_rng, rng.data(), sizeof(int4) * rng.size(), hipMemcpyHostToDevice));
+    hipLaunchKernelGGL(k_link, dim3(c->vgrid), dim3(64), 0, c->stream, c->d_vblk, c->d_nbr, c->d_link);
+    HIPCHK(c, hipGetLastError());
+    HIPCHK(c, hipStreamSynchronize(c->stream));  // the next launch may be on another stream
     drop_graphs(c);
     return TLW_OK;
 }

@@ -3034,6 +3034,15 @@ __global__ __launch_bounds__(kSurfBlock) void k_surface(KArgs a) {
     surface_body<N, BC, SC, CURV, MORT>(a, blockIdx.x);
 }
 
+// KArgs::link of one volume workgroup's elements, when the tile is set.
+__global__ __launch_bounds__(64) void k_link(const int4* vblk, const int* nbr, int* link) {
+    const int4 b = vblk[blockIdx.x];
+    for (int q = 4 * b.x + (int)threadIdx.x; q < 4 * (b.x + b.y); q += 64) {
+        const int nb = nbr[q];
+        link[q] = (nb >= b.x && nb < b.x + b.y) ? kResolved : nb;
+    }
+}
+
 // AMR solution transfer between two TreeMesh leaf sets (Trixi's refine! and
 // coarsen! of the DG solution, src/callbacks_step/amr_dg2d.jl in Trixi.jl,
 // which the reference's AMR callback runs before resizing its caches,
