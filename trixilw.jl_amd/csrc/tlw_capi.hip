@@ -66,7 +66,7 @@ struct tlw_ctx {
     int4* d_vblk = nullptr;
     int4* d_sblk = nullptr;
     int* d_link = nullptr;
-    std::vector<int> h_nbr;  // the neighbour table, for the links of a new tile
+    std::vector<int> h_nbr;  // the neighbour table of a mesh with boundary faces (build_tables), else empty
     int4* d_rng = nullptr;
     int vgrid = 0, sgrid = 0, vcap = 0;
     int sbnd = 0;  // the first sbnd node-per-lane workgroups hold the elements with a boundary face (0: mixed)
@@ -572,7 +572,8 @@ int upload_meshes(tlw_ctx* c, const tlw_mesh_desc* ms, int ninst, const tlw_curv
     }
     HIPCHK(c, hipMemcpy(c->d_state, c->h_state, sizeof(DevState) * ninst, hipMemcpyHostToDevice));
     HIPCHK(c, hipMemcpy(c->d_nbr, nbr.data(), sizeof(int) * 4 * E, hipMemcpyHostToDevice));
-    c->h_nbr.assign(nbr.begin(), nbr.end());
+    c->h_nbr.clear();
+    if (c->bc_faces) c->h_nbr = nbr;
     HIPCHK(c, hipMemcpy(c->d_invj, invj.data(), sizeof(double) * E, hipMemcpyHostToDevice));
     HIPCHK(c, hipMemcpy(c->d_center, center.data(), sizeof(double) * 2 * E, hipMemcpyHostToDevice));
     HIPCHK(c, hipMemcpy(c->d_length, length.data(), sizeof(double) * E, hipMemcpyHostToDevice));
