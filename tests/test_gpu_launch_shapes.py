@@ -75,3 +75,29 @@ def test_blended_and_pure_workgroups(oracle_mod, N, tile, mesh_kind):
     assert any(blended) and not all(blended)
     assert_close(du, ref, what=f"{mesh_kind} N={N} tile={tile}")
     semi.close()
+
+
+# MDRK has its own line: one element below it and on it, both stages against the oracle
+@pytest.mark.parametrize("N,nx,ny,tile", [(3, 16, 5, 8), (3, 127, 129, 8), (3, 128, 128, 16), (4, 128, 128, 5),
+                                          (4, 145, 113, 10)])
+def test_default_tile_mdrk(oracle_mod, N, nx, ny, tile):
+    import trixilw_hip as tlw
+
+    torch = torch_mod()
+    print(f"default MDRK tile N={N} {nx}x{ny}", flush=True)
+    semi, o, u_lex, mesh = setup_curved(oracle_mod, N, nx, ny, A=0.02, td="mdrk")
+    assert semi.elements_per_workgroup() == tile
+    dt = 0.2 * o.max_dt(u_lex)
+    ref1 = o.rhs(u_lex, 0.0, dt, kind="mdrk1")
+    us = u_lex + dt * ref1
+    o.set_us(us)
+    ref2 = o.rhs(u_lex, 0.0, dt, kind="mdrk2")
+    u = to_dev(mesh, u_lex)
+    du = torch.empty_like(u)
+    semi.cache["dt"][0] = dt
+    tlw.rhs_mdrk1(du, u, semi, 0.0)
+    assert_close(to_lex(mesh, du), ref1, what=f"MDRK stage 1 N={N} {nx}x{ny}")
+    semi.set_us(to_dev(mesh, us))
+    tlw.rhs_mdrk2(du, u, semi, 0.0)
+    assert_close(to_lex(mesh, du), ref2, what=f"MDRK stage 2 N={N} {nx}x{ny}")
+    semi.close()

@@ -162,13 +162,24 @@ constexpr int kEbChoices3[3] = {4, 8, 16};
 const int* eb_choices(int N) { return N == 4 ? kEbChoices4 : kEbChoices3; }
 // The tile of a context that has not been given one, by its number of elements:
 // small tiles spread a small mesh over the chip, large ones keep more faces inside
-// a workgroup.  Steps of the device loop in us, Euler LW in Z-order, tiles as
-// above: polydeg 4 32² 15.1 / 16.2 / 17.2, 128² 40.7 / 40.6 / 50.7, 256² 118 / 110 / 151
-// (15 elements are six waves, a workgroup and a half on four SIMDs); polydeg 3 32²
-// 14.6 / 14.8 / 15.5, 64² 17.9 / 16.1 / 16.9, 128² 28.3 / 26.4 / 26.9, 256² 70.9 / 65.9 / 62.8.
-// MDRK and Navier-Stokes cross over at the same sizes.
-int default_eb(int N, int E) {
+// a workgroup.  Steps of the device loop in us, tiles as above.  polydeg 4 (15
+// elements are six waves, a workgroup and a half on four SIMDs), LW in strips: Euler
+// 32² 13.9 / 14.7 / 15.9, 128² 39.8 / 40.3 / 50.1, 256² 111 / 107 / 148, Navier-Stokes
+// 128² 62.5 / 63.2 / 81.3, 256² 198 / 198 / 262; MDRK 128² 62.3 / 61.0 / 75.7, 256²
+// 171 / 162 / 223.
+// polydeg 3 LW, Z-order: Euler 16² 12.3 / 12.1 / 13.1, 32² 12.7 / 12.2 / 13.2, 64²
+// 16.3 / 14.5 / 15.2, 128² 28.1 / 27.2 / 27.0 (a rhs call 25.6 / 21.6 / 23.6), 256²
+// 67.3 / 65.7 / 64.7; Navier-Stokes 16² 15.8 / 15.7 / 16.9, 64² 21.5 / 19.5 / 19.5,
+// 128² 37.2 / 38.2 / 37.5.  Up to 2048 elements 4 and 8 are within 5 % of each other
+// and both ahead of 16; a warped 96² takes 23.1 / 21.2 / 23.8.
+// The two launches of an MDRK step gain from the 16-element tile as soon as it fills
+// the chip, 1024 workgroups: 128² Euler 47.6 / 44.6 / 44.2, Navier-Stokes 63.1 / 64.7 /
+// 61.1, warped Navier-Stokes 66.0 / 66.8 / 64.0 and at 120² 67.1 / 63.9 / 64.7, at 96²
+// 50.6 / 48.4 / 51.5; below, 8 is level with 4 at 16² (19.8 / 19.4 / 21.0) and ahead
+// of it at 32² (20.7 / 20.0 / 21.8) and 64² (27.0 / 23.0 / 25.2).
+int default_eb(int N, int E, bool mdrk) {
     if (N == 4) return E <= 16384 ? 5 : 10;
+    if (mdrk) return E < 16384 ? 8 : 16;
     return E <= 2048 ? 4 : E <= 32768 ? 8 : 16;
 }
 int min_eb(int N) { return N == 4 ? 5 : 4; }
@@ -528,7 +539,8 @@ int upload_meshes(tlw_ctx* c, const tlw_mesh_desc* ms, int ninst, const tlw_curv
     HIPCHK(c, hipMalloc(&c->d_us, sizeof(double) * nd));
     // tables and partials sized for the smallest tile, so the tile can change freely
     c->vcap = (E + min_eb(c->N) - 1) / min_eb(c->N) + ninst;
-    if (!c->ebv_given) c->ebv = default_eb(c->N, E);  // at most 256 nodes, as Navier-Stokes walls need
+    // at most 256 nodes, as Navier-Stokes walls need
+    if (!c->ebv_given) c->ebv = default_eb(c->N, E, c->time_disc == TLW_MDRK);
     const int scap = (E + surf_eb(c->N) - 1) / surf_eb(c->N) + ninst;
     // hyperbolic-parabolic: the viscous partials follow in a second block of the same size
     c->pv_off = c->parabolic ? c->vcap + scap : 0;
