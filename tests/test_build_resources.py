@@ -58,3 +58,13 @@ def test_hot_kernels_stay_out_of_private_memory(usage):
             assert u["ScratchSize"] == 0 and u["Occupancy"] >= 1, (name, u)
         else:
             assert u["Occupancy"] >= 2, (name, u)
+
+
+def test_adjoint_kernels_stay_out_of_private_memory(usage):
+    adj = {k: v for k, v in usage.items() if re.match(r"_ZN3tlw\d+k_adj", k)}
+    # LW, MDRK and shock-capturing steps, each with its face records, at both degrees
+    assert len(adj) == 2 * (2 + 4 + 2), sorted(adj)
+    for name, u in adj.items():
+        # the N=4 LW kernel holds the derivatives of four Taylor levels and spills 84 B
+        lw4 = re.match(r"_ZN3tlw9k_adjointILi4E", name) is not None
+        assert u["ScratchSize"] <= (84 if lw4 else 0), (name, u)
