@@ -151,3 +151,47 @@ def test_ensemble_one_launch_matches_separate_batches(oracle_mod, tiles, graphs)
     ens.close()
     for b, _ in groups.values():
         b.close()
+
+
+def test_ensemble_with_only_the_polydeg4_tile_given(oracle_mod):
+    """An ensemble made through the C ABI whose polydeg-4 context was given 10 elements per
+    workgroup and whose polydeg-3 context (here of few elements, default 4) was given none
+    advances with the tiles (16, 10), to the same bits."""
+    import ctypes as C
+
+    import torch
+    import trixilw_hip as tlw
+
+    torch_mod()
+    L, K = tlw._lib.lib(), 4
+    groups = _c4_groups(tlw, n_instances=5, seed=27)
+    u0s = [groups[N][0].compute_coefficients() for N in (3, 4)]
+    cfls = [groups[N][1] for N in (3, 4)]
+    h3, h4 = (groups[N][0].handle for N in (3, 4))
+    dp = C.POINTER(C.c_double)
+
+    def states(ens):
+        for h, u in zip((h3, h4), u0s):
+            u = np.ascontiguousarray(u)
+            tlw._lib.check(L.tlw_set_state(h, u.ctypes.data_as(dp), u.size), h)
+        assert L.tlw_ensemble_solve_init(ens, 0.0, float("inf"), cfls[0], cfls[1]) == 0
+        assert L.tlw_ensemble_advance(ens, K, None) == 0, L.tlw_ensemble_last_error(ens).decode()
+        out = []
+        for h, u in zip((h3, h4), u0s):
+            v = np.empty_like(np.ascontiguousarray(u))
+            tlw._lib.check(L.tlw_get_state(h, v.ctypes.data_as(dp), v.size), h)
+            out.append(v)
+        return out
+
+    eb = C.c_int32()
+    tlw._lib.check(L.tlw_get_elements_per_workgroup(h3, C.byref(eb)), h3)
+    assert eb.value != 16
+    ens = C.c_void_p()
+    assert L.tlw_create_ensemble(h3, h4, C.byref(ens)) == 0
+    tlw._lib.check(L.tlw_set_elements_per_workgroup(h4, 10), h4)
+    got = states(ens)
+    tlw._lib.check(L.tlw_set_elements_per_workgroup(h3, 16), h3)
+    ref = states(ens)
+    L.tlw_ensemble_destroy(ens)
+    for a, b in zip(got, ref):
+        assert np.array_equal(a, b)

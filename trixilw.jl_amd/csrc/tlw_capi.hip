@@ -1963,6 +1963,16 @@ int tlw_ensemble_advance(tlw_ensemble* e, int32_t max_steps, int32_t* finished) 
     if (max_steps < 0) return ens_fail(e, TLW_EINVAL, "max_steps < 0");
     tlw_ctx* c3 = e->c3;
     tlw_ctx* c4 = e->c4;
+    // a polydeg-3 context that was given no tile takes 16 beside a 10 that was given,
+    // whatever its default on its own
+    if (!c3->ebv_given && c4->ebv_given && c4->ebv == 10 && c3->ebv != 16) {
+        const int own = c3->ebv;
+        c3->ebv = 16;
+        if (int rc = build_tables(c3)) {
+            c3->ebv = own;
+            return ens_fail(e, rc, c3->err);
+        }
+    }
     const bool pair16 = c3->ebv == 16 && c4->ebv == 10, pair8 = c3->ebv == 8 && c4->ebv == 5;
     if (!pair16 && !pair8)
         return ens_fail(e, TLW_EINVAL, "tiles (elements per workgroup) must be (16, 10) or (8, 5)");
