@@ -302,8 +302,10 @@ int tlw_ensemble_solve_init(tlw_ensemble* ens, double t0, double t_final, double
 int tlw_ensemble_advance(tlw_ensemble* ens, int32_t max_steps, int32_t* finished_host);
 const char* tlw_ensemble_last_error(const tlw_ensemble* ens);
 void tlw_ensemble_destroy(tlw_ensemble* ens);
-/* Replay tlw_advance's steps from a captured HIP graph (one graph per step count, captured on
- * first use; needs an explicit stream from tlw_set_stream).  No counterpart in the reference. */
+/* Replay tlw_advance's steps from a captured HIP graph (one graph per step count, captured on its
+ * first use for the first count and on the second for others, at most 16, other counts being
+ * launched step by step; needs an explicit stream from tlw_set_stream).  No counterpart in the
+ * reference. */
 int tlw_enable_graphs(tlw_ctx* ctx, int32_t enable);
 
 /* AMR or any host-side mesh change: rebuild the device mesh (src/callbacks/amr.jl:2-20 resize!) */

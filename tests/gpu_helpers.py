@@ -68,6 +68,18 @@ def assert_close(a, b, tol=TOL, what=""):
     assert l2 <= tol and li <= tol, f"{what}: rel L2 {l2:.3e}, rel Linf {li:.3e}"
 
 
+def traced(fn):
+    """fn's result, and the names of the runtime calls and kernels that it made."""
+    torch = torch_mod()
+    from torch.profiler import ProfilerActivity, profile
+
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CPU, ProfilerActivity.CUDA]) as p:
+        out = fn()
+        torch.cuda.synchronize()
+    return out, [e.name for e in p.events()]
+
+
 GAMMA = 1.4
 
 

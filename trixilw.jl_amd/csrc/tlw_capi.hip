@@ -15,6 +15,7 @@
 #include <cstdio>
 #include <cstring>
 #include <map>
+#include <set>
 #include <string>
 #include <vector>
 
@@ -129,6 +130,7 @@ struct tlw_ctx {
     long long dtpresc_n = 0;
     bool graphs = false;
     std::map<int, hipGraphExec_t> graph_cache;
+    std::set<int> graph_seen;  // step counts launched without a graph once (advance_graph)
     hipStream_t graph_stream = nullptr;
     std::string err;
 };
@@ -194,6 +196,7 @@ constexpr int kSplitSurface = 4096;  // workgroups (build_tables)
 void drop_graphs(tlw_ctx* c) {
     for (auto& kv : c->graph_cache) (void)hipGraphExecDestroy(kv.second);
     c->graph_cache.clear();
+    c->graph_seen.clear();
 }
 
 void free_mesh(tlw_ctx* c) {
@@ -1031,8 +1034,13 @@ void enqueue_step(tlw_ctx* c) {
     }
 }
 
-// Replays max_steps steps from a graph captured on first use for this step
-// count and stream.  The captured launches contain no memory sets.
+// Replays max_steps steps from a graph captured for this step count and stream: the
+// first count of a context at once, a further one when it is asked for again, up to
+// kMaxGraphs of them; else the steps are launched one by one.  A host whose last
+// count follows from the remaining time (solve_lwfr) so captures and keeps its
+// regular chunk and not a graph for every remainder.  The captured launches contain
+// no memory sets.
+constexpr size_t kMaxGraphs = 16;
 int advance_graph(tlw_ctx* c, int max_steps) {
     if (!c->stream) return fail(c, TLW_EINVAL, "graph replay needs an explicit stream (tlw_set_stream)");
     if (c->graph_stream != c->stream) {
@@ -1041,6 +1049,11 @@ int advance_graph(tlw_ctx* c, int max_steps) {
     }
     auto it = c->graph_cache.find(max_steps);
     if (it == c->graph_cache.end()) {
+        if (!c->graph_cache.empty() &&
+            (c->graph_cache.size() >= kMaxGraphs || c->graph_seen.insert(max_steps).second)) {
+            for (int k = 0; k < max_steps; ++k) enqueue_step(c);
+            return TLW_OK;
+        }
         hipGraph_t g = nullptr;
         hipError_t e = hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal);
         if (e == hipSuccess) {
