@@ -839,6 +839,16 @@ void launch_finalize(tlw_ctx* c, int reduce) {
     if (c->N == 4) launch_finalize_t<4>(c, reduce);
     else launch_finalize_t<3>(c, reduce);
 }
+template <int N, bool BC, bool RED> auto surface_kernel_t(const tlw_ctx* c) -> void (*)(KArgs) {
+    if (c->curved) return c->sc ? k_surface<N, BC, true, true, false, RED> : k_surface<N, BC, false, true, false, RED>;
+    if (c->n_mortars > 0) return k_surface<N, BC, false, false, true, RED>;  // plain FR on refined cells
+    return c->sc ? k_surface<N, BC, true, false, false, RED> : k_surface<N, BC, false, false, false, RED>;
+}
+// with or without boundary code, for a launch that reduces or not
+template <int N> auto surface_kernel(const tlw_ctx* c, bool bc, bool red) -> void (*)(KArgs) {
+    if (bc) return red ? surface_kernel_t<N, true, true>(c) : surface_kernel_t<N, true, false>(c);
+    return red ? surface_kernel_t<N, false, true>(c) : surface_kernel_t<N, false, false>(c);
+}
 template <int N> void launch_surface_t(tlw_ctx* c, const KArgs& a) {
     if (c->curved && c->has_boundary && a.in_sel == SEL_EXPLICIT && !a.u) {
         // the curvilinear boundary faces read uⁿ: never launch without it
@@ -855,23 +865,8 @@ template <int N> void launch_surface_t(tlw_ctx* c, const KArgs& a) {
         if (count <= 0) return;
         KArgs q = a;
         q.sblk += first;
-        const dim3 g(count), b(kSurfBlock);
-        if (c->curved && c->sc) {
-            if (bc) hipLaunchKernelGGL(HIP_KERNEL_NAME(k_surface<N, true, true, true>), g, b, 0, c->stream, q);
-            else hipLaunchKernelGGL(HIP_KERNEL_NAME(k_surface<N, false, true, true>), g, b, 0, c->stream, q);
-        } else if (c->curved) {
-            if (bc) hipLaunchKernelGGL(HIP_KERNEL_NAME(k_surface<N, true, false, true>), g, b, 0, c->stream, q);
-            else hipLaunchKernelGGL(HIP_KERNEL_NAME(k_surface<N, false, false, true>), g, b, 0, c->stream, q);
-        } else if (c->n_mortars > 0) {  // plain FR on a TreeMesh with refined cells
-            if (bc) hipLaunchKernelGGL(HIP_KERNEL_NAME(k_surface<N, true, false, false, true>), g, b, 0, c->stream, q);
-            else hipLaunchKernelGGL(HIP_KERNEL_NAME(k_surface<N, false, false, false, true>), g, b, 0, c->stream, q);
-        } else if (c->sc) {
-            if (bc) hipLaunchKernelGGL(HIP_KERNEL_NAME(k_surface<N, true, true>), g, b, 0, c->stream, q);
-            else hipLaunchKernelGGL(HIP_KERNEL_NAME(k_surface<N, false, true>), g, b, 0, c->stream, q);
-        } else {
-            if (bc) hipLaunchKernelGGL(HIP_KERNEL_NAME(k_surface<N, true, false>), g, b, 0, c->stream, q);
-            else hipLaunchKernelGGL(HIP_KERNEL_NAME(k_surface<N, false, false>), g, b, 0, c->stream, q);
-        }
+        void (*kernel)(KArgs) = surface_kernel<N>(c, bc, a.reduce != RED_NONE);
+        hipLaunchKernelGGL(kernel, dim3(count), dim3(kSurfBlock), 0, c->stream, q);
     };
     const bool bc = c->n_mortars > 0 ? c->bc_faces : c->has_boundary;
     const int nb = !bc ? 0 : c->sbnd > 0 ? c->sbnd : c->sgrid;

@@ -2787,7 +2787,13 @@ __device__ inline void boundary_record_curved(const KArgs& a, int e, int face, i
 // CFL maxima and the admissibility test.
 // BC: the mesh has domain-boundary faces; MORT: it has faces on L2 mortars (a
 // mesh with mortars and no boundary face compiles no boundary code).
-template <int N, bool BC, bool SC, bool CURV = false, bool MORT = false>
+// RED: the launch reduces (a.reduce is not RED_NONE) and reads every node's value,
+// which goes out together with the faces' links.  One that does not (a rhs, MDRK
+// stage 1, a step with the limiter) reads only what it corrects: a rhs at 256² then
+// takes 103.5 us instead of 105.9 (N=4) and 58.9 instead of 60.3 (N=3), MDRK stage 2
+// alone at 512² 206 instead of 211 (N=3) and 326 instead of 331 (N=4).  A kernel of
+// its own, as the choice at run time costs a step of a 32² mesh 1.5 %.
+template <int N, bool BC, bool SC, bool CURV, bool MORT, bool RED>
 __device__ __forceinline__ void surface_body(const KArgs& a, int bid) {
     using G_ = SGeo<N>;
     constexpr int n = G_::n, NN = G_::NN, EB = G_::EB, S = G_::S;
@@ -2810,21 +2816,15 @@ __device__ __forceinline__ void surface_body(const KArgs& a, int bid) {
     const double invJ = CURV ? a.ijn[(size_t)e * NN + node] : a.inv_jac[e];
     const int fx = (i == 0) ? 0 : ((i == n - 1) ? 1 : -1);
     const int fy = (j == 0) ? 2 : ((j == n - 1) ? 3 : -1);
-    // A launch that reduces reads every node's value, which goes out together with the
-    // faces' links; one that does not (a rhs, MDRK stage 1, a step with the limiter)
-    // reads only what it corrects: a rhs at 256² then takes 105.7 us instead of 109.8
-    // (N=4) and 58.9 instead of 60.3 (N=3), MDRK stage 2 alone at 512² 208 instead of
-    // 212 (N=3) and 327 instead of 335 (N=4).
-    const bool reduces = a.reduce != RED_NONE;
     const size_t off = ((size_t)e * NN + node) * 4;
     int nbx = kResolved, nby = kResolved;
     if (fx >= 0) nbx = a.link[4 * e + fx];
     if (fy >= 0) nby = a.link[4 * e + fy];
     double val[4];
-    if (reduces) load4(out + off, val);
+    if constexpr (RED) load4(out + off, val);
     const bool extx = nbx != kResolved, exty = nby != kResolved;
     if (act && (extx || exty)) {
-        if (!reduces) load4(out + off, val);
+        if constexpr (!RED) load4(out + off, val);
         double surf[4] = {0.0, 0.0, 0.0, 0.0};
         constexpr int RQ = kRQ<SC>;
         auto do_face = [&](int f, int l, int nb) {
@@ -3012,7 +3012,7 @@ __device__ __forceinline__ void surface_body(const KArgs& a, int bid) {
         for (int v = 0; v < 4; ++v) val[v] = fma(fac, surf[v], val[v]);
         store4(out + off, val);
     }
-    if (!reduces) return;
+    if constexpr (!RED) return;
     // Every node's final value, corrected here or finalised by the volume kernel:
     // CFL maxima (Trixi max_dt) and the admissibility test of the updated state
     // cover all nodes here.
@@ -3035,9 +3035,9 @@ __device__ __forceinline__ void surface_body(const KArgs& a, int bid) {
     cfl_maxima<N>(a.slots, blk.z, tid, nel, lec * NN + node, act, node == 0, l1, l2, lv, invJ, CURV, par);
 }
 
-template <int N, bool BC, bool SC, bool CURV = false, bool MORT = false>
+template <int N, bool BC, bool SC, bool CURV, bool MORT, bool RED>
 __global__ __launch_bounds__(kSurfBlock) void k_surface(KArgs a) {
-    surface_body<N, BC, SC, CURV, MORT>(a, blockIdx.x);
+    surface_body<N, BC, SC, CURV, MORT, RED>(a, blockIdx.x);
 }
 
 // KArgs::link of one volume workgroup's elements, when the tile is set.
@@ -3536,9 +3536,9 @@ __global__ __launch_bounds__((VGeo<4, EB4>::NT), kVolWaves<false>) void k_volume
 
 __global__ __launch_bounds__(kSurfBlock) void k_surface_pair(KArgs a3, KArgs a4, int g3) {
     if ((int)blockIdx.x < g3)
-        surface_body<3, false, false, false>(a3, blockIdx.x);
+        surface_body<3, false, false, false, false, true>(a3, blockIdx.x);
     else
-        surface_body<4, false, false, false>(a4, blockIdx.x - g3);
+        surface_body<4, false, false, false, false, true>(a4, blockIdx.x - g3);
 }
 
 __global__ __launch_bounds__(kFinalizeWave) void k_finalize_pair(FinArgs f3, FinArgs f4, int n3) {
