@@ -63,12 +63,12 @@ struct tlw_ctx {
     double* d_partial = nullptr;
     double* d_alpha_tmp = nullptr;
     double* d_alpha = nullptr;
-    // workgroup tables (KArgs::vblk, sblk, link) and per-instance partial ranges
+    // workgroup tables (KArgs::vblk, sblk, link) and each instance's range of volume workgroups
     int4* d_vblk = nullptr;
     int4* d_sblk = nullptr;
     int* d_link = nullptr;
     std::vector<int> h_nbr;  // the neighbour table of a mesh with boundary faces (build_tables), else empty
-    int4* d_rng = nullptr;
+    int2* d_rng = nullptr;
     int vgrid = 0, sgrid = 0, vcap = 0;
     int sbnd = 0;  // the first sbnd node-per-lane workgroups hold the elements with a boundary face (0: mixed)
     bool sc = false;
@@ -86,7 +86,6 @@ struct tlw_ctx {
     double* d_sqrk = nullptr;  // calc_fn_low! normals of subcell face n-1 [E][n][4]
     bool bad_launch = false;  // a launch was refused for a missing input (reported by check_launch)
     size_t slot_off = 0;      // offset of the CFL maxima slots in d_partial
-    int pv_off = 0;           // offset of the viscous CFL partials (0: none)
     int ebv = 0;              // elements per volume workgroup
     bool ebv_given = false;   // by tlw_set_elements_per_workgroup or tlw_autotune; else default_eb of the mesh
     bool positivity = false;  // Zhang-Shu limiter in the device loop
@@ -213,7 +212,8 @@ void free_mesh(tlw_ctx* c) {
     c->d_invj = c->d_center = c->d_length = c->d_trace = c->d_us = c->d_auxU = c->d_auxF = nullptr;
     c->d_buf[0] = c->d_buf[1] = nullptr;
     c->d_partial = c->d_alpha_tmp = c->d_alpha = nullptr;
-    c->d_vblk = c->d_sblk = c->d_rng = nullptr;
+    c->d_vblk = c->d_sblk = nullptr;
+    c->d_rng = nullptr;
     c->d_link = nullptr;
     c->d_state = nullptr;
     c->h_state = nullptr;
@@ -235,9 +235,10 @@ void free_mesh(tlw_ctx* c) {
 // Workgroup tables for the current tile: volume workgroups of ebv elements and
 // node-per-lane workgroups of the surface size, both restarted at every
 // instance boundary, the faces that leave a volume workgroup (KArgs::link) and each
-// instance's range of partials (volume workgroups, then the node-per-lane grid after them).
+// instance's range of volume workgroups.
 int build_tables(tlw_ctx* c) {
-    std::vector<int4> vb, sb, rng(c->ninst);
+    std::vector<int4> vb, sb;
+    std::vector<int2> rng(c->ninst);
     const int seb = surf_eb(c->N);
     for (int k = 0; k < c->ninst; ++k) {
         const int f0 = c->inst_first[k], f1 = c->inst_first[k + 1];
@@ -247,9 +248,7 @@ int build_tables(tlw_ctx* c) {
             vb.push_back(make_int4(e, nel, k, 0));
         }
         rng[k].y = (int)vb.size();
-        rng[k].z = (int)sb.size();
         for (int e = f0; e < f1; e += seb) sb.push_back(make_int4(e, std::min(seb, f1 - e), k, 0));
-        rng[k].w = (int)sb.size();
     }
     // The boundary code holds the surface kernel to two waves per SIMD (181 VGPRs
     // against 78): on a large mesh the workgroups without a boundary face come last
@@ -268,14 +267,10 @@ int build_tables(tlw_ctx* c) {
     if ((int)vb.size() > c->vcap) return fail(c, TLW_EINVAL, "volume workgroup table exceeds its allocation");
     c->vgrid = (int)vb.size();
     c->sgrid = (int)sb.size();
-    for (auto& r : rng) {  // surface partials follow the volume ones
-        r.z += c->vgrid;
-        r.w += c->vgrid;
-    }
     HIPCHK(c, hipStreamSynchronize(c->stream));
     HIPCHK(c, hipMemcpy(c->d_vblk, vb.data(), sizeof(int4) * vb.size(), hipMemcpyHostToDevice));
     HIPCHK(c, hipMemcpy(c->d_sblk, sb.data(), sizeof(int4) * sb.size(), hipMemcpyHostToDevice));
-    HIPCHK(c, hipMemcpy(c->d_rng, rng.data(), sizeof(int4) * rng.size(), hipMemcpyHostToDevice));
+    HIPCHK(c, hipMemcpy(c->d_rng, rng.data(), sizeof(int2) * rng.size(), hipMemcpyHostToDevice));
     hipLaunchKernelGGL(k_link, dim3(c->vgrid), dim3(64), 0, c->stream, c->d_vblk, c->d_nbr, c->d_link);
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipStreamSynchronize(c->stream));  // the next launch may be on another stream
@@ -545,17 +540,16 @@ int upload_meshes(tlw_ctx* c, const tlw_mesh_desc* ms, int ninst, const tlw_curv
     // at most 256 nodes, as Navier-Stokes walls need
     if (!c->ebv_given) c->ebv = default_eb(c->N, E, c->time_disc == TLW_MDRK);
     const int scap = (E + surf_eb(c->N) - 1) / surf_eb(c->N) + ninst;
-    // hyperbolic-parabolic: the viscous partials follow in a second block of the same size
-    c->pv_off = c->parabolic ? c->vcap + scap : 0;
-    // partials, then per instance 2·kSlots CFL/viscous maxima slots, zero between reductions
-    c->slot_off = (size_t)((c->parabolic ? 2 : 1) * (c->vcap + scap) + 1);
+    // a temporal-error sum per volume workgroup, then per instance 2·kSlots CFL/viscous
+    // maxima slots, zero between reductions
+    c->slot_off = (size_t)c->vcap;
     const size_t npart = c->slot_off + (size_t)ninst * 2 * kSlots;
     HIPCHK(c, hipMalloc(&c->d_partial, sizeof(double) * npart));
     HIPCHK(c, hipMemset(c->d_partial, 0, sizeof(double) * npart));
     HIPCHK(c, hipMalloc(&c->d_vblk, sizeof(int4) * (size_t)c->vcap));
     HIPCHK(c, hipMalloc(&c->d_sblk, sizeof(int4) * (size_t)scap));
     HIPCHK(c, hipMalloc(&c->d_link, sizeof(int) * 4 * (size_t)E));
-    HIPCHK(c, hipMalloc(&c->d_rng, sizeof(int4) * (size_t)ninst));
+    HIPCHK(c, hipMalloc(&c->d_rng, sizeof(int2) * (size_t)ninst));
     if (c->hconst.ns_walls) HIPCHK(c, hipMalloc(&c->d_fvb, sizeof(double) * (size_t)E * 4 * c->n * 6));
     if (pd) {
         HIPCHK(c, hipMalloc(&c->d_plink, sizeof(int4) * plink.size()));
@@ -668,9 +662,7 @@ KArgs base_args(tlw_ctx* c) {
     a.c = c->d_const;
     a.st = c->d_state;
     a.partial = c->d_partial;
-    a.pv_off = c->pv_off;
-    a.vol_grid = c->vgrid;
-    a.ebv = c->ebv;
+    a.parabolic = c->parabolic;
     a.vblk = c->d_vblk;
     a.sblk = c->d_sblk;
     a.link = c->d_link;
@@ -825,7 +817,7 @@ void launch_volume(tlw_ctx* c, const KArgs& a, int kind) {
     else launch_volume_t<3>(c, a, kind);
 }
 FinArgs fin_args(tlw_ctx* c, int reduce) {
-    return FinArgs{c->d_state, c->d_partial, c->d_rng, reduce, c->pv_off, c->d_partial + c->slot_off,
+    return FinArgs{c->d_state, c->d_partial, c->d_rng, reduce, c->parabolic, c->d_partial + c->slot_off,
                    DtLog{c->d_dtlog, c->dtlog_cap, c->d_dtpresc, c->dtpresc_n}};
 }
 template <int N> void launch_finalize_t(tlw_ctx* c, int reduce) {

@@ -190,11 +190,7 @@ struct KArgs {
     DevState* st;
     double* auxU;      // optional full Ũ
     double* auxF;      // optional full F̃
-    // per-workgroup partials: the volume kernel's temporal-error sums (adaptive
-    // steps), then the node-per-lane kernels' maxima of J⁻¹(max λ1 + max λ2)
-    double* partial;
-    int vol_grid;      // number of volume workgroups (offset of the node-per-lane partials)
-    int ebv;           // elements per volume workgroup
+    double* partial;   // the volume workgroups' temporal-error sums (adaptive steps)
     // Workgroup tables: {first element, elements, instance, 0} per workgroup of the
     // volume grid (vblk) and of the node-per-lane grids (sblk).  Workgroups never
     // straddle two instances of a batch, so each reads one instance's state.
@@ -203,10 +199,9 @@ struct KArgs {
     const int* link;   // [E][4] nbr for the faces that leave a volume workgroup, kResolved for the others
     const double* alpha_tmp;  // indicator values before smoothing [E]
     double* alpha_out;        // smoothed blending factors [E] (optional)
-    // hyperbolic-parabolic CFL reduction: the per-workgroup maxima of the
-    // viscous bound J⁻² max(4μ/(3ρ), μκ/(ρ Pr)) sit pv_off entries after the
-    // advective ones (0: no parabolic terms)
-    int pv_off;
+    // hyperbolic-parabolic: the CFL reduction takes the maximum of the viscous bound
+    // J⁻² max(4μ/(3ρ), μκ/(ρ Pr)) too
+    int parabolic;
     // curvilinear StructuredMesh (null on a TreeMesh): per node the contravariant
     // vectors (Ja11, Ja12, Ja21, Ja22) [E][n²][4] and inverse Jacobian [E][n²],
     // per face node the shared face normal (n1, n2, |n|, 0) [E][4][n][4]
@@ -2780,7 +2775,7 @@ __device__ inline void boundary_record_curved(const KArgs& a, int e, int face, i
     make_record(r, p4est_form ? Uo : uo, Fo, fabs(fma(b1, nf[0], b2 * nf[1])), sqrt_gs(c->gamma * pb * ir) * nf[2]);
 }
 
-// Surface kernel: the faces that leave a volume workgroup (a.ebv elements).
+// Surface kernel: the faces that leave a volume workgroup.
 // Each interface is evaluated by both neighbours from identical inputs, so
 // both see the same bits.  In step mode every lane then takes its node's
 // final value (corrected here or finalised by the volume kernel) into the
@@ -3020,7 +3015,7 @@ __device__ __forceinline__ void surface_body(const KArgs& a, int bid) {
         if (act && !admissible(val, c->gamma)) a.st[blk.z].bad_state = 1;
         return;
     }
-    const bool par = a.pv_off > 0;
+    const bool par = a.parabolic != 0;
     double l1, l2;
     bool bad;
     if constexpr (CURV) {
@@ -3189,7 +3184,7 @@ __global__ __launch_bounds__(kSurfBlock) void k_max_speed(KArgs a) {
         node_speeds(val, c->gamma, l1, l2, bad);
     }
     if (act && bad) a.st[blk.z].bad_state = 1;
-    const bool par = a.pv_off > 0;
+    const bool par = a.parabolic != 0;
     const double lv = par ? (curv ? lam_visc_curved(val, invJ, c) : lam_visc(val, invJ, c)) : 0.0;
     cfl_maxima<N>(a.slots, blk.z, tid, nel, lec * NN + node, act, node == 0, l1, l2, lv, invJ, curv, par);
 }
@@ -3340,7 +3335,7 @@ __global__ __launch_bounds__(kSurfBlock) void k_limiter(KArgs a) {
     if (a.reduce == RED_NONE) return;
     // CFL maxima of the limited state (curvilinear speeds carry the node's |J⁻¹|;
     // Navier-Stokes adds the viscous bound)
-    const bool curv = a.Ja != nullptr, par = a.pv_off > 0;
+    const bool curv = a.Ja != nullptr, par = a.parabolic != 0;
     const double invJ = curv ? a.ijn[(size_t)e * NN + node] : a.inv_jac[e];
     double l1, l2;
     bool bad;
@@ -3409,12 +3404,13 @@ struct DtLog {
     long long presc_n;
 };
 // The arguments of one context's finalize launch; reduce is RED_QUERY, RED_INIT or
-// RED_STEP, pv_off > 0 with parabolic terms.
+// RED_STEP, or RED_ADAPT for k_finalize_adaptive, which reads partial and rng (the range
+// of each instance's volume workgroups).
 struct FinArgs {
     DevState* st_all;
     const double* partial;
-    const int4* rng;
-    int reduce, pv_off;
+    const int2* rng;
+    int reduce, parabolic;
     double* slots;
     DtLog dl;
 };
@@ -3426,7 +3422,7 @@ __global__ __launch_bounds__(kFinalizeBlock) void k_finalize_adaptive(FinArgs f)
     __shared__ double s[kFinalizeBlock];
     const double* partial = f.partial;
     DevState* st = f.st_all + blockIdx.x;
-    const int4 r = f.rng[blockIdx.x];
+    const int2 r = f.rng[blockIdx.x];
     if (st->finished) return;
     double m[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     int k = r.x + (int)threadIdx.x;
@@ -3459,7 +3455,7 @@ template <int N> __device__ __forceinline__ void finalize_body(const FinArgs& f,
     const int lane = threadIdx.x;
     DevState* st = f.st_all + bid;
     double* sl = f.slots + (size_t)bid * 2 * kSlots + lane;
-    const bool par = f.pv_off > 0;
+    const bool par = f.parabolic != 0;
     double m[Q], mv[Q];
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
