@@ -266,8 +266,10 @@ __global__ __launch_bounds__((VGeo<N, EB>::NT), 2) void k_adjoint(KArgs a) {
     if (fy >= 0) face(fy, i, Gb);
 
     // --- volume term D̂·(F̃, G̃): (F̄, Ḡ) += D̂ᵀ s̄
-    double* ex0 = lds;          // exchange buffers, 4 doubles per node each
-    double* ex1 = lds + 4 * S;  // (the forward's last reads were of s2)
+    // exchange buffers, 4 doubles per node each, in lds to lds + 8 S: adj_forward uses what
+    // lies above (its last contraction may still be running), so no barrier goes before
+    double* ex0 = lds;
+    double* ex1 = lds + 4 * S;
     if (act) put4<S>(ex0, sidx, sb);
     __syncthreads();
     {

@@ -864,8 +864,8 @@ template <int N> void launch_surface_t(tlw_ctx* c, const KArgs& a) {
     const int nb = !bc ? 0 : c->sbnd > 0 ? c->sbnd : c->sgrid;
     launch(true, 0, nb);
     launch(false, nb, c->sgrid - nb);
-    // the step's CFL partials come from the surface kernel alone; with adaptive
-    // steps the volume kernel's temporal-error sums are read by the finalize kernel
+    // the step's CFL maxima come from the surface kernel alone; with adaptive steps the
+    // finalize kernel reads the volume kernel's temporal-error sums
     if (a.reduce != RED_NONE) launch_finalize(c, a.reduce);
 }
 void launch_surface(tlw_ctx* c, const KArgs& a) {
@@ -976,10 +976,10 @@ void enqueue_step(tlw_ctx* c) {
     KArgs a = base_args(c);
     a.use_state_dt = 1;
     a.step_mode = 1;
-    // Without a limiter the CFL reduction of uⁿ⁺¹ is split between the volume
-    // kernel (nodes it finalises) and the surface kernel (the rest); with the
-    // positivity limiter (applied after the update, lwfr.jl:226) the limiter
-    // kernel takes it over the limited state.
+    // Without a limiter the surface kernel takes the CFL maxima of uⁿ⁺¹, over every
+    // node; with the positivity limiter (applied after the update, lwfr.jl:226) the
+    // limiter kernel takes them over the limited state.  An adaptive step sums its
+    // temporal errors in the volume kernel and tests uⁿ⁺¹ in the surface kernel.
     const int red = c->adaptive ? RED_ADAPT : (c->positivity ? RED_NONE : RED_STEP);
     if (c->time_disc == TLW_LW) {
         KArgs v = a;

@@ -1744,7 +1744,7 @@ __device__ __forceinline__ void par_level(bool act, int sidx, int sbase, int i, 
 }
 
 // lw_volume_kernel_3!/4! with viscous terms (dg_2d_parabolic.jl:725-1189,
-// 1191-1860): the Euler procedure of lw3_element/lw_element on the total
+// 1191-1860): the Euler procedure of lw_element on the total
 // flux, with the states of ∇u advanced by the same Taylor coefficients.
 // Buffer use: s0 keeps f(uⁿ) for the 5- and 3-point stencils, s1 takes each
 // flux derivative, s2 each time derivative; the final F̃ exchange is in s2.
