@@ -491,7 +491,12 @@ int tlw_apply_positivity_limiter(tlw_ctx* ctx, double* u_dev);
 /* Tile of the fused volume kernel (no counterpart in the reference, whose @threaded loop
  * has no tile): elements per workgroup, one lane per GLL node.  polydeg 4: 5, 10 or 15
  * (default 5, above 16384 elements 10); polydeg 3: 4, 8 or 16 (default with LW 4, above 2048
- * elements 8, above 32768 16; with MDRK 8, from 16384 elements 16).  Results do not depend on the tile.
+ * elements 8, above 32768 16; with MDRK 8, from 16384 elements 16).  Results agree to
+ * rounding across tiles, not to the last bit: a face inside a workgroup enters a node's sum before
+ * its one rounded update, a face between workgroups after it, and an adaptive step sums its
+ * temporal errors by workgroup.  The default counts all elements of the context, so an instance of
+ * a batch, or a mesh after tlw_rebuild_mesh, may run another tile than the same mesh alone; a tile
+ * that was set stays, and with it the instance gives the same bits in both.
  * tlw_autotune times `reps` rhs evaluations per tile on the current state buffer (after
  * tlw_set_state), keeps the fastest and writes it to *chosen and the per-rhs milliseconds
  * of the three tiles, in the order above, to ms[3] (may be NULL).  The other state buffer

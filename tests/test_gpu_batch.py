@@ -195,3 +195,27 @@ def test_ensemble_with_only_the_polydeg4_tile_given(oracle_mod):
     L.tlw_ensemble_destroy(ens)
     for a, b in zip(got, ref):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("N,tile", [(3, 4), (3, 16), (4, 10)])
+def test_a_given_tile_gives_the_bits_of_the_instance_alone(oracle_mod, N, tile):
+    """The default tile counts all elements of a batch; with a tile that was set, an instance
+    gives the same state and time in a batch and alone."""
+    import trixilw_hip as tlw
+
+    torch_mod()
+    # 16² on, half the CFL number: an 8² mesh of polydeg 3 does not hold a vortex of strength 5 admissible
+    batch, meshes, ics = make_batch(N, "lw", [4, 5, 4], [(5.0, 0.5), (2.5, 0.7), (4.0, 0.4)])
+    L = tlw._lib.lib()
+    tlw._lib.check(L.tlw_set_elements_per_workgroup(batch.handle, tile), batch.handle)
+    cfl = 0.5 * tlw.trixi2lw(0.98, batch.solver)
+    u0 = batch.compute_coefficients()
+    u, status = batch.solve(u0, cfl, 6)
+    for k, (part, ref) in enumerate(zip(batch.split(u0), batch.split(u))):
+        alone = tlw.SemidiscretizationBatch([meshes[k]], tlw.LW(), tlw.CompressibleEulerEquations2D(1.4), [ics[k]],
+                                            batch.solver)
+        tlw._lib.check(L.tlw_set_elements_per_workgroup(alone.handle, tile), alone.handle)
+        got, st = alone.solve(part, cfl, 6)
+        assert np.array_equal(got, ref) and st["t"][0] == status["t"][k]
+        alone.close()
+    batch.close()
