@@ -503,6 +503,10 @@ int tlw_apply_positivity_limiter(tlw_ctx* ctx, double* u_dev);
  * (and, for MDRK, the stage buffer) is used as scratch. */
 int tlw_set_elements_per_workgroup(tlw_ctx* ctx, int32_t elements);
 int tlw_get_elements_per_workgroup(const tlw_ctx* ctx, int32_t* elements);
+/* How the context launches at present, for tests and measurements (no counterpart in the
+ * reference): the number of surface workgroups that run apart with the boundary code (0: one
+ * surface launch), and the number of captured step sequences (tlw_enable_graphs). */
+int tlw_launch_info(const tlw_ctx* ctx, int32_t* boundary_workgroups, int32_t* graphs);
 int tlw_autotune(tlw_ctx* ctx, int32_t reps, int32_t* chosen, double* ms);
 
 /* Copy an element-cache array to the host.  TLW_AUX_U: Ũ [v,i,j,e], len 4 n^2 E, and

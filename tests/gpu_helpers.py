@@ -68,16 +68,15 @@ def assert_close(a, b, tol=TOL, what=""):
     assert l2 <= tol and li <= tol, f"{what}: rel L2 {l2:.3e}, rel Linf {li:.3e}"
 
 
-def traced(fn):
-    """fn's result, and the names of the runtime calls and kernels that it made."""
-    torch = torch_mod()
-    from torch.profiler import ProfilerActivity, profile
+def launch_info(semi):
+    """(surface workgroups that run apart with the boundary code, captured step sequences)"""
+    import ctypes as C
 
-    torch.cuda.synchronize()
-    with profile(activities=[ProfilerActivity.CPU, ProfilerActivity.CUDA]) as p:
-        out = fn()
-        torch.cuda.synchronize()
-    return out, [e.name for e in p.events()]
+    from trixilw_hip import _lib
+
+    b, g = C.c_int32(), C.c_int32()
+    _lib.check(_lib.lib().tlw_launch_info(semi.handle, C.byref(b), C.byref(g)), semi.handle)
+    return b.value, g.value
 
 
 GAMMA = 1.4

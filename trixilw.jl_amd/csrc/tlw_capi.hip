@@ -1686,6 +1686,13 @@ int tlw_get_elements_per_workgroup(const tlw_ctx* c, int32_t* elements) {
     return TLW_OK;
 }
 
+int tlw_launch_info(const tlw_ctx* c, int32_t* boundary_workgroups, int32_t* graphs) {
+    if (!c || !boundary_workgroups || !graphs) return TLW_EINVAL;
+    *boundary_workgroups = c->sbnd;
+    *graphs = (int32_t)c->graph_cache.size();
+    return TLW_OK;
+}
+
 int tlw_autotune(tlw_ctx* c, int32_t reps, int32_t* chosen, double* ms_out) {
     if (!c) return TLW_EINVAL;
     if (reps < 1) return fail(c, TLW_EINVAL, "reps >= 1 required");

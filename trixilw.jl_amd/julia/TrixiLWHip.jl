@@ -447,6 +447,9 @@ set_elements_per_workgroup!(ctx, eb) = check(ctx, ccall((:tlw_set_elements_per_w
     (Ptr{Cvoid}, Int32), ctx, eb))
 elements_per_workgroup(ctx) = (e = Ref{Int32}(0);
     check(ctx, ccall((:tlw_get_elements_per_workgroup, lib), Cint, (Ptr{Cvoid}, Ref{Int32}), ctx, e)); e[])
+# (surface workgroups run apart with the boundary code, captured step sequences)
+launch_info(ctx) = (b = Ref{Int32}(0); g = Ref{Int32}(0);
+    check(ctx, ccall((:tlw_launch_info, lib), Cint, (Ptr{Cvoid}, Ref{Int32}, Ref{Int32}), ctx, b, g)); (b[], g[]))
 # pick the volume tile once per mesh, after set_state!
 autotune!(ctx; reps = 3) = (c = Ref{Int32}(0); ms = zeros(3);
     check(ctx, ccall((:tlw_autotune, lib), Cint, (Ptr{Cvoid}, Int32, Ref{Int32}, Ptr{Float64}), ctx, reps, c, ms));

@@ -37,6 +37,7 @@ EXPORTED = (
     "tlw_create_ensemble", "tlw_ensemble_set_stream", "tlw_ensemble_enable_graphs", "tlw_ensemble_solve_init",
     "tlw_ensemble_advance", "tlw_ensemble_last_error", "tlw_ensemble_destroy", "tlw_adjoint_mdrk",
     "tlw_create_nonconforming", "tlw_rebuild_mesh_nonconforming", "tlw_transfer_solution", "tlw_create_p4est",
+    "tlw_launch_info",
 )
 
 
@@ -213,6 +214,8 @@ def lib():
     L.tlw_set_elements_per_workgroup.argtypes = [vp, i32]
     L.tlw_get_elements_per_workgroup.restype = C.c_int
     L.tlw_get_elements_per_workgroup.argtypes = [vp, C.POINTER(i32)]
+    L.tlw_launch_info.restype = C.c_int
+    L.tlw_launch_info.argtypes = [vp, C.POINTER(i32), C.POINTER(i32)]
     L.tlw_set_positivity_limiter.restype = C.c_int
     L.tlw_set_positivity_limiter.argtypes = [vp, i32, C.c_double, C.c_double]
     L.tlw_apply_positivity_limiter.restype = C.c_int
