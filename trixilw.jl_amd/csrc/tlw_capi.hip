@@ -171,8 +171,9 @@ const int* eb_choices(int N) { return N == 4 ? kEbChoices4 : kEbChoices3; }
 // polydeg 3 LW, Z-order: Euler 16² 12.3 / 12.1 / 13.1, 32² 12.7 / 12.2 / 13.2, 64²
 // 16.3 / 14.5 / 15.2, 128² 28.1 / 27.2 / 27.0 (a rhs call 25.6 / 21.6 / 23.6), 256²
 // 67.3 / 65.7 / 64.7; Navier-Stokes 16² 15.8 / 15.7 / 16.9, 64² 21.5 / 19.5 / 19.5,
-// 128² 37.2 / 38.2 / 37.5.  Up to 2048 elements 4 and 8 are within 5 % of each other
-// and both ahead of 16; a warped 96² takes 23.1 / 21.2 / 23.8.
+// 128² 37.2 / 38.2 / 37.5.  Both small tiles are ahead of 16 up to 2048 elements and
+// neither always of the other (a warped 40² Euler 13.5 / 12.5 / 14.1, a warped 48²
+// Navier-Stokes 18.4 / 19.2 / 18.8); a warped 96² takes 23.1 / 21.2 / 23.8.
 // The two launches of an MDRK step gain from the 16-element tile as soon as it fills
 // the chip, 1024 workgroups: 128² Euler 47.6 / 44.6 / 44.2, Navier-Stokes 63.1 / 64.7 /
 // 61.1, warped Navier-Stokes 66.0 / 66.8 / 64.0 and at 120² 67.1 / 63.9 / 64.7, at 96²
